@@ -8,10 +8,10 @@
 // Matching bf16 / fp16 operands take the large-tile kernel of gemm_fast.hpp
 // (256 x 256 workgroup tiles of v_mfma_f32_32x32x16, operands copied straight
 // into LDS, persistent grid in XCD bands, split-K for short grids, fused
-// bias / residual / GELU epilogues) wherever its shape and alignment checks
-// pass (fast_ok).  Everything else -- fp32 and mixed dtypes, odd strides,
-// shapes it does not take, and efla_rt_set_gemm_backend(1) -- runs the generic
-// kernel below.
+// bias / residual / GELU epilogues), operands of odd strides or sizes from
+// padded copies.  Everything else -- fp32 and mixed dtypes, small odd shapes
+// (kPadMinWork), and efla_rt_set_gemm_backend(1) -- runs the generic kernel
+// below.
 //
 // The generic kernel covers all three products with one template.  Operands
 // are described as (m,k) and (k,n) matrices whose contiguous index is either k
@@ -427,69 +427,84 @@ struct FastOp {
 };
 
 static bool aligned_to(const void* p, uintptr_t a) { return ((uintptr_t)p & (a - 1)) == 0; }
+static long up8(long x) { return (x + 7) & ~7L; }
 
-// Whether the large-tile kernel takes the problem: whole 16-byte rows and
-// chunks along k (K % 8), along every line-contiguous operand's lines and
-// along the output's columns (N % 8); 16-byte aligned operands and outputs
-// (the epilogue moves 16-byte row pieces); 32-bit in-tile offsets
-// (256 * ld * 2 < 2^31).
-static bool fast_ok(long M, long N, long K, const FastOp& a, const FastOp& b, const void* d,
-                    long ldd, const void* bias, const void* c, long ldc, const void* aux,
-                    long ldaux) {
-    const long lim = (long)1 << 22;
-    if (M < 1 || N < 1 || K < 1 || M > INT32_MAX / 2 || N > INT32_MAX / 2) return false;
-    if (K % 8 || N % 8 || (!a.kc && M % 8)) return false;
-    for (long ld : {a.ld, b.ld, ldd})
-        if (ld % 8 || ld >= lim) return false;
-    if (!aligned_to(a.p, 16) || !aligned_to(b.p, 16) || !aligned_to(d, 16)) return false;
-    if (bias && !aligned_to(bias, 16)) return false;
-    if (c && (ldc % 8 || ldc >= lim || !aligned_to(c, 16))) return false;
-    if (aux && (ldaux % 8 || ldaux >= lim || !aligned_to(aux, 16))) return false;
-    return true;
-}
+// 32-bit in-tile offsets: 256 * ld * 2 < 2^31
+constexpr long kFastLdLimit = (long)1 << 22;
 
-template <typename T, int EPI, int NW>
-static void fast_kernel_launch_nw(const FastOp& a, const FastOp& b, const gf::Opnd& A,
-                                  const gf::Opnd& B, long M, long N, long K,
-                                  const gf::EpiArgs<T>& ea, int ksplit, long kper, long tiles,
-                                  const char* name, hipStream_t st) {
-    // persistent: at most one workgroup per CU (the LDS allows no more)
-    const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
-    const long items = tiles * ksplit;
-    const dim3 grid((unsigned)(items < cus ? items : cus)), block(64 * NW);
-    if (a.kc && b.kc)
-        EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, true, true, EPI, NW>), grid, block, st, A, B,
-                    M, N, K, ea, ksplit, kper);
-    else if (a.kc)
-        EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, true, false, EPI, NW>), grid, block, st, A, B,
-                    M, N, K, ea, ksplit, kper);
-    else if (b.kc)
-        EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, false, true, EPI, NW>), grid, block, st, A, B,
-                    M, N, K, ea, ksplit, kper);
-    else
-        EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, false, false, EPI, NW>), grid, block, st, A,
-                    B, M, N, K, ea, ksplit, kper);
+// Whether an operand's rows can be copied straight into LDS: 16-byte aligned
+// whole pieces.  Otherwise the product runs on a padded copy of it.
+static bool direct_rows(const FastOp& o, long lines, long K) {
+    return (o.kc ? K : lines) % 8 == 0 && o.ld % 8 == 0 && o.ld < kFastLdLimit &&
+           aligned_to(o.p, 16);
 }
 
 // 8 waves (two per SIMD) measured faster than 4 at every config-4 shape
-template <typename T, int EPI>
+template <typename T, int EPI, bool RAGGED>
 static void fast_kernel_launch(const FastOp& a, const FastOp& b, const gf::Opnd& A,
                                const gf::Opnd& B, long M, long N, long K,
                                const gf::EpiArgs<T>& ea, int ksplit, long kper, long tiles,
                                const char* name, hipStream_t st) {
-    fast_kernel_launch_nw<T, EPI, 8>(a, b, A, B, M, N, K, ea, ksplit, kper, tiles, name, st);
+    // persistent: at most one workgroup per CU (the LDS allows no more)
+    const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    const long items = tiles * ksplit;
+    const dim3 grid((unsigned)(items < cus ? items : cus)), block(64 * 8);
+    // the GELU forms exist for the layouts their entry points have
+    constexpr bool fwd = EPI != gf::EPI_DGELU, any = EPI != gf::EPI_DGELU && EPI != gf::EPI_GELU_AUX;
+    if constexpr (any || !fwd)
+        if (a.kc && b.kc)
+            EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, true, true, EPI, 8, RAGGED>), grid, block,
+                        st, A, B, M, N, K, ea, ksplit, kper);
+    if constexpr (fwd)
+        if (a.kc && !b.kc)
+            EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, true, false, EPI, 8, RAGGED>), grid, block,
+                        st, A, B, M, N, K, ea, ksplit, kper);
+    if constexpr (any) {
+        if (!a.kc && b.kc)
+            EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, false, true, EPI, 8, RAGGED>), grid, block,
+                        st, A, B, M, N, K, ea, ksplit, kper);
+        if (!a.kc && !b.kc)
+            EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, false, false, EPI, 8, RAGGED>), grid,
+                        block, st, A, B, M, N, K, ea, ksplit, kper);
+    }
 }
 
-// Large-tile product.  Problems with fewer output tiles than the GPU has CUs
+// A product of whole 16-byte pieces always takes the kernel.  One with an odd
+// contraction, an operand to pad or an unaligned output is worth it from this
+// many multiply-adds on; below, both ways are a few launches long.  Measured
+// (generic kernel / this one with its padding, us; m x k x n):
+//     60 x 256 x 264     fwd   23 / 10    dA   19 / 12   dB   12 / 12
+//     60 x 512 x 517     fwd   58 / 16    dA   61 / 19   dB   15 / 12
+//   2100 x 768 x 2316    fwd  100 / 35    dA  376 / 44   dB  312 / 39
+//   2100 x 768 x 16001   fwd  400 / 90    dA 4387 / 116  dB  523 / 89
+//   2500 x 1024 x 4096   dB   269 / 47  (rows read in place: only k is odd)
+constexpr long kPadMinWork = (long)1 << 22;
+// padded copies past this many bytes are not made: such a product stays on the
+// generic kernel, which needs no scratch
+constexpr size_t kPadMaxBytes = (size_t)4 << 30;
+
+// Large-tile product, or -1 if it does not take the problem (the generic
+// kernel does).  Problems with fewer output tiles than the GPU has CUs
 // and a long contraction are split along k: fp32
 // partial tiles go to the stream's cached workspace and a second kernel adds
 // them in split order and runs the epilogue (plain epilogues only).
+// Workspace: [head_bytes for the caller (ea.cpart) | padded A | padded B |
+// partials]; with head_bytes the lease stays with the caller.
 template <typename T, int EPI>
 static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
-                       const gf::EpiArgs<T>& ea, const char* name, hipStream_t st) {
-    const gf::Opnd A{(const char*)a.p, a.ld, (int)M}, B{(const char*)b.p, b.ld, (int)N};
+                       const gf::EpiArgs<T>& ea, const char* name, hipStream_t st,
+                       size_t head_bytes = 0, WsLease* head_lease = nullptr) {
+    if (M < 1 || N < 1 || K < 1 || M > INT32_MAX / 2 || N > INT32_MAX / 2) return -1;
+    const bool pa = !direct_rows(a, M, K), pb = !direct_rows(b, N, K);
+    // whole 16-byte pieces everywhere: nothing but split-K partials needs scratch
+    const bool out_whole = N % 8 == 0 && ea.ldd % 8 == 0 && aligned_to(ea.d, 16) &&
+                           aligned_to(ea.bias, 16) &&
+                           (!ea.c || (ea.ldc % 8 == 0 && aligned_to(ea.c, 16))) &&
+                           (!ea.aux || (ea.ldaux % 8 == 0 && aligned_to(ea.aux, 16)));
+    const bool plain = !pa && !pb && K % 8 == 0 && out_whole;
+    if (!plain && (double)M * (double)N * (double)K < (double)kPadMinWork) return -1;
     const long tiles = ((M + gf::BM - 1) / gf::BM) * ((N + gf::BN - 1) / gf::BN);
-    if (tiles > 0x7FFFFFFFL / 64) return kInvalidConfiguration;
+    if (tiles > 0x7FFFFFFFL / 64) return plain ? kInvalidConfiguration : -1;
     int ksplit = 1;
     const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
     if ((EPI == gf::EPI_PLAIN || EPI == gf::EPI_RESID) && tiles < cus) {
@@ -497,24 +512,80 @@ static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
         const long most = K / (4 * gf::BK);  // at least 4 k-iterations each
         ksplit = (int)std::max(1L, std::min({want, most, 32L}));
     }
+    long kper = K;
+    if (ksplit > 1) {
+        kper = ((K + ksplit - 1) / ksplit + gf::BK - 1) / gf::BK * gf::BK;
+        ksplit = (int)((K + kper - 1) / kper);
+    }
+    // scratch
+    auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    auto padded = [&](const FastOp& o, long lines, long& rows, long& cols) {
+        rows = o.kc ? lines : K;
+        cols = o.kc ? K : lines;
+        return (double)rows * (double)up8(cols) * sizeof(T);
+    };
+    long ra, ca, rb, cb;
+    const double da = pa ? padded(a, M, ra, ca) : 0., db = pb ? padded(b, N, rb, cb) : 0.;
+    if (da + db > (double)kPadMaxBytes || (pa && up8(ca) >= kFastLdLimit) ||
+        (pb && up8(cb) >= kFastLdLimit))
+        return -1;
+    const size_t ba = up((size_t)da), bb = up((size_t)db);
+    const size_t bp = ksplit > 1 ? (size_t)ksplit * M * up8(N) * sizeof(float) : 0;
+    const size_t need = up(head_bytes) + ba + bb + bp;
+    char* ws = nullptr;
+    WsLease own;
+    if (need) {
+        void* p = nullptr;
+        // a product that the generic kernel would take without scratch does
+        // so where scratch is not to be had (a stream under capture, memory)
+        if (!plain && !workspace_available(need, st)) return -1;
+        const int rc = workspace_acquire(need, st, &p, head_lease ? *head_lease : own);
+        if (rc != kSuccess) {
+            if (plain) return rc;
+            (void)hipGetLastError();
+            (head_lease ? *head_lease : own).release();
+            return -1;
+        }
+        ws = (char*)p;
+    }
+    gf::EpiArgs<T> ep = ea;
+    if (head_bytes) ep.cpart = (float*)ws;
+    gf::Opnd A{(const char*)a.p, a.ld, (int)M}, B{(const char*)b.p, b.ld, (int)N};
+    auto pad = [&](const FastOp& o, long rows, long cols, char* dst, gf::Opnd& out) {
+        const long ldp = up8(cols);
+        EFLA_LAUNCH("gemm_pad", gf::pad_rows_kernel<T>,
+                    dim3((unsigned)((ldp / 8 + 255) / 256),
+                         (unsigned)std::min<long>(rows, 2048)),
+                    dim3(256), st, (const T*)o.p, o.ld, rows, cols, (T*)dst, ldp);
+        out.base = dst;
+        out.ld = ldp;
+        if (!o.kc) out.nlines = (int)ldp;
+    };
+    if (pa) pad(a, ra, ca, ws + up(head_bytes), A);
+    if (pb) pad(b, rb, cb, ws + up(head_bytes) + ba, B);
+    const bool ragged = !out_whole;
     if (ksplit == 1) {
-        fast_kernel_launch<T, EPI>(a, b, A, B, M, N, K, ea, 1, K, tiles, name, st);
+        if (ragged)
+            fast_kernel_launch<T, EPI, true>(a, b, A, B, M, N, K, ep, 1, K, tiles, name, st);
+        else
+            fast_kernel_launch<T, EPI, false>(a, b, A, B, M, N, K, ep, 1, K, tiles, name, st);
         return (int)hipPeekAtLastError();
     }
-    const long kper = ((K + ksplit - 1) / ksplit + gf::BK - 1) / gf::BK * gf::BK;
-    ksplit = (int)((K + kper - 1) / kper);
-    void* ws = nullptr;
-    WsLease lease;
-    EFLA_CHECK((hipError_t)workspace_acquire((size_t)ksplit * M * N * sizeof(float), st, &ws,
-                                             lease));
-    gf::EpiArgs<T> ep = ea;
-    ep.part = (float*)ws;
-    fast_kernel_launch<T, gf::EPI_PARTIAL>(a, b, A, B, M, N, K, ep, ksplit, kper, tiles, name,
-                                           st);
-    long g = (M * (N / 4) + 255) / 256;
-    if (g > 4096) g = 4096;
-    EFLA_LAUNCH("gemm_splitk_reduce", gf::gemm_splitk_reduce<T>, dim3((unsigned)g), dim3(256), st,
-                ep, M, N, ksplit);
+    if constexpr (EPI == gf::EPI_PLAIN || EPI == gf::EPI_RESID) {
+        ep.part = (float*)(ws + up(head_bytes) + ba + bb);
+        const long g = std::min(4096L, (M * ((N + 3) / 4) + 255) / 256);
+        if (ragged) {
+            fast_kernel_launch<T, gf::EPI_PARTIAL, true>(a, b, A, B, M, N, K, ep, ksplit, kper,
+                                                         tiles, name, st);
+            EFLA_LAUNCH("gemm_splitk_reduce", (gf::gemm_splitk_reduce<T, true>),
+                        dim3((unsigned)g), dim3(256), st, ep, M, N, ksplit);
+        } else {
+            fast_kernel_launch<T, gf::EPI_PARTIAL, false>(a, b, A, B, M, N, K, ep, ksplit, kper,
+                                                          tiles, name, st);
+            EFLA_LAUNCH("gemm_splitk_reduce", (gf::gemm_splitk_reduce<T, false>),
+                        dim3((unsigned)g), dim3(256), st, ep, M, N, ksplit);
+        }
+    }
     return (int)hipPeekAtLastError();
 }
 
@@ -574,15 +645,16 @@ extern "C" int gemm_forward_hip(const void* a, const void* b, const void* bias, 
     if (dtype_a == dtype_b && dtype_b == dtype_c) {
         // C[m, n] = A[m, k] B[k, n]: A k-contiguous, B line (n) contiguous
         const FastOp fa{a, (long)k, true}, fb{b, (long)n, false};
-        if (dtype_a != kDtypeF32 && backend() != 1 &&
-            fast_ok((long)m, (long)n, (long)k, fa, fb, c, (long)n, bias, nullptr, 0, nullptr, 0)) {
-            if (dtype_a == kDtypeBF16)
-                return fast_launch<bf16, gf::EPI_PLAIN>(fa, fb, (long)m, (long)n, (long)k,
-                                                        epi<bf16>(c, (long)n, bias), "gemm_fwd",
-                                                        stream);
-            return fast_launch<f16, gf::EPI_PLAIN>(fa, fb, (long)m, (long)n, (long)k,
-                                                   epi<f16>(c, (long)n, bias), "gemm_fwd",
-                                                   stream);
+        if (dtype_a != kDtypeF32 && backend() != 1) {
+            const int rc =
+                dtype_a == kDtypeBF16
+                    ? fast_launch<bf16, gf::EPI_PLAIN>(fa, fb, (long)m, (long)n, (long)k,
+                                                       epi<bf16>(c, (long)n, bias), "gemm_fwd",
+                                                       stream)
+                    : fast_launch<f16, gf::EPI_PLAIN>(fa, fb, (long)m, (long)n, (long)k,
+                                                      epi<f16>(c, (long)n, bias), "gemm_fwd",
+                                                      stream);
+            if (rc >= 0) return rc;
         }
     }
     switch (dtype_a) {
@@ -634,8 +706,7 @@ extern "C" int gemm_backward_hip(const void* grad_c, const void* a, const void* 
         int rc = -1;
         // dA = dC B^T: contraction over n, both operands n-contiguous
         const FastOp fa{grad_c, N, true}, fb{b, N, true};
-        if (backend() != 1 &&
-            fast_ok(M, K, N, fa, fb, grad_a, K, nullptr, nullptr, 0, nullptr, 0))
+        if (backend() != 1)
             rc = fast_launch<bf16, gf::EPI_PLAIN>(fa, fb, M, K, N, epi<bf16>(grad_a, K),
                                                   "gemm_bwd_da", stream);
         if (rc < 0)
@@ -649,8 +720,7 @@ extern "C" int gemm_backward_hip(const void* grad_c, const void* a, const void* 
         int rc = -1;
         // dB = A^T dC: contraction over m, A k- (line-) contiguous, dC n-contiguous
         const FastOp fa{a, K, false}, fb{grad_c, N, false};
-        if (backend() != 1 &&
-            fast_ok(K, N, M, fa, fb, grad_b, N, nullptr, nullptr, 0, nullptr, 0))
+        if (backend() != 1)
             rc = fast_launch<bf16, gf::EPI_PLAIN>(fa, fb, K, N, M, epi<bf16>(grad_b, N),
                                                   "gemm_bwd_db", stream);
         if (rc < 0)
@@ -702,24 +772,25 @@ extern "C" int gemm_ex_hip(int trans_a, int trans_b, size_t m, size_t n, size_t 
     // is B of a stored k x n (n-contiguous) or B^T of a stored n x k
     const FastOp fa{a, (long)lda, trans_a == 0}, fb{b, (long)ldb, trans_b != 0};
     const void* cc = beta != 0.f ? c : nullptr;
-    if (dtype != kDtypeF32 && backend() != 1 &&
-        fast_ok((long)m, (long)n, (long)k, fa, fb, d, (long)ldd, bias, cc, (long)ldc, nullptr, 0)) {
-        if (cc) {
-            if (dtype == kDtypeBF16)
-                return fast_launch<bf16, gf::EPI_RESID>(
-                    fa, fb, (long)m, (long)n, (long)k,
-                    epi<bf16>(d, (long)ldd, bias, alpha, beta, cc, (long)ldc), "gemm_ex", stream);
-            return fast_launch<f16, gf::EPI_RESID>(
+    if (dtype != kDtypeF32 && backend() != 1) {
+        int rc;
+        if (cc && dtype == kDtypeBF16)
+            rc = fast_launch<bf16, gf::EPI_RESID>(
+                fa, fb, (long)m, (long)n, (long)k,
+                epi<bf16>(d, (long)ldd, bias, alpha, beta, cc, (long)ldc), "gemm_ex", stream);
+        else if (cc)
+            rc = fast_launch<f16, gf::EPI_RESID>(
                 fa, fb, (long)m, (long)n, (long)k,
                 epi<f16>(d, (long)ldd, bias, alpha, beta, cc, (long)ldc), "gemm_ex", stream);
-        }
-        if (dtype == kDtypeBF16)
-            return fast_launch<bf16, gf::EPI_PLAIN>(fa, fb, (long)m, (long)n, (long)k,
-                                                    epi<bf16>(d, (long)ldd, bias, alpha),
-                                                    "gemm_ex", stream);
-        return fast_launch<f16, gf::EPI_PLAIN>(fa, fb, (long)m, (long)n, (long)k,
-                                               epi<f16>(d, (long)ldd, bias, alpha), "gemm_ex",
-                                               stream);
+        else if (dtype == kDtypeBF16)
+            rc = fast_launch<bf16, gf::EPI_PLAIN>(fa, fb, (long)m, (long)n, (long)k,
+                                                  epi<bf16>(d, (long)ldd, bias, alpha), "gemm_ex",
+                                                  stream);
+        else
+            rc = fast_launch<f16, gf::EPI_PLAIN>(fa, fb, (long)m, (long)n, (long)k,
+                                                 epi<f16>(d, (long)ldd, bias, alpha), "gemm_ex",
+                                                 stream);
+        if (rc >= 0) return rc;
     }
     switch (dtype) {
         case kDtypeBF16: return ex_generic<bf16>(trans_a, trans_b, m, n, k, alpha, a, lda, b, ldb,
@@ -749,13 +820,13 @@ extern "C" int gemm_gelu_forward_hip(const void* a, const void* b, const void* b
     if (m > ((size_t)1 << 40) || n > ((size_t)1 << 40) || k > ((size_t)1 << 40))
         return kInvalidValue;
     const FastOp fa{a, (long)k, true}, fb{b, (long)n, false};
-    if (k > 0 && backend() == 0 &&
-        fast_ok((long)m, (long)n, (long)k, fa, fb, out, (long)n, bias, nullptr, 0, pre,
-                (long)n))
-        return fast_launch<bf16, gf::EPI_GELU_AUX>(
+    if (k > 0 && backend() == 0) {
+        const int rc = fast_launch<bf16, gf::EPI_GELU_AUX>(
             fa, fb, (long)m, (long)n, (long)k,
             epi<bf16>(out, (long)n, bias, 1.f, 0.f, nullptr, 0, pre, (long)n), "gemm_gelu_fwd",
             stream);
+        if (rc >= 0) return rc;
+    }
     // the product, then GELU over it (the same functions, so the same bits)
     const int rc = gemm_forward_hip(a, b, bias, pre, m, k, n, kDtypeBF16, kDtypeBF16, kDtypeBF16,
                                     stream);
@@ -783,29 +854,32 @@ extern "C" int gemm_gelu_backward_hip(const void* grad_c, const void* a, const v
             if (!grad_c || !b || !pre) return kInvalidValue;
             // grad_pre = (grad_c b^T) * GELU'(pre): contraction over n, both n-contiguous
             const FastOp fa{grad_c, (long)n, true}, fb{b, (long)n, true};
-            if (n > 0 && backend() == 0 &&
-                fast_ok((long)m, (long)k, (long)n, fa, fb, grad_pre, (long)k, nullptr, nullptr,
-                        0, pre, (long)k)) {
+            int done = -1;
+            if (n > 0 && backend() == 0) {
                 gf::EpiArgs<bf16> ea = epi<bf16>(grad_pre, (long)k, nullptr, 1.f, 0.f, nullptr, 0,
                                                  (void*)pre, (long)k);
                 // grad_pre's column sums from the epilogue: one fp32 row per
-                // 128 output rows, then their sum
-                void* ws = nullptr;
+                // 128 output rows, then their sum (whole 16-byte pieces only)
                 WsLease lease;
                 const long prow = ((long)m + 127) / 128;
-                if (grad_pre_bias) {
-                    EFLA_CHECK((hipError_t)workspace_acquire((size_t)prow * k * sizeof(float),
-                                                             stream, &ws, lease));
-                    ea.cpart = (float*)ws;
-                }
-                int rc = fast_launch<bf16, gf::EPI_DGELU>(fa, fb, (long)m, (long)k, (long)n, ea,
-                                                          "gemm_gelu_bwd_da", stream);
-                if (rc != kSuccess) return rc;
-                if (grad_pre_bias)
+                const bool sums = grad_pre_bias && k % 8 == 0;
+                done = fast_launch<bf16, gf::EPI_DGELU>(
+                    fa, fb, (long)m, (long)k, (long)n, ea, "gemm_gelu_bwd_da", stream,
+                    sums ? (size_t)prow * k * sizeof(float) : 0, &lease);
+                if (done > 0) return done;
+                if (done == 0 && sums) {
                     EFLA_LAUNCH("gemm_gelu_bwd_dbias", colsum_rows_kernel,
                                 dim3((unsigned)((k + 63) / 64)), dim3(NTH), stream,
-                                (const float*)ws, prow, (bf16*)grad_pre_bias, (long)k);
-            } else {
+                                (const float*)lease.ptr(), prow, (bf16*)grad_pre_bias,
+                                (long)k);
+                } else if (done == 0 && grad_pre_bias) {
+                    lease.release();  // colsum_bf16 takes its own
+                    const int rc = colsum_bf16((const bf16*)grad_pre, (long)m, (long)k,
+                                               (bf16*)grad_pre_bias, stream);
+                    if (rc != kSuccess) return rc;
+                }
+            }
+            if (done < 0) {
                 int rc = gemm_backward_hip(grad_c, a, b, grad_pre, nullptr, nullptr, m, k, n,
                                            stream);
                 if (rc != kSuccess) return rc;

@@ -28,6 +28,16 @@
 // A k-tail (K not a multiple of 64) runs one last iteration through registers
 // with the missing k zeroed.  Rows and columns past M or N are clamped on load
 // (they only reach outputs that are not stored).
+//
+// What an operand has to be: 16-byte aligned rows of whole 8-element pieces
+// (ld % 8 == 0) whose contiguous extent is a multiple of 8 or zero up to the
+// next one.  An operand that is not (an odd vocabulary, a 12-head projection
+// row of 2316 values) is first copied into such rows by pad_rows_kernel; the
+// contraction length itself is free.  The output, bias, residual and
+// pre-activation may have any stride and element alignment in the RAGGED form
+// of the kernel: they are moved in 8-element pieces with unaligned 16-byte
+// accesses, the last piece of a row of N % 8 != 0 element by element.  (One
+// form for both costs the aligned products 0.5 to 2 %.)
 #pragma once
 #include "gelu.hpp"
 #include "mfma.hpp"
@@ -121,7 +131,9 @@ __device__ __forceinline__ void copy_tile(const Opnd& op, int line0, long k0, ch
     }
 }
 
-// The k-tail tile through registers: k >= K reads as zero (K % 8 == 0).
+// The k-tail tile through registers: k >= K reads as zero.  A k-contiguous
+// operand's row is zero between K and the next multiple of 8 (K % 8 == 0, or
+// rows padded by pad_rows_kernel), so its pieces are read whole.
 template <bool KC, int NTH>
 __device__ __forceinline__ void copy_tile_tail(const Opnd& op, int line0, long k0, long K,
                                                char* tile, int tid) {
@@ -148,8 +160,6 @@ __device__ __forceinline__ void copy_tile_tail(const Opnd& op, int line0, long k
 }
 
 // --- epilogues ---------------------------------------------------------------
-// Called once per 4 consecutive outputs D[m][n .. n+3] (n % 4 == 0, all inside
-// the matrix) with their fp32 sums.
 // PLAIN: alpha acc (+ bias); RESID: that + beta C; GELU_AUX: pre = acc (+ bias)
 // and GELU(pre); DGELU: bf16(acc) GELU'(pre); PARTIAL: fp32 split-K partials.
 enum EpiKind { EPI_PLAIN = 0, EPI_GELU_AUX = 1, EPI_DGELU = 2, EPI_PARTIAL = 3, EPI_RESID = 4 };
@@ -164,60 +174,60 @@ struct EpiArgs {
     float alpha, beta;
     T* aux;  // GELU_AUX: pre-activation out; DGELU: pre-activation in
     long ldaux;
-    float* part;   // PARTIAL: fp32 partial sums [split][M][N]
+    float* part;   // PARTIAL: fp32 partial sums [split][M][N rounded up to 8]
     float* cpart;  // DGELU: column sums of the output, one fp32 row per 128 output
                    // rows ([M / 128][N]), or NULL
 };
 
-template <typename T>
-__device__ __forceinline__ void load4(const T* p, float* v) {
-    typedef __attribute__((__vector_size__(4 * sizeof(T)))) T t4;
-    const t4 x = *reinterpret_cast<const t4*>(p);
+// W elements at p (element-aligned), the first cnt of them if cnt < W; those
+// past cnt read as zero and are not written
+template <int W, typename T, bool RAGGED = true>
+struct Piece {
+    typedef __attribute__((__vector_size__(W * sizeof(T)))) T vec;
+    typedef vec uvec __attribute__((aligned(sizeof(T))));
+    static __device__ __forceinline__ vec load(const T* p, long cnt) {
+        if constexpr (!RAGGED) return *reinterpret_cast<const vec*>(p);  // whole and aligned
+        if (cnt >= W) return *reinterpret_cast<const uvec*>(p);
+        vec x{};
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = (float)x[e];
-}
-template <typename T>
-__device__ __forceinline__ void store4(T* p, const float* v) {
-    typedef __attribute__((__vector_size__(4 * sizeof(T)))) T t4;
-    *reinterpret_cast<t4*>(p) = t4{(T)v[0], (T)v[1], (T)v[2], (T)v[3]};
-}
+        for (int e = 0; e < W; ++e)
+            if (e < cnt) x[e] = p[e];
+        return x;
+    }
+    static __device__ __forceinline__ void store(T* p, vec x, long cnt) {
+        if constexpr (!RAGGED) {
+            *reinterpret_cast<vec*>(p) = x;
+            return;
+        }
+        if (cnt >= W) {
+            *reinterpret_cast<uvec*>(p) = x;
+            return;
+        }
+#pragma unroll
+        for (int e = 0; e < W; ++e)
+            if (e < cnt) p[e] = x[e];
+    }
+};
 
-template <typename T, int EPI>
-__device__ __forceinline__ void epilogue4(const EpiArgs<T>& ea, long m, long n, const float* acc) {
-    if constexpr (EPI == EPI_PARTIAL) return;  // handled by the kernel
+// columns n .. n + 3 of row m of the output, cnt = N - n of them in the matrix
+template <typename T, bool RAGGED>
+__device__ __forceinline__ void epilogue4(const EpiArgs<T>& ea, long m, long n, long cnt,
+                                          const float* acc) {
+    typedef Piece<4, T, RAGGED> P4;
     float v[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = ea.alpha * acc[e];
     if (ea.bias) {
-        float b[4];
-        load4(ea.bias + n, b);
+        const typename P4::vec b = P4::load(ea.bias + n, cnt);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += b[e];
-    }
-    if constexpr (EPI == EPI_GELU_AUX) {
-        store4(ea.aux + m * ea.ldaux + n, v);  // pre-activation for the backward
-        float r[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = gelu::gelu_f<true>((float)(T)v[e]);
-        store4(ea.d + m * ea.ldd + n, r);
-        return;
-    }
-    if constexpr (EPI == EPI_DGELU) {
-        float u[4];
-        load4(ea.aux + m * ea.ldaux + n, u);
-        float r[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) r[e] = (float)(T)v[e] * gelu::gelu_df<true>(u[e]);
-        store4(ea.d + m * ea.ldd + n, r);
-        return;
+        for (int e = 0; e < 4; ++e) v[e] += (float)b[e];
     }
     if (ea.beta != 0.f) {
-        float c[4];
-        load4(ea.c + m * ea.ldc + n, c);
+        const typename P4::vec c = P4::load(ea.c + m * ea.ldc + n, cnt);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += ea.beta * c[e];
+        for (int e = 0; e < 4; ++e) v[e] += ea.beta * (float)c[e];
     }
-    store4(ea.d + m * ea.ldd + n, v);
+    P4::store(ea.d + m * ea.ldd + n, typename P4::vec{(T)v[0], (T)v[1], (T)v[2], (T)v[3]}, cnt);
 }
 
 // --- epilogue staged through LDS ---------------------------------------------
@@ -238,13 +248,14 @@ __device__ __forceinline__ unsigned ep_off(int row, int col) {  // col % 4 == 0
     return (unsigned)(row * (128 * TNI) + (((col >> 2) ^ (row & 15)) << 4));
 }
 
-template <typename T, int EPI, int TNI, bool AHEAD>
+template <typename T, int EPI, int TNI, bool AHEAD, bool RAGGED>
 __device__ __forceinline__ void epilogue_wave(const EpiArgs<T>& ea, const floatx16 (&acc)[TNI][4],
                                               int split, long mw, long nw, long M, long N, int l,
                                               char* wp) {
     constexpr int WC = 32 * TNI;  // columns of the wave's block
     constexpr int NP = WC / 16;   // 8-element pieces per lane and 32-row pass
-    typedef __attribute__((__vector_size__(8 * sizeof(T)))) T t8;
+    typedef Piece<8, T, RAGGED> P8;
+    typedef typename P8::vec t8;
     // DGELU with column sums: this lane's 8 columns (piece c8 = l % (WC / 8)
     // of every row it finishes) summed over its rows
     float csum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -271,7 +282,7 @@ __device__ __forceinline__ void epilogue_wave(const EpiArgs<T>& ea, const floatx
             long n;
             piece(s, row, n);
             const long m = mw + 32 * j + row;
-            dst[s] = (m < M && n < N) ? *reinterpret_cast<const t8*>(src + m * lds + n) : t8{};
+            dst[s] = (m < M && n < N) ? P8::load(src + m * lds + n, N - n) : t8{};
         }
     };
     t8 inp[2][NP];
@@ -306,14 +317,14 @@ __device__ __forceinline__ void epilogue_wave(const EpiArgs<T>& ea, const floatx
                 *reinterpret_cast<const mf::floatx4*>(wp + ep_off<TNI>(row, 8 * c8 + 4));
             if (m >= M || n >= N) continue;
             if constexpr (EPI == EPI_PARTIAL) {
-                float* dst = ea.part + ((long)split * M + m) * N + n;
+                float* dst = ea.part + ((long)split * M + m) * (RAGGED ? (N + 7) & ~7L : N) + n;
                 *reinterpret_cast<mf::floatx4*>(dst) = v0;
                 *reinterpret_cast<mf::floatx4*>(dst + 4) = v1;
                 continue;
             }
             float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
             if (ea.bias) {
-                const t8 bb = *reinterpret_cast<const t8*>(ea.bias + n);
+                const t8 bb = P8::load(ea.bias + n, N - n);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[e] += (float)bb[e];
             }
@@ -322,7 +333,7 @@ __device__ __forceinline__ void epilogue_wave(const EpiArgs<T>& ea, const floatx
                 t8 pre;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) pre[e] = (T)v[e];
-                *reinterpret_cast<t8*>(ea.aux + m * ea.ldaux + n) = pre;
+                P8::store(ea.aux + m * ea.ldaux + n, pre, N - n);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) y[e] = (T)gelu::gelu_f<true>((float)pre[e]);
             } else if constexpr (EPI == EPI_DGELU) {
@@ -345,7 +356,7 @@ __device__ __forceinline__ void epilogue_wave(const EpiArgs<T>& ea, const floatx
 #pragma unroll
                 for (int e = 0; e < 8; ++e) y[e] = (T)v[e];
             }
-            *reinterpret_cast<t8*>(ea.d + m * ea.ldd + n) = y;
+            P8::store(ea.d + m * ea.ldd + n, y, N - n);
         }
     }
     if constexpr (EPI == EPI_DGELU) {
@@ -386,7 +397,7 @@ struct Item {
     long kbeg, klen;
 };
 
-template <typename T, bool AKC, bool BKC, int EPI, int NW>
+template <typename T, bool AKC, bool BKC, int EPI, int NW, bool RAGGED>
 __global__ void __launch_bounds__(64 * NW) gemm_fast_kernel(Opnd A, Opnd B, long M, long N,
                                                             long K, EpiArgs<T> ea, int ksplit,
                                                             long kper) {
@@ -538,7 +549,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_fast_kernel(Opnd A, Opnd B, long
         {
             const int le = mf::tid_in((int)it) & 63;
             char* wp = smem + 2 * (buf ^ 1) * TILE_BYTES + (4096 * TNI) * w;
-            epilogue_wave<T, EPI, TNI, AKC && BKC>(ea, acc, cur.split, (long)cur.m0 + wm,
+            epilogue_wave<T, EPI, TNI, AKC && BKC, RAGGED>(ea, acc, cur.split, (long)cur.m0 + wm,
                                                     (long)cur.n0 + wn, M, N, le, wp);
         }
         __syncthreads();  // the next item's first copies refill the buffer
@@ -550,18 +561,34 @@ __global__ void __launch_bounds__(64 * NW) gemm_fast_kernel(Opnd A, Opnd B, long
 
 // D = epilogue(sum over splits of the fp32 partials), 4 outputs per thread,
 // the splits added in order (so the result does not depend on scheduling).
-template <typename T>
+template <typename T, bool RAGGED>
 __global__ void __launch_bounds__(256) gemm_splitk_reduce(EpiArgs<T> ea, long M, long N,
                                                           int ksplit) {
-    const long nq = N / 4, total = M * nq;
+    const long ldp = RAGGED ? (N + 7) & ~7L : N;
+    const long nq = RAGGED ? (N + 3) / 4 : N / 4, total = M * nq;
     for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long)gridDim.x * 256) {
         const long m = i / nq, n = 4 * (i - m * nq);
-        mf::floatx4 s = *reinterpret_cast<const mf::floatx4*>(ea.part + m * N + n);
+        mf::floatx4 s = *reinterpret_cast<const mf::floatx4*>(ea.part + m * ldp + n);
         for (int k = 1; k < ksplit; ++k)
-            s += *reinterpret_cast<const mf::floatx4*>(ea.part + ((long)k * M + m) * N + n);
+            s += *reinterpret_cast<const mf::floatx4*>(ea.part + ((long)k * M + m) * ldp + n);
         const float v[4] = {s[0], s[1], s[2], s[3]};
-        epilogue4<T, EPI_PLAIN>(ea, m, n, v);
+        epilogue4<T, RAGGED>(ea, m, n, N - n, v);
     }
+}
+
+// dst[r][0 .. ldp) = src[r][0 .. cols) then zeros, for the rows r of a matrix
+// with any row stride and element alignment; dst 16-byte aligned, ldp = cols
+// rounded up to 8.  One 8-element piece per thread and row, grid y over rows.
+// Bound by its bytes (read once, written once).
+template <typename T>
+__global__ void __launch_bounds__(256) pad_rows_kernel(const T* __restrict__ src, long ld,
+                                                       long rows, long cols,
+                                                       T* __restrict__ dst, long ldp) {
+    const long c = 8 * ((long)blockIdx.x * 256 + threadIdx.x);
+    if (c >= ldp) return;
+    for (long r = blockIdx.y; r < rows; r += gridDim.y)
+        *reinterpret_cast<typename Piece<8, T>::vec*>(dst + r * ldp + c) =
+            Piece<8, T>::load(src + r * ld + c, cols - c);
 }
 
 }  // namespace gf

@@ -87,6 +87,7 @@ class WsLease {
     WsLease& operator=(const WsLease&) = delete;
     ~WsLease() { release(); }
     void release();
+    void* ptr() const;  // the leased buffer
     WsEntry* entry = nullptr;
 };
 
@@ -95,6 +96,11 @@ class WsLease {
 // never takes a second lease on the same (stream, slot) while holding one.
 int workspace_acquire(size_t bytes, hipStream_t stream, void** ptr, WsLease& lease,
                       int slot = 0);
+
+// Whether workspace_acquire(bytes, stream) can be expected to work: the cached
+// buffer is large enough already, or the stream is not under capture (a buffer
+// cannot grow there).  For callers that have a slower way without scratch.
+bool workspace_available(size_t bytes, hipStream_t stream, int slot = 0);
 
 // Zero-fill through a kernel (no hipMemsetAsync, so the call is safe inside
 // stream capture).

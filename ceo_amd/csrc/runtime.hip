@@ -347,6 +347,25 @@ int workspace_acquire(size_t bytes, hipStream_t stream, void** ptr, WsLease& lea
     return kSuccess;
 }
 
+void* WsLease::ptr() const { return entry ? entry->ptr : nullptr; }
+
+bool workspace_available(size_t bytes, hipStream_t stream, int slot) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    WsEntry* e = ws_entry(dev, stream, slot);
+    if (e->owner.load() == std::this_thread::get_id()) return false;
+    {
+        std::lock_guard<std::mutex> lk(e->mu);
+        if (e->bytes >= bytes) return true;
+    }
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return st == hipStreamCaptureStatusNone;
+}
+
 int device_cu_count() {
     static std::atomic<int> cached[64];
     int dev = 0;

@@ -574,3 +574,79 @@ def test_gemm_gelu_config4_mlp():
     print(f"  rel-L2 pre {e1:.2e} out {e2:.2e} dpre {e3:.2e} dw {e4:.2e} dbias {e5:.2e} "
           f"dpre colsum {e6:.2e}", flush=True)
     assert max(e1, e2, e3, e4, e5, e6) <= 1e-2
+
+
+# odd contractions, strides and alignments on the large-tile kernel: operands
+# read in place (dB of an odd row count), padded copies, outputs whose rows end
+# in a partial 8-element piece or start off a 16-byte boundary, with and
+# without split-K.  Bound: the product is rounded once to bf16 (2^-9 at most,
+# relative) after an fp32 sum, the residual forms round nothing else.
+_ODD = [(333, 519, 1031), (900, 64, 2316), (257, 2316, 264), (1250, 1000, 24), (65, 4097, 320)]
+
+
+@pytest.mark.parametrize("m,k,n", _ODD)
+def test_gemm_odd_shapes_large_tile(m, k, n):
+    from ceo_amd import nn
+
+    announce(f"gemm odd {m}x{k}x{n}: forward, dA, dB, residual views, GELU forms")
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+
+    def r(*s):
+        return torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+
+    def off(got, ref):
+        return ((got.double() - ref).norm() / ref.norm()).item()
+
+    a, b, dc, bias = r(m, k), r(k, n), r(m, n), r(n)
+    A, B, D = a.double(), b.double(), dc.double()
+    errs = {"fwd": off(nn.gemm_forward(a, b, bias), A @ B + bias.double())}
+    da, db, _ = nn.gemm_backward(dc, a, b)
+    errs.update(da=off(da, D @ B.T), db=off(db, A.T @ D))
+    # views: columns of a wider row, one element off a 16-byte boundary
+    wide, res = torch.zeros(m, n + 13, dtype=torch.bfloat16, device="cuda"), r(m, n + 3)
+    out, c = wide[:, 1:1 + n], res[:, 2:2 + n]
+    av, bv = r(m, k + 5)[:, 3:3 + k], r(n, k + 8)[:, 1:1 + k]
+    nn.gemm_ex(av, bv, out, bias=bias, c=c, alpha=0.5, beta=1.0, trans_b=True)
+    errs["ex"] = off(out, 0.5 * av.double() @ bv.double().T + bias.double() + c.double())
+    assert not wide[:, 0].any() and not wide[:, n + 1:].any()
+    pre, act = nn.gemm_gelu_forward(a, b, bias)
+    errs["pre"] = off(pre, A @ B + bias.double())
+    errs["gelu"] = off(act, torch.nn.functional.gelu(pre.double(), approximate="tanh"))
+    pb = torch.empty(k, dtype=torch.bfloat16, device="cuda")
+    u = r(m, k)
+    dpre, _, _ = nn.gemm_gelu_backward(dc, a, b, u, need_b=False, out_pre_bias=pb)
+    x = u.double().requires_grad_(True)
+    (gl,) = torch.autograd.grad(torch.nn.functional.gelu(x, approximate="tanh"), x,
+                                da.double())
+    # GELU' crosses zero: its fp32 evaluation adds a unit or two to the rounding
+    errs["dgelu"] = 0.5 * off(dpre, gl)
+    errs["dpre_bias"] = off(pb, dpre.double().sum(0))
+    print("  rel-L2:", {n_: f"{v:.2e}" for n_, v in errs.items()}, flush=True)
+    assert all(v <= 2.0 ** -9 for v in errs.values()), errs
+
+
+def test_gemm_odd_shape_ignores_what_surrounds_it():
+    """Operand views with NaN in every element around them: padded copies and
+    the k tail read nothing outside the views."""
+    from ceo_amd import nn
+
+    m, k, n = 300, 331, 517
+    announce(f"gemm odd {m}x{k}x{n} inside NaN")
+    g = torch.Generator(device="cuda").manual_seed(11)
+
+    def inside(rows, cols, left):
+        t = torch.full((rows + 2, cols + left + 9), float("nan"), dtype=torch.bfloat16,
+                       device="cuda")
+        v = t[1:1 + rows, left:left + cols]
+        v.copy_(torch.randn(rows, cols, generator=g, device="cuda"))
+        return v
+
+    for ta in (False, True):
+        for tb in (False, True):
+            for left in (0, 8, 3):
+                a = inside(k, m, left) if ta else inside(m, k, left)
+                b = inside(n, k, left) if tb else inside(k, n, left)
+                out = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+                nn.gemm_ex(a, b, out, trans_a=ta, trans_b=tb)
+                ref = (a.double().T if ta else a.double()) @ (b.double().T if tb else b.double())
+                assert ((out.double() - ref).norm() / ref.norm()).item() <= 2.0 ** -9

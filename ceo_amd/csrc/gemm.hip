@@ -37,6 +37,7 @@
 #include "../../include/efla_runtime.h"
 #include "common.hpp"
 #include "gemm_fast.hpp"
+#include "gemm_skinny.hpp"
 #include "internal.hpp"
 
 namespace efla {
@@ -469,6 +470,76 @@ static void fast_kernel_launch(const FastOp& a, const FastOp& b, const gf::Opnd&
     }
 }
 
+// Few-row products (gemm_skinny.hpp) up to this many rows, four 16-row tiles a
+// wave; from 65 on the large tile.  Measured (this at 64 rows / large tile at
+// 65, us): 1024 x 3088 8.2 / 15.1, 1024 x 1024 7.7 / 13.1, 4096 x 1024
+// 11.1 / 18.3, 1024 x 32000 27.1 / 26.4; transposed weights (dA) 9.4 / 17.4,
+// 7.8 / 13.2, 8.4 / 15.4, 29.6 / 38.6.
+constexpr long kSkinnyRows = 64;
+
+// whether gemm_skinny_kernel takes the problem
+static bool skinny_ok(const FastOp& a, const FastOp& b, long M, long N, long K) {
+    if (M > kSkinnyRows || !a.kc || K % 8 || a.ld % 8 || !aligned_to(a.p, 16)) return false;
+    if (K > INT32_MAX || N > INT32_MAX / 2) return false;
+    return b.kc ? b.ld % 8 == 0 && aligned_to(b.p, 16)
+                : N % 2 == 0 && b.ld % 2 == 0 && aligned_to(b.p, 4);
+}
+
+template <typename T, int EPI, int MT>
+static void skinny_launch_mt(const FastOp& a, const FastOp& b, long M, long N, long K, long kper,
+                             const gf::EpiArgs<T>& ea, const char* name, hipStream_t st) {
+    const dim3 grid((unsigned)((N + gs::BN - 1) / gs::BN), (unsigned)((K + kper - 1) / kper));
+    if (b.kc)
+        EFLA_LAUNCH(name, (gs::gemm_skinny_kernel<T, true, EPI, MT>), grid, dim3(gs::NTH), st,
+                    (const T*)a.p, a.ld, (const T*)b.p, b.ld, (int)M, (int)N, (int)K, (int)kper,
+                    ea);
+    else
+        EFLA_LAUNCH(name, (gs::gemm_skinny_kernel<T, false, EPI, MT>), grid, dim3(gs::NTH), st,
+                    (const T*)a.p, a.ld, (const T*)b.p, b.ld, (int)M, (int)N, (int)K, (int)kper,
+                    ea);
+}
+
+template <typename T, int EPI>
+static void skinny_launch_rows(const FastOp& a, const FastOp& b, long M, long N, long K,
+                               long kper, const gf::EpiArgs<T>& ea, const char* name,
+                               hipStream_t st) {
+    if (M <= 16) skinny_launch_mt<T, EPI, 1>(a, b, M, N, K, kper, ea, name, st);
+    else if (M <= 32) skinny_launch_mt<T, EPI, 2>(a, b, M, N, K, kper, ea, name, st);
+    else skinny_launch_mt<T, EPI, 4>(a, b, M, N, K, kper, ea, name, st);
+}
+
+template <typename T, int EPI>
+static int skinny_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
+                         const gf::EpiArgs<T>& ea, const char* name, hipStream_t st) {
+    // a workgroup takes 2.5 ns (16 rows) to 4.7 ns (64 rows) per row of the
+    // weights, a split's reduction about 4 us: split k over the idle CUs from
+    // 2048 rows on, at least 512 rows to a workgroup
+    const long cols = (N + gs::BN - 1) / gs::BN;
+    const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    if constexpr (EPI == gf::EPI_PLAIN || EPI == gf::EPI_RESID) {
+        const long ks = std::min(cus / cols, K / 512);
+        const long kper = ks > 1 ? (K + ks * 32 - 1) / (ks * 32) * 32 : K;
+        const int n = (int)((K + kper - 1) / kper);
+        const size_t bytes = (size_t)n * M * up8(N) * sizeof(float);
+        if (K >= 2048 && n > 1 && workspace_available(bytes, st)) {
+            void* ws = nullptr;
+            WsLease lease;
+            if (workspace_acquire(bytes, st, &ws, lease) == kSuccess) {
+                gf::EpiArgs<T> ep = ea;
+                ep.part = (float*)ws;
+                skinny_launch_rows<T, gf::EPI_PARTIAL>(a, b, M, N, K, kper, ep, name, st);
+                const long g = std::min(4096L, (M * ((N + 3) / 4) + 255) / 256);
+                EFLA_LAUNCH("gemm_splitk_reduce", (gf::gemm_splitk_reduce<T, true>),
+                            dim3((unsigned)g), dim3(256), st, ep, M, N, n);
+                return (int)hipPeekAtLastError();
+            }
+            (void)hipGetLastError();
+        }
+    }
+    skinny_launch_rows<T, EPI>(a, b, M, N, K, K, ea, name, st);
+    return (int)hipPeekAtLastError();
+}
+
 // A product of whole 16-byte pieces always takes the kernel.  One with an odd
 // contraction, an operand to pad or an unaligned output is worth it from this
 // many multiply-adds on; below, both ways are a few launches long.  Measured
@@ -495,6 +566,8 @@ static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
                        const gf::EpiArgs<T>& ea, const char* name, hipStream_t st,
                        size_t head_bytes = 0, WsLease* head_lease = nullptr) {
     if (M < 1 || N < 1 || K < 1 || M > INT32_MAX / 2 || N > INT32_MAX / 2) return -1;
+    if constexpr (EPI != gf::EPI_DGELU)
+        if (skinny_ok(a, b, M, N, K)) return skinny_launch<T, EPI>(a, b, M, N, K, ea, name, st);
     const bool pa = !direct_rows(a, M, K), pb = !direct_rows(b, N, K);
     // whole 16-byte pieces everywhere: nothing but split-K partials needs scratch
     const bool out_whole = N % 8 == 0 && ea.ldd % 8 == 0 && aligned_to(ea.d, 16) &&

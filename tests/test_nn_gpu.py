@@ -650,3 +650,39 @@ def test_gemm_odd_shape_ignores_what_surrounds_it():
                 nn.gemm_ex(a, b, out, trans_a=ta, trans_b=tb)
                 ref = (a.double().T if ta else a.double()) @ (b.double().T if tb else b.double())
                 assert ((out.double() - ref).norm() / ref.norm()).item() <= 2.0 ** -9
+
+
+# few rows (the kernel that streams the weights once): row counts around the
+# 16-row tiles, columns that end in a partial 32-column workgroup, both layouts
+# of the weights, every epilogue.  Bound as above: one bf16 rounding.
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 33, 64, 65])
+@pytest.mark.parametrize("k,n", [(32, 34), (1024, 264), (96, 3088), (2072, 66)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_gemm_few_rows(m, k, n, dt):
+    from ceo_amd import nn
+
+    announce(f"gemm few rows {m}x{k}x{n} {dt}")
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+
+    def r(*s):
+        return torch.randn(*s, generator=g, device="cuda").to(dt)
+
+    def off(got, ref):
+        return ((got.double() - ref).norm() / ref.norm()).item()
+
+    a, b, bt, bias, c = r(m, k), r(k, n), r(n, k), r(n), r(m, n)
+    A, B, Bt = a.double(), b.double(), bt.double()
+    errs = {"fwd": off(nn.gemm_forward(a, b, bias), A @ B + bias.double()),
+            "bt": off(nn.gemm_ex(a, bt, torch.empty_like(c), trans_b=True), A @ Bt.T)}
+    ref = 0.5 * (A @ B) + bias.double() + 2 * c.double()
+    nn.gemm_ex(a, b, c, bias=bias, c=c, alpha=0.5, beta=2.0)  # over its own residual
+    errs["ex"] = off(c, ref)
+    if dt == torch.bfloat16:
+        pre, act = nn.gemm_gelu_forward(a, b, bias)
+        errs["pre"] = off(pre, A @ B + bias.double())
+        errs["gelu"] = off(act, torch.nn.functional.gelu(pre.double(), approximate="tanh"))
+    print("  rel-L2:", {n_: f"{v:.2e}" for n_, v in errs.items()}, flush=True)
+    assert all(v <= 2.0 ** -9 for v in errs.values()), errs
+    if m <= 64:  # a row does not depend on how many others there are
+        assert torch.equal(nn.gemm_forward(a[:1].contiguous(), b, bias),
+                           nn.gemm_forward(a, b, bias)[:1])

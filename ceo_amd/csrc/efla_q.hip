@@ -35,6 +35,7 @@
 #include "efla_q_seq.hpp"
 #include "efla_q_fast.hpp"
 #include "efla_q_bwd.hpp"
+#include "efla_q_step.hpp"
 
 namespace efla {
 namespace q {
@@ -1051,6 +1052,28 @@ static int run_bwd(const Problem& p, const T* q, const T* k, const T* v, const T
     return (int)hipPeekAtLastError();
 }
 
+// A few tokens continued from a carried state (efla_q_step.hpp).  The line:
+// up to kStepTokens tokens per sequence; the step kernel's time grows with the
+// tokens, the chunked path's is that of one 64-token chunk whatever their
+// number.  Measured (step / chunked, us; sequences x heads, K x V):
+//                          1 token      4 tokens     8 tokens     12 tokens
+//   64 x 16, 128 x 128   22.2 / 59.9  37.5 / 59.0  54.3 / 60.3  71.5 / 59.1
+//    8 x 16, 128 x 128    4.8 / 13.4   9.1 / 13.6  14.9 / 13.9  20.8 / 13.6
+//    1 x  4,  64 x  64    3.2 / 10.0   6.7 / 10.0  11.3 / 10.0  16.3 /  9.9
+//  256 x  8,  64 x 128   22.5 / 75.5  43.2 / 74.5  73.5 / 74.8 103.3 / 75.1
+// Only continuations (an initial state) of equal-length sequences take it: a
+// sequence run from its start gives the same bits alone and in a packed batch.
+constexpr long kStepTokens = 6;
+
+template <typename T, int K, int V>
+static int run_step(const Problem& p, const T* q, const T* k, const T* v, const T* beta,
+                    const float* S0, T* o, float* ST, hipStream_t st) {
+    EFLA_LAUNCH("efla_q_fwd_step", (step::step_kernel<T, K, V>),
+                dim3((unsigned)p.N * p.H * (V / step::VS)), dim3(step::NT), st, q, k, v, beta,
+                p.T, p.H, S0, ST, o, p.ld);
+    return (int)hipPeekAtLastError();
+}
+
 // (dtype, K, V) combinations compiled in.
 static bool supported(int dtype, size_t K, size_t V) {
     if (dtype == kDtypeBF16)
@@ -1197,7 +1220,8 @@ static int chunk_fwd(const void* q, const void* k, const void* v, const void* be
                      const int32_t* cu_seqlens, size_t batch_size, size_t seq_len,
                      size_t num_seqs, size_t num_heads, size_t head_dim_k, size_t head_dim_v,
                      size_t chunk_size, int dtype, void* workspace, size_t workspace_bytes,
-                     unsigned flags, const int64_t* token_strides, hipStream_t stream) {
+                     unsigned flags, const int64_t* token_strides, hipStream_t stream,
+                     bool scratch_only = false) {
     Problem p;
     bool empty;
     int rc = make_problem(q, k, v, beta, cu_seqlens, batch_size, seq_len, num_seqs, num_heads,
@@ -1220,6 +1244,20 @@ static int chunk_fwd(const void* q, const void* k, const void* v, const void* be
         return fill_zero(final_state, sbytes, stream);
     }
     if (output == nullptr) return kInvalidValue;
+    // a short continuation whose workspace nobody reads afterwards (a caller's
+    // workspace must end up holding T and b for a backward)
+    if (initial_state && !p.varlen && p.T <= kStepTokens && !save &&
+        (workspace == nullptr || scratch_only)) {
+        if (dtype == kDtypeBF16)
+            EFLA_Q_DISPATCH_BF16(run_step, p, (const bf16*)q, (const bf16*)k, (const bf16*)v,
+                                 (const bf16*)beta, initial_state, (bf16*)output, final_state,
+                                 stream);
+        else
+            return run_step<float, 64, 64>(p, (const float*)q, (const float*)k, (const float*)v,
+                                           (const float*)beta, initial_state, (float*)output,
+                                           final_state, stream);
+        return kInvalidValue;
+    }
     const size_t need = dtype == kDtypeBF16 ? carve_fwd<bf16>(p, nullptr, nullptr, save)
                                             : carve_fwd<float>(p, nullptr, nullptr, save);
     void* ws = workspace;
@@ -1371,7 +1409,7 @@ extern "C" int efla_chunk_fwd_noalloc_hip(const void* q, const void* k, const vo
     // so nothing has to be cleared between calls
     return chunk_fwd(q, k, v, beta, initial_state, output, final_state, cu_seqlens, batch_size,
                      seq_len, num_seqs, num_heads, head_dim_k, head_dim_v, chunk_size, dtype,
-                     scr, EFLA_NOALLOC_SCRATCH_BYTES, 0u, nullptr, stream);
+                     scr, EFLA_NOALLOC_SCRATCH_BYTES, 0u, nullptr, stream, true);
 }
 
 extern "C" int efla_chunk_fwd_strided_hip(

@@ -468,3 +468,43 @@ def test_token_stride_rejects_other_layouts():
         token_stride(x.transpose(1, 2))  # heads outside the token row
     with pytest.raises(ValueError):
         token_stride(torch.zeros(3, 5, 3, 64, device="cuda:0")[::2])  # a gap between batches
+
+
+# A few tokens from a carried state: around the longest that the step kernel
+# takes, the smallest problem, each state shape, fused projection rows.  Its
+# state stays in fp32 throughout: S_T to 1e-5 (K + T fp32 sums of 128 terms);
+# the bf16 output is rounded once, to 2^-9.
+@pytest.mark.parametrize("T", [1, 2, 5, 6, 7])
+@pytest.mark.parametrize("dtype,K,V", [(torch.bfloat16, 64, 64), (torch.bfloat16, 64, 256),
+                                       (torch.bfloat16, 128, 128), (torch.bfloat16, 128, 64),
+                                       (torch.float32, 64, 64)])
+def test_steps_from_carried_state(oracle, dtype, K, V, T):
+    from ceo_amd.efla import chunk_efla_fwd
+
+    B, H = (1, 1) if T == 2 else (3, 5)
+    announce(f"steps from a carried state B={B} T={T} H={H} K={K} V={V} {dtype}")
+    x = oracle.make_efla_inputs(0x57E9 + T, B * T, H, K, V, bf16=dtype == torch.bfloat16)
+    x["k"].reshape(B * T, H, K)[0, 0] = 0.0  # lambda = 0
+    x["beta"].reshape(B * T, H)[-1, -1] = 0.0
+    S0 = (np.random.default_rng(3).standard_normal((B, H, K, V)) * 0.5).astype(np.float32)
+    shapes = {"q": (B, T, H, K), "k": (B, T, H, K), "v": (B, T, H, V), "beta": (B, T, H)}
+    g = {n: to_dev(x[n], dtype, s) for n, s in shapes.items()}
+    s0 = torch.from_numpy(S0).cuda()
+    o, st = chunk_efla_fwd(g["q"], g["k"], g["v"], g["beta"], s0, True)
+    torch.cuda.synchronize()
+    ro, rst = oracle.q_forward(x["q"], x["k"], x["v"], x["beta"], S0=S0, T=T)
+    eo, es = rel_l2(o, ro), rel_l2(st, rst)
+    print(f"  rel-L2 o {eo:.2e} S_T {es:.2e}", flush=True)
+    steps = T <= 6
+    assert eo <= (1e-5 if dtype == torch.float32 else 2.0 ** -9 if steps else TOL[dtype])
+    assert es <= (1e-5 if dtype == torch.float32 or steps else TOL[dtype])
+    assert torch.equal(s0, torch.from_numpy(S0).cuda())
+    if dtype == torch.bfloat16:
+        # the same from column slices of one row per token
+        row = torch.zeros(B * T, H * (2 * K + V) + 8, dtype=dtype, device="cuda")
+        q, k, v = (row[:, a:a + n].view(B, T, H, -1) for a, n in
+                   ((0, H * K), (H * K, H * K), (2 * H * K, H * V)))
+        for t, n in ((q, "q"), (k, "k"), (v, "v")):
+            t.copy_(g[n])
+        o2, st2 = chunk_efla_fwd(q, k, v, g["beta"], s0, True)
+        assert torch.equal(o, o2) and torch.equal(st, st2)

@@ -832,6 +832,7 @@ struct Problem {
     long slots;     // chunk slots launched for per-chunk kernels
     int nt;         // chunks per sequence (fixed-length case)
     TokLd ld;       // token strides of q, k, v, dq, dk, dv (bf16 path)
+    int nseg = 1, segc = 0;  // segments per sequence of the scans (plan_segments)
 };
 
 // Workspace layouts.  The forward's layout is a prefix of the backward's:
@@ -843,6 +844,7 @@ template <typename T>
 struct FwdWs {
     int32_t *cu_s, *coff, *order;
     T *W, *U;     // generic path
+    float *segX, *segM;  // bf16 path, sequences in segments
     bf16* Tc;     // bf16 path
     float* bc;    // bf16 path
     float* dcc;   // bf16 path: dc/dlambda, dc/dbeta per token
@@ -856,6 +858,7 @@ template <typename T>
 struct BwdWs {
     int32_t *cu_s, *coff, *order;
     T *W, *U;
+    float *segX, *segM;  // bf16 path, sequences in segments
     bf16* Tc;
     float* bc;
     float* dcc;  // bf16 path: dc/dlambda, dc/dbeta per token, as the forward's prep wrote them
@@ -900,6 +903,16 @@ static void carve_prefix(const Problem& p, Carve& c, int32_t** cu_s, int32_t** c
     }
 }
 
+// The segments' start states and transitions (with one segment: nothing).  They
+// end the layout, behind what a forward hands to its backward.
+static void carve_segments(const Problem& p, Carve& c, float** X, float** M) {
+    *X = *M = nullptr;
+    if (p.nseg <= 1) return;
+    const size_t n = (size_t)p.N * p.nseg * p.H;
+    *X = c.take<float>(n * p.K * p.V);
+    *M = c.take<float>(n * p.K * p.K);
+}
+
 // with_states: room for the bf16 path's chunk states (the generic path always
 // keeps them)
 template <typename T>
@@ -908,6 +921,7 @@ static size_t carve_fwd(const Problem& p, void* base, FwdWs<T>* out, bool with_s
     FwdWs<T> w{};
     carve_prefix<T>(p, c, &w.cu_s, &w.coff, &w.order, &w.W, &w.U, &w.Tc, &w.bc, &w.dcc,
                     &w.bco, &w.h, &w.Pc, &w.Vn, with_states);
+    carve_segments(p, c, &w.segX, &w.segM);
     if (out) *out = w;
     return c.off + 256;
 }
@@ -925,6 +939,7 @@ static size_t carve_bwd(const Problem& p, void* base, BwdWs<T>* out) {
         w.dW = c.take<T>((size_t)p.ntok * p.H * p.K);
         w.dKp = c.take<float>((size_t)p.ntok * p.H * p.K);
     }
+    carve_segments(p, c, &w.segX, &w.segM);
     if (out) *out = w;
     return c.off + 256;
 }
@@ -941,7 +956,82 @@ static SeqInfo make_seqinfo(const Problem& p, const int32_t* cu_s, const int32_t
     s.N = p.N;
     s.T = p.T;
     s.nt = p.nt;
+    s.nseg = p.varlen ? 1 : p.nseg;
+    s.segc = p.varlen || p.nseg == 1 ? p.nt : p.segc;
     return s;
+}
+
+// How many segments the bf16 scans cut a sequence of a fixed-length batch
+// into.  A scan is one chain of dependent chunks per (sequence, head, 64 value
+// columns): with few of them most CUs idle and the call takes nt chunk times.
+// In segments it takes a first pass over all but one segment (states from
+// zero and K x K transitions), a combine over the segments and the scan proper
+// from the true start states, nt / nseg chunk times each:
+//   nt * scan   against   segc * (pass + scan) + nseg * comb + 12 us
+// with the chunk times of a lone workgroup, scan and pass 2.0 and 1.4 us
+// (d_k = 128) or 1.4 and 0.8 (d_k = 64); the pass's longer where it has more
+// workgroups than the CUs.  Measured, forward / forward + backward (us), by
+// number of segments:
+//   sequences x tokens x heads, K x V          1          3          4          8
+//   1 x 8100 x 16, 128 x 128 (32 chains)   285 / 633  184 / 465  151 / 396  127 / 364
+//   1 x 2048 x 16, 128 x 128                78 / 164   63 / 143   57 / 132   61 / 147
+//   1 x 1024 x  4, 128 x 128                43 / 86    41 / 90    38 / 83
+//   1 x 16384 x 2, 128 x 256               533 / 1012 315 / 655  243 / 516  149 / 327
+//   1 x 4096 x  8,  64 x 64                102 / 206   69 / 156   57 / 128   42 / 96
+//   1 x 8192 x 32, 128 x 128 (64 chains)   320 / 788  211 / 607  205 / 634  223 / 672
+// The scan's workgroups stay at one per CU (its LDS allows no more).  The
+// plan depends on nothing but the problem's shape and the device, so every call
+// on a problem, with saved states or without, gives the same bits; it keeps
+// the forward's scratch within the fixed array of the entry that allocates
+// nothing, whose results are the same too.
+static void plan_segments(Problem* p, int dtype) {
+    p->nseg = 1;
+    p->segc = p->nt;
+    if (dtype != kDtypeBF16 || p->varlen || p->nt < 16) return;
+    const double scan = p->K == 128 ? 2.0 : 1.4, pass = p->K == 128 ? 1.4 : 0.8,
+                 comb = p->K == 128 ? 2.0 : 1.0, launches = 12., margin = 1.1;
+    const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    const long chains = (long)p->N * p->H * (p->V / 64);
+    const long pass_chains = (long)p->N * p->H * ((p->V + p->K) / 64);
+    double best = p->nt * scan / margin;
+    for (int n = 3; n <= 32 && (long)n * chains <= cus; ++n) {
+        const int segc = (p->nt + n - 1) / n;
+        if ((p->nt + segc - 1) / segc != n) continue;
+        const long w = pass_chains * (n - 1);  // two of the pass's workgroups fit on a CU
+        const double slow = w <= cus ? 1. : 2. * (double)((w + 2 * cus - 1) / (2 * cus));
+        const double t = segc * (slow * pass + scan) + n * comb + launches;
+        if (t >= best) continue;
+        Problem trial = *p;
+        trial.nseg = n;
+        if (carve_fwd<bf16>(trial, nullptr, nullptr, false) > EFLA_NOALLOC_SCRATCH_BYTES) continue;
+        best = t;
+        p->nseg = n;
+        p->segc = segc;
+    }
+}
+
+// The first pass and the combine over the segments' states, forward ...
+template <int K, int V>
+static void seg_forward(const Problem& p, const SeqInfo& si, const bf16* k, const bf16* v,
+                        const bf16* Tc, const float* bc, const float* S0, const fast::SegOut& seg,
+                        const char* pass, hipStream_t st) {
+    EFLA_LAUNCH(pass, (fast::scan_h_kernel<K, V, true>),
+                dim3(p.N * (p.nseg - 1) * p.H * ((V + K) / fast::VS)), dim3(fast::NT), st, k, v,
+                Tc, bc, si, p.H, S0, (bf16*)nullptr, p.ld, seg);
+    EFLA_LAUNCH("efla_q_seg_combine", (fast::seg_combine_kernel<K, V, false>),
+                dim3(p.N * p.H * (V / 16)), dim3(256), st, seg, p.nseg, p.H, S0);
+}
+// ... and backwards
+template <int K, int V, bool PS>
+static void seg_backward(const Problem& p, const SeqInfo& si, const bf16* q, const bf16* k,
+                         const bf16* dO, const bf16* Tc, const float* bc, const bf16* Pc,
+                         const float* dST, const fast::SegOut& seg, hipStream_t st) {
+    EFLA_LAUNCH("efla_q_bwd_seg", (fast::scan_dh_kernel<K, V, PS, true>),
+                dim3(p.N * (p.nseg - 1) * p.H * ((V + K) / fast::VS)),
+                dim3(fast::dh_threads<K>()), st, q, k, dO, Tc, bc, Pc, si, p.H, dST,
+                (float*)nullptr, (bf16*)nullptr, p.ld, seg);
+    EFLA_LAUNCH("efla_q_seg_combine", (fast::seg_combine_kernel<K, V, true>),
+                dim3(p.N * p.H * (V / 16)), dim3(256), st, seg, p.nseg, p.H, dST);
 }
 
 static int build_offsets(const Problem& p, const int32_t* cu, int32_t* cu_s, int32_t* coff,
@@ -964,9 +1054,14 @@ static int run_fwd(const Problem& p, const T* q, const T* k, const T* v, const T
     if constexpr (__is_same(T, bf16)) {
         EFLA_LAUNCH("efla_q_fwd_prep", (fast::prep_kernel<K>), dim3(H, p.slots),
                     dim3(fast::NT), st, k, beta, si, H, w.Tc, w.bc, w.dcc, p.ld.k);
+        const float* start = S0;
+        if (si.nseg > 1) {
+            seg_forward<K, V>(p, si, k, v, w.Tc, w.bc, S0, {w.segX, w.segM}, "efla_q_fwd_seg", st);
+            start = w.segX;
+        }
         EFLA_LAUNCH("efla_q_fwd_scan", (fast::scan_o_kernel<K, V>),
-                    dim3(p.N * H * (V / fast::VS)), dim3(fast::NTS), st, q, k, v, w.Tc, w.bc, si,
-                    H, S0, ST, o, w.h, w.Pc, p.ld);
+                    dim3(p.N * si.nseg * H * (V / fast::VS)), dim3(fast::NTS), st, q, k, v, w.Tc,
+                    w.bc, si, H, start, ST, o, w.h, w.Pc, p.ld);
         return (int)hipPeekAtLastError();
     }
     EFLA_LAUNCH("efla_q_fwd_prep", (fwd_prep_kernel<T, K, V>), dim3(p.slots, H), dim3(NTH), st,
@@ -991,14 +1086,25 @@ static int run_bwd(const Problem& p, const T* q, const T* k, const T* v, const T
     // forward recompute: the WY factors unless the forward's are in the
     // workspace (reuse), the chunk states unless the forward saved them
     if constexpr (__is_same(T, bf16)) {
-        const dim3 scan_grid(p.N * H * (V / fast::VS));
+        const dim3 scan_grid(p.N * si.nseg * H * (V / fast::VS));
+        const fast::SegOut seg{w.segX, w.segM};
         if (!reuse)
             EFLA_LAUNCH("efla_q_bwd_re_prep", (fast::prep_kernel<K>), dim3(H, p.slots),
                         dim3(fast::NT), st, k, beta, si, H, w.Tc, w.bc, w.dcc, p.ld.k);
-        if (!reuse_states)
-            EFLA_LAUNCH("efla_q_bwd_re_state", (fast::scan_h_kernel<K, V>), scan_grid,
+        if (!reuse_states) {
+            if (si.nseg > 1)
+                seg_forward<K, V>(p, si, k, v, w.Tc, w.bc, S0, seg, "efla_q_bwd_re_seg", st);
+            EFLA_LAUNCH("efla_q_bwd_re_state", (fast::scan_h_kernel<K, V, false>), scan_grid,
                         dim3(fast::NT), st, k, v, (const bf16*)w.Tc, (const float*)w.bc, si, H,
-                        S0, w.h, p.ld);
+                        si.nseg > 1 ? (const float*)w.segX : S0, w.h, p.ld, fast::SegOut{});
+        }
+        if (si.nseg > 1) {
+            if (reuse_states)
+                seg_backward<K, V, true>(p, si, q, k, dO, w.Tc, w.bc, w.Pc, dST, seg, st);
+            else
+                seg_backward<K, V, false>(p, si, q, k, dO, w.Tc, w.bc, nullptr, dST, seg, st);
+        }
+        const float* end = si.nseg > 1 ? (const float*)w.segX : dST;
         // persistent gradient kernel: one workgroup per CU (its LDS allows no
         // more), each looping over (chunk, head) items.  EFLA_GRAD_WORKGROUPS
         // caps the grid (tests use it to run many items per workgroup at
@@ -1015,17 +1121,17 @@ static int run_bwd(const Problem& p, const T* q, const T* k, const T* v, const T
         // allow it without spills (d_v <= 128), else 8
         constexpr int NG = V <= 128 ? 4 : 2;
         if (reuse_states) {
-            EFLA_LAUNCH("efla_q_bwd_state", (fast::scan_dh_kernel<K, V, true>), scan_grid,
+            EFLA_LAUNCH("efla_q_bwd_state", (fast::scan_dh_kernel<K, V, true, false>), scan_grid,
                         dim3(fast::dh_threads<K>()), st, q, k, dO, (const bf16*)w.Tc, (const float*)w.bc,
-                        (const bf16*)w.Pc, si, H, dST, dS0, w.dh, p.ld);
+                        (const bf16*)w.Pc, si, H, end, dS0, w.dh, p.ld, fast::SegOut{});
             EFLA_LAUNCH("efla_q_bwd_grad", (fast::grad_kernel<K, V, true, NG>), grad_grid,
                         dim3(fast::grad_threads<NG>()), st, q, k, v, dO, (const bf16*)w.Tc,
                         (const float*)w.bc, (const float*)w.dcc, (const bf16*)w.Pc, w.h, w.dh,
                         si, H, nitems, dq, dk, dv, dbeta, p.ld);
         } else {
-            EFLA_LAUNCH("efla_q_bwd_state", (fast::scan_dh_kernel<K, V, false>), scan_grid,
+            EFLA_LAUNCH("efla_q_bwd_state", (fast::scan_dh_kernel<K, V, false, false>), scan_grid,
                         dim3(fast::dh_threads<K>()), st, q, k, dO, (const bf16*)w.Tc, (const float*)w.bc,
-                        (const bf16*)nullptr, si, H, dST, dS0, w.dh, p.ld);
+                        (const bf16*)nullptr, si, H, end, dS0, w.dh, p.ld, fast::SegOut{});
             EFLA_LAUNCH("efla_q_bwd_grad", (fast::grad_kernel<K, V, false, NG>), grad_grid,
                         dim3(fast::grad_threads<NG>()), st, q, k, v, dO, (const bf16*)w.Tc,
                         (const float*)w.bc, (const float*)w.dcc, (const bf16*)nullptr, w.h, w.dh,
@@ -1131,6 +1237,7 @@ static int make_problem(const void* q, const void* k, const void* v, const void*
                   (long)(H * V)};
     if ((size_t)p->N * H > (size_t)INT32_MAX || (size_t)p->slots > (size_t)INT32_MAX)
         return kInvalidConfiguration;
+    plan_segments(p, dtype);
     if (seq_len == 0) {
         *empty = true;
         return kSuccess;
@@ -1165,6 +1272,7 @@ static bool ws_problem(size_t batch, size_t seq_len, size_t num_seqs, size_t H, 
     const size_t fixed = batch * (size_t)p->nt;
     const size_t packed = ntok / BT + N;
     p->slots = (long)(fixed > packed ? fixed : packed);
+    plan_segments(p, dtype);
     return true;
 }
 
@@ -1258,8 +1366,16 @@ static int chunk_fwd(const void* q, const void* k, const void* v, const void* be
                                            final_state, stream);
         return kInvalidValue;
     }
-    const size_t need = dtype == kDtypeBF16 ? carve_fwd<bf16>(p, nullptr, nullptr, save)
-                                            : carve_fwd<float>(p, nullptr, nullptr, save);
+    auto size = [&] {
+        return dtype == kDtypeBF16 ? carve_fwd<bf16>(p, nullptr, nullptr, save)
+                                   : carve_fwd<float>(p, nullptr, nullptr, save);
+    };
+    size_t need = size();
+    if (workspace && workspace_bytes < need && p.nseg > 1) {  // room for one chain only
+        p.nseg = 1;
+        p.segc = p.nt;
+        need = size();
+    }
     void* ws = workspace;
     WsLease lease;
     if (ws == nullptr) {
@@ -1313,8 +1429,16 @@ static int chunk_bwd(const void* q, const void* k, const void* v, const void* be
         return fill_zero(grad_initial_state, sbytes, stream);
     }
     if (!grad_output || !grad_q || !grad_k || !grad_v || !grad_beta) return kInvalidValue;
-    const size_t need = dtype == kDtypeBF16 ? carve_bwd<bf16>(p, nullptr, nullptr)
-                                            : carve_bwd<float>(p, nullptr, nullptr);
+    auto size = [&] {
+        return dtype == kDtypeBF16 ? carve_bwd<bf16>(p, nullptr, nullptr)
+                                   : carve_bwd<float>(p, nullptr, nullptr);
+    };
+    size_t need = size();
+    if (workspace && workspace_bytes < need && p.nseg > 1) {  // room for one chain only
+        p.nseg = 1;
+        p.segc = p.nt;
+        need = size();
+    }
     void* ws = workspace;
     WsLease lease;
     if (ws == nullptr) {

@@ -70,30 +70,152 @@ struct ScanHSmem {
     ScanHBuf<K> buf[2];  // chunk n in buf[n & 1]
 };
 
-template <int K, int V>
+//
+// SEG (scan_h_kernel and scan_dh_kernel): the first pass over a sequence cut
+// into segments (SeqInfo::nseg).  Nothing is written per chunk; each segment
+// but the last of the pass gives, in fp32, the state it ends with from a zero
+// start (the true start for the first one) to seg.X and, from extra slices that
+// carry the identity with all values zero, its transition K x K to seg.M.
+struct SegOut {
+    float* X;  // [seq][segment][head][K][V]: the state the segment starts its scan with
+    float* M;  // [seq][segment][head][K][K]
+};
+
+// workgroup of a SEG pass -> segment, head, slice (values, then transition
+// columns); false where there is nothing to do
+template <int K, int V, bool REV>
+__device__ __forceinline__ bool seg_map(const SeqInfo& si, int H, int& seq, int& h, int& vsl,
+                                        bool& trans, bool& first) {
+    constexpr int NVS = V / VS;
+    int bh;
+    scan_map(blockIdx.x, si.N * (si.nseg - 1) * H, NVS + K / VS, bh, vsl);
+    const int u = bh / H, p = u % (si.nseg - 1) + (REV ? 1 : 0);
+    h = bh % H;
+    seq = u / (si.nseg - 1) * si.nseg + p;
+    first = p == (REV ? si.nseg - 1 : 0);
+    trans = vsl >= NVS;
+    if (trans) vsl -= NVS;
+    return !(trans && first);
+}
+
+// a SEG pass's results: segment `seq`'s end state of slice columns v0.. to the
+// next segment's X, or its transition columns to its own M
+template <int K, int V, bool REV>
+__device__ __forceinline__ void seg_store(const SegOut& seg, int seq, int h, int H, bool trans,
+                                          int vcol, const floatx4* S) {
+    const int g = mf::lane() >> 4, ldo = trans ? K : V;
+    float* dst = (trans ? seg.M + ((long)seq * H + h) * K * K
+                        : seg.X + ((long)(seq + (REV ? -1 : 1)) * H + h) * K * V) + vcol;
+#pragma unroll
+    for (int fb = 0; fb < K / 16; ++fb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dst[(long)pim(fb, 4 * g + i) * ldo] = S[fb][i];
+}
+
+// The segments' start states, in the order of the scan (j = 0 .. nseg - 1;
+// segment j, or nseg - 1 - j for REV): X[0] = S0 (or 0), X[1] is in place (the
+// first pass ran segment 0 from S0), X[j + 1] += M[j] X[j].  All in fp32 (fp32
+// MFMA): a workgroup carries 16 state columns of one (sequence, head) through
+// the segments, its four waves a quarter of the rows each; the column block
+// sits in LDS between segments, the next segment's M rows and X are loaded
+// during the current product.  nseg - 2 dependent products of K x K x 16,
+// about 2 us each (K = 128; 1 us for K = 64).
+template <int K, int V, bool REV>
+__global__ void __launch_bounds__(256) seg_combine_kernel(SegOut seg, int nseg, int H,
+                                                          const float* __restrict__ S0) {
+    constexpr int RT = K / 64;  // 16-row tiles per wave
+    __shared__ float X[2][K][16 + 1];
+    const int w = mf::wave(), l = mf::lane(), g = l >> 4, r = l & 15;
+    constexpr int NC = V / 16;
+    const int col = (int)(blockIdx.x % NC) * 16 + r;
+    const int bh = blockIdx.x / NC, seq = bh / H, h = bh % H;
+    auto at = [&](int j) {
+        return (long)(seq * nseg + (REV ? nseg - 1 - j : j)) * H + h;
+    };
+    // X[0]
+    float* x0 = seg.X + at(0) * K * V + col;
+    const float* s0 = S0 ? S0 + (long)bh * K * V + col : nullptr;
+    for (int row = threadIdx.x >> 4; row < K; row += 16)
+        x0[(long)row * V] = s0 ? s0[(long)row * V] : 0.f;
+    floatx4 m[RT][K / 16], c[RT];
+    auto fetch = [&](int j) {  // M[j]'s rows and X[j + 1]
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            const int row0 = 16 * (w + 4 * t);
+            const float* mp = seg.M + at(j) * K * K + (long)(row0 + r) * K + 4 * g;
+#pragma unroll
+            for (int i = 0; i < K / 16; ++i) m[t][i] = *reinterpret_cast<const floatx4*>(mp + 16 * i);
+            const float* xp = seg.X + at(j + 1) * K * V + (long)(row0 + 4 * g) * V + col;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c[t][e] = xp[(long)e * V];
+        }
+    };
+    if (nseg > 2) fetch(1);
+    for (int row = threadIdx.x >> 4; row < K; row += 16)
+        X[1][row][r] = seg.X[at(1) * K * V + (long)row * V + col];
+    __syncthreads();
+    for (int j = 1; j + 1 < nseg; ++j) {
+        floatx4 a[RT];
+#pragma unroll
+        for (int t = 0; t < RT; ++t) a[t] = c[t];
+#pragma unroll
+        for (int i = 0; i < K / 16; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float xv = X[j & 1][16 * i + 4 * g + e][r];
+#pragma unroll
+                for (int t = 0; t < RT; ++t) a[t] = mma_f32(m[t][i][e], xv, a[t]);
+            }
+        if (j + 2 < nseg) fetch(j + 1);
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            const int row0 = 16 * (w + 4 * t) + 4 * g;
+            float* xp = seg.X + at(j + 1) * K * V + (long)row0 * V + col;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                xp[(long)e * V] = a[t][e];
+                X[(j + 1) & 1][row0 + e][r] = a[t][e];
+            }
+        }
+        __syncthreads();
+    }
+}
+
+template <int K, int V, bool SEG>
 __global__ void __launch_bounds__(NT) scan_h_kernel(const bf16* __restrict__ k,
                                                     const bf16* __restrict__ v,
                                                     const bf16* __restrict__ Tc,
                                                     const float* __restrict__ bc, SeqInfo si,
                                                     int H, const float* __restrict__ S0,
-                                                    bf16* __restrict__ hist, TokLd ld) {
+                                                    bf16* __restrict__ hist, TokLd ld,
+                                                    SegOut seg) {
     constexpr int LDK = ldb<K>(), NVS = V / VS;
     __shared__ __attribute__((aligned(16))) ScanHSmem<K> sm;
     const int w = mf::wave(), l = mf::lane(), g = l >> 4, r = l & 15;
-    int bh, vsl;
-    scan_map(blockIdx.x, si.N * H, NVS, bh, vsl);
-    bh = scan_seq_head(si, bh, H);
-    const int seq = bh / H, h = bh % H, v0 = vsl * VS;
+    int seq, h, vsl;
+    bool trans = false, first = true;
+    if constexpr (SEG) {
+        if (!seg_map<K, V, false>(si, H, seq, h, vsl, trans, first)) return;
+    } else {
+        int bh;
+        scan_map(blockIdx.x, si.N * si.nseg * H, NVS, bh, vsl);
+        bh = scan_seq_head(si, bh, H);
+        seq = bh / H;
+        h = bh % H;
+    }
+    const int v0 = vsl * VS;
     long sbos, slen;
     int slot0;
     seq_bounds(si, seq, sbos, slen, slot0);
     const int nch = (int)((slen + 63) / 64);
-    const long sbase = (long)bh * K * V;
+    const long sbase = ((long)(SEG ? seq / si.nseg : seq) * H + h) * K * V;
     const int vcol = v0 + 16 * w + r;
     floatx4 S[K / 16];
 #pragma unroll
-    for (int fb = 0; fb < K / 16; ++fb) S[fb] = zero4();
-    if (S0) {
+    for (int fb = 0; fb < K / 16; ++fb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[fb][i] = SEG && trans && pim(fb, 4 * g + i) == vcol ? 1.f : 0.f;
+    if (S0 && first && !trans) {
 #pragma unroll
         for (int fb = 0; fb < K / 16; ++fb)
 #pragma unroll
@@ -104,8 +226,9 @@ __global__ void __launch_bounds__(NT) scan_h_kernel(const bf16* __restrict__ k,
     auto prefetch = [&](int n) {
         const long bos = sbos + (long)n * 64;
         const int len = (int)min((long)64, slen - (long)n * 64);
-        pre.load(nullptr, k, v, Tc, bc, bos, len, h, V, v0, (long)(slot0 + n) * H + h, 0, ld.k,
-                 ld.v);
+        pre.load(nullptr, k, v, Tc, bc, bos, len, h, V, SEG && trans ? 0 : v0,
+                 (long)(slot0 + n) * H + h, 0, ld.k, ld.v);
+        if (SEG && trans) pre.rv.valid = 0;  // staged as zeros
     };
     if (nch > 0) {
         prefetch(0);
@@ -118,7 +241,7 @@ __global__ void __launch_bounds__(NT) scan_h_kernel(const bf16* __restrict__ k,
         bf16x8 sb[K / 32];
 #pragma unroll
         for (int kb = 0; kb < K / 32; ++kb) sb[kb] = frag_from_c(S[2 * kb], S[2 * kb + 1]);
-        store_state_frag<K>(hist + ((long)(slot0 + n) * H + h) * V * K, sb, vcol);
+        if constexpr (!SEG) store_state_frag<K>(hist + ((long)(slot0 + n) * H + h) * V * K, sb, vcol);
         floatx4 vn[4];
         chunk_vn<K>(cb, w, sb, vn);
         const bf16x8 vb0 = frag_from_c(vn[0], vn[1]), vb1 = frag_from_c(vn[2], vn[3]);
@@ -133,6 +256,7 @@ __global__ void __launch_bounds__(NT) scan_h_kernel(const bf16* __restrict__ k,
             if (n + 2 < nch) prefetch(n + 2);
         }
     }
+    if constexpr (SEG) seg_store<K, V, false>(seg, seq, h, H, trans, vcol, S);
 }
 
 // ---------------------------------------------------------------------------
@@ -191,7 +315,7 @@ template <int K>
 constexpr int dh_threads() {
     return dh_copy_waves<K>() ? NTS : NT;
 }
-template <int K, int V, bool PS>
+template <int K, int V, bool PS, bool SEG>
 __global__ void __launch_bounds__(dh_threads<K>()) scan_dh_kernel(const bf16* __restrict__ q,
                                                       const bf16* __restrict__ k,
                                                       const bf16* __restrict__ dO,
@@ -200,14 +324,23 @@ __global__ void __launch_bounds__(dh_threads<K>()) scan_dh_kernel(const bf16* __
                                                       const bf16* __restrict__ Pc, SeqInfo si,
                                                       int H, const float* __restrict__ dST,
                                                       float* __restrict__ dS0,
-                                                      bf16* __restrict__ dhist, TokLd ld) {
+                                                      bf16* __restrict__ dhist, TokLd ld,
+                                                      SegOut seg) {
     constexpr int LDK = ldb<K>(), NVS = V / VS;
     __shared__ __attribute__((aligned(16))) ScanDhSmem<K, PS> sm;
     const int w = mf::wave(), l = mf::lane(), g = l >> 4, r = l & 15;
-    int bh, vsl;
-    scan_map(blockIdx.x, si.N * H, NVS, bh, vsl);
-    bh = scan_seq_head(si, bh, H);
-    const int seq = bh / H, h = bh % H, v0 = vsl * VS;
+    int seq, h, vsl;
+    bool trans = false, first = true;
+    if constexpr (SEG) {
+        if (!seg_map<K, V, true>(si, H, seq, h, vsl, trans, first)) return;
+    } else {
+        int bh;
+        scan_map(blockIdx.x, si.N * si.nseg * H, NVS, bh, vsl);
+        bh = scan_seq_head(si, bh, H);
+        seq = bh / H;
+        h = bh % H;
+    }
+    const int v0 = vsl * VS;
     long sbos, slen;
     int slot0;
     seq_bounds(si, seq, sbos, slen, slot0);
@@ -226,7 +359,9 @@ __global__ void __launch_bounds__(dh_threads<K>()) scan_dh_kernel(const bf16* __
             const long bos = sbos + (long)n * 64;
             const int len = (int)min((long)64, slen - (long)n * 64);
             const long cid = (long)(slot0 + n) * H + h;
-            R.c.load(q, k, dO, Tc, bc, bos, len, h, V, v0, cid, ld.q, ld.k, (long)H * V, ct);
+            R.c.load(q, k, dO, Tc, bc, bos, len, h, V, SEG && trans ? 0 : v0, cid, ld.q, ld.k,
+                     (long)H * V, ct);
+            if (SEG && trans) R.c.rv.valid = 0;  // staged as zeros
             if constexpr (PS) load_tri(R.p, Pc + cid * TRI_ELEMS, ct);
         };
         auto stage = [&](Regs& R, ScanDhBuf<K, PS>& bf) {
@@ -258,12 +393,15 @@ __global__ void __launch_bounds__(dh_threads<K>()) scan_dh_kernel(const bf16* __
         }
         return;
     }
-    const long sbase = (long)bh * K * V;
+    const long sbase = ((long)(SEG ? seq / si.nseg : seq) * H + h) * K * V;
     const int vcol = v0 + 16 * w + r;
     floatx4 dS[K / 16];
 #pragma unroll
-    for (int fb = 0; fb < K / 16; ++fb) dS[fb] = zero4();
-    if (dST) {
+    for (int fb = 0; fb < K / 16; ++fb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            dS[fb][i] = SEG && trans && pim(fb, 4 * g + i) == vcol ? 1.f : 0.f;
+    if (dST && first && !trans) {
 #pragma unroll
         for (int fb = 0; fb < K / 16; ++fb)
 #pragma unroll
@@ -282,7 +420,9 @@ __global__ void __launch_bounds__(dh_threads<K>()) scan_dh_kernel(const bf16* __
         const long bos = sbos + (long)n * 64;
         const int len = (int)min((long)64, slen - (long)n * 64);
         const long cid = (long)(slot0 + n) * H + h;
-        pre.load(q, k, dO, Tc, bc, bos, len, h, V, v0, cid, ld.q, ld.k, (long)H * V);
+        pre.load(q, k, dO, Tc, bc, bos, len, h, V, SEG && trans ? 0 : v0, cid, ld.q, ld.k,
+                 (long)H * V);
+        if (SEG && trans) pre.rv.valid = 0;  // staged as zeros
         if constexpr (PS) load_tri(rp, Pc + cid * TRI_ELEMS);
     };
     auto stage = [&](ScanDhBuf<K, PS>& bf) {
@@ -302,7 +442,7 @@ __global__ void __launch_bounds__(dh_threads<K>()) scan_dh_kernel(const bf16* __
         bf16x8 sb[K / 32];
 #pragma unroll
         for (int kb = 0; kb < K / 32; ++kb) sb[kb] = frag_from_c(dS[2 * kb], dS[2 * kb + 1]);
-        store_state_frag<K>(dhist + ((long)(slot0 + n) * H + h) * V * K, sb, vcol);
+        if constexpr (!SEG) store_state_frag<K>(dhist + ((long)(slot0 + n) * H + h) * V * K, sb, vcol);
         // dO^T in c-order over the tokens; its partners (P, Q) are read the same way
         const bf16x8 do0 = mf::frag_trc(cb.Vs, LD64, 0, 16 * w), do1 = mf::frag_trc(cb.Vs, LD64, 32, 16 * w);
         // K dS part of dVn (P^T dO is added once P is complete); tile tb row
@@ -356,11 +496,16 @@ __global__ void __launch_bounds__(dh_threads<K>()) scan_dh_kernel(const bf16* __
             dS[fb] = acc;
         }
     }
-    if (dS0) {
+    if constexpr (SEG) {
+        seg_store<K, V, true>(seg, seq, h, H, trans, vcol, dS);
+        return;
+    }
+    if (dS0 && seq % si.nseg == 0) {
+        float* d0 = dS0 + ((long)(seq / si.nseg) * H + h) * K * V + vcol;
 #pragma unroll
         for (int fb = 0; fb < K / 16; ++fb)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) dS0[sbase + (long)pim(fb, 4 * g + i) * V + vcol] = dS[fb][i];
+            for (int i = 0; i < 4; ++i) d0[(long)pim(fb, 4 * g + i) * V] = dS[fb][i];
     }
 }
 

@@ -454,7 +454,7 @@ __global__ void __launch_bounds__(NTS) scan_o_kernel(const bf16* __restrict__ q,
     __shared__ __attribute__((aligned(16))) ScanSmem<K> sm;
     const int w = mf::wave(), l = mf::lane(), g = l >> 4, r = l & 15;
     int bh, vsl;
-    scan_map(blockIdx.x, si.N * H, NVS, bh, vsl);
+    scan_map(blockIdx.x, si.N * si.nseg * H, NVS, bh, vsl);
     bh = scan_seq_head(si, bh, H);
     const int seq = bh / H, h = bh % H, v0 = vsl * VS;
     long sbos, slen;
@@ -581,11 +581,12 @@ __global__ void __launch_bounds__(NTS) scan_o_kernel(const bf16* __restrict__ q,
             S[fb] = mma(mf::frag_tr(cb.Kr, LDK, 32, c0, 8), vb1, S[fb]);
         }
     }
-    if (ST) {
+    if (ST && seq % si.nseg == si.nseg - 1) {
+        float* st = ST + ((long)(seq / si.nseg) * H + h) * K * V + vcol;
 #pragma unroll
         for (int fb = 0; fb < K / 16; ++fb)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) ST[sbase + (long)pim(fb, 4 * g + i) * V + vcol] = S[fb][i];
+            for (int i = 0; i < 4; ++i) st[(long)pim(fb, 4 * g + i) * V] = S[fb][i];
     }
 }
 

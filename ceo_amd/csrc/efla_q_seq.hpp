@@ -22,6 +22,11 @@ struct SeqInfo {
     int N;
     long T;
     int nt;  // chunks per sequence (fixed-length case)
+    // Fixed-length case: the scans may take every sequence as nseg segments of
+    // segc chunks (the last may be shorter), one chain each; "sequence"
+    // seq * nseg + p of a scan is then segment p of sequence seq.  1 and nt
+    // where a sequence is one chain.
+    int nseg, segc;
 };
 
 constexpr int LPT_MAX_SEQS = 1024;  // one sequence per thread of the offsets kernel
@@ -35,9 +40,12 @@ __device__ __forceinline__ int scan_seq_head(const SeqInfo& s, int bh, int H) {
 __device__ __forceinline__ void seq_bounds(const SeqInfo& s, int seq, long& bos, long& len,
                                            int& slot0) {
     if (s.cu == nullptr) {
-        bos = (long)seq * s.T;
-        len = s.T;
-        slot0 = seq * s.nt;
+        const int p = seq % s.nseg;
+        seq /= s.nseg;
+        const long t0 = (long)p * s.segc * BT, left = s.T - t0, most = (long)s.segc * BT;
+        bos = (long)seq * s.T + t0;
+        len = left < most ? left : most;
+        slot0 = seq * s.nt + p * s.segc;
     } else {
         bos = s.cu[seq];
         len = (long)s.cu[seq + 1] - bos;

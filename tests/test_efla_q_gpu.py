@@ -508,3 +508,51 @@ def test_steps_from_carried_state(oracle, dtype, K, V, T):
             t.copy_(g[n])
         o2, st2 = chunk_efla_fwd(q, k, v, g["beta"], s0, True)
         assert torch.equal(o, o2) and torch.equal(st, st2)
+
+
+# Sequences long enough, and chains few enough, that the scans take each one as
+# segments (first pass from zero states, combine, second pass): ragged ends,
+# every state shape, initial and final states, and keys' steps small enough
+# (beta down to 0.02) that a segment's start state matters to its end.
+@pytest.mark.parametrize("B,T,H,K,V,slow", [(1, 4100, 2, 128, 128, False),
+                                            (1, 4100, 2, 128, 128, True),
+                                            (2, 2560, 3, 64, 64, True),
+                                            (1, 3001, 4, 128, 256, True),
+                                            (1, 2111, 1, 64, 128, False)])
+def test_segmented_scans(oracle, B, T, H, K, V, slow):
+    def small_beta(oracle_, x, bf):
+        x["beta"] = oracle_.round_bf16(x["beta"] * 0.04)
+        return x
+
+    _case(oracle, 0x5E6 + T, B, T, H, K, V, torch.bfloat16, s0=True, dst=True,
+          xform=small_beta if slow else None)
+
+
+def test_segmented_scans_same_bits_every_way(oracle):
+    """Saved states, saved factors only, nothing saved, and a workspace with
+    room for the factors but not the segments' states."""
+    from ceo_amd.efla import chunk_efla_bwd, chunk_efla_fwd, new_workspace
+
+    B, T, H, K, V = 1, 4100, 2, 128, 128
+    announce(f"segmented scans, saved / recomputed B={B} T={T} H={H} K={K} V={V}")
+    x = oracle.make_efla_inputs(4321, B * T, H, K, V, bf16=True)
+    g = {n: to_dev(a, torch.bfloat16, (B, T, H, K) if n in "qk" else
+                   (B, T, H) if n == "beta" else (B, T, H, V)) for n, a in x.items()}
+    a4 = (g["q"], g["k"], g["v"], g["beta"])
+    s0 = 0.1 * torch.randn(B, H, K, V, generator=torch.Generator().manual_seed(5)).cuda()
+    o, st = chunk_efla_fwd(*a4, s0, True)
+    ref = chunk_efla_bwd(*a4, g["do"], s0)
+    for states in (False, True):
+        ws = new_workspace(g["q"], g["v"])
+        o2, st2 = chunk_efla_fwd(*a4, s0, True, workspace=ws, save_states=states)
+        assert torch.equal(o, o2) and torch.equal(st, st2)
+        got = chunk_efla_bwd(*a4, g["do"], s0, workspace=ws, reuse_forward=True,
+                             reuse_states=states)
+        for a, b, n in zip(got, ref, ("dq", "dk", "dv", "dbeta", "dh0")):
+            assert torch.equal(a, b), n
+    # a smaller workspace is still taken: one chain per sequence
+    slots = (T + 63) // 64
+    small = torch.empty(slots * H * (5184 + 64 * 4 + 128 * 4) + 65536, dtype=torch.uint8,
+                        device="cuda:0")
+    o3, _ = chunk_efla_fwd(*a4, s0, workspace=small)
+    assert rel_l2(o3, o.float().cpu().numpy()) <= 2e-2

@@ -5,15 +5,17 @@
 //   lambda = |k_t|^2, c = c(beta, lambda)
 //   u = S^T k_t, S <- bf16(S + (c k_t)(v_t - u)^T)   (state re-rounded every token)
 //   o_t = S k_t                                        (needs d_k == d_v)
-// The work of a token is serial per (b, h), so a token's cost is its chain of
-// dependent steps.  For d = 64 and 128 (k, v, dO aligned to d / 8 bytes) the
+// The recurrence is serial per (b, h), so a token's cost is its chain of
+// dependent steps.  For d = 32, 64 and 128 (k, v, dO aligned to d / 8 bytes) the
 // state lives in registers (r_fast_kernel): consecutive lanes own one value
 // column, S^T k and the update are lane-local, and o = S k (a sum over
 // columns) is formed by MFMAs from a transposed LDS copy of the new state, one
 // barrier per token pair.  The value columns evolve independently, so when
 // B H leaves half of the CUs idle each (b, h) is split over two workgroups of
-// half the columns (their fp32 row sums meet in one zeroed fp32 buffer by
-// atomic adds, rounded once by r_combine_kernel).  Each
+// half the columns (d = 64, 128; their fp32 row sums meet in one zeroed fp32
+// buffer by atomic adds, rounded once by r_combine_kernel).  With still fewer
+// (b, h) a chain pass runs the bare recurrence first (r_chain_kernel) and the
+// token loops then run for groups of tokens at once (RGroups).  Each
 // segment's k, c k and v are staged in LDS at once, the next segment's reads
 // in flight; every token's c(beta, |k|^2) comes from a separate parallel
 // kernel.  Other d keep one workgroup per (b, h) and the state in LDS (row
@@ -25,8 +27,9 @@
 // The backward recomputes states from bf16 checkpoints (exact, since the
 // states are bf16 values), rebuilds one segment's states at a time into a
 // workspace, and runs the reference's BPTT (efla.cu:315-454) over the segment
-// in reverse: for d = 64 / 128 with 32-token segments, dL/dS in fp32
-// registers and the same column split (r_ckpt_kernel for the checkpoints,
+// in reverse: for d = 32 / 64 / 128 with 32-token segments, dL/dS in fp32
+// registers and the same column split and groups (r_chain_kernel for the
+// checkpoints and the groups' dL/dS, which is affine and never rounded;
 // r_bwd_fast_kernel: a barrier-free rebuild, one barrier per reverse token),
 // otherwise with 64-token segments and dL/dS in LDS (d <= 128) or the
 // workspace (d <= 256).
@@ -44,7 +47,7 @@ namespace r {
 constexpr int NTH = 256;
 constexpr int MAXD = 256;
 constexpr int SEG = 64;   // checkpoint spacing of the backward
-constexpr int SEGF = 32;  // the same for the register-resident backward (d = 64, 128)
+constexpr int SEGF = 32;  // the same for the register-resident backward (d = 32, 64, 128)
 
 __device__ __forceinline__ float block_sum(float x, float* red) {
     // wave reduction then across the 4 waves
@@ -141,12 +144,12 @@ __global__ void __launch_bounds__(NTH) r_forward_kernel(const bf16* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// forward, register-resident state (d = 64 or 128; other d take
+// forward, register-resident state (d = 32, 64 or 128; other d take
 // r_forward_kernel)
 // ---------------------------------------------------------------------------
 // c(beta, |k_t|^2) of every token, [b * H + h][t] (fp32), and dc/dlambda
 // when dcout is set: 16 lanes per
-// (token, head) row of d = 16 P values (P = 4 or 8), 16-byte loads, the
+// (token, head) row of d = 16 P values (P = 2, 4 or 8), P values per lane, the
 // squares summed per lane and then across the 16 lanes.
 template <int P>
 __global__ void __launch_bounds__(NTH) r_coeff_kernel(const bf16* __restrict__ k,
@@ -329,6 +332,23 @@ struct SegRows {
     }
 };
 
+// Token groups.  The state's recurrence is a chain over the tokens whatever
+// is done; its outputs are not.  With few (b, h), whose token loops leave CUs
+// idle, a chain pass (r_chain_kernel: no outputs, no barriers, more workgroups
+// per (b, h)) first runs the recurrences alone and leaves the state, and for the
+// backward dL/dS, where groups of `segs` segments of SEGF tokens begin and end;
+// the token loops then run once per group, all groups at once.  The chain pass
+// forms every column by the same operations in the same order as the token
+// loops, so the results are the same bits as with one group.
+struct RGroups {
+    int nbh;          // B H
+    int n, segs;      // groups per (b, h); segments per group
+    const bf16* ck;   // n > 1: start states [bh][group], column-major (the backward: of
+                      // every segment)
+    const float* gck; // the backward, n > 1: dL/dS after each group but the last
+                      // [bh][group], column-major
+};
+
 template <int D, int NS, int SG>
 struct RFastSmem {
     static constexpr bool CKS = NS > 1;  // c k staged (fp32); else formed per row
@@ -342,28 +362,38 @@ template <int D, int NS, int LPC, int SG>
 __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_fast_kernel(
     const bf16* __restrict__ k, const bf16* __restrict__ v, const float* __restrict__ coef,
     bf16* __restrict__ state, bf16* __restrict__ out, float* __restrict__ part_out,
-    int H, long T) {
+    int H, long Tall, RGroups gr) {
     constexpr int NC = D / NS, NT = rfast_threads<D, NS, LPC>(), NW = NT / 64;
     constexpr int RPL = D / LPC, NP = RPL / 2, LDS = D + 8;
     constexpr bool CKS = RFastSmem<D, NS, SG>::CKS;
-    static_assert(RPL % 8 == 0 && (D == 64 || D == 128) && NC % 32 == 0 && NT % 64 == 0 &&
-                      NT <= 1024 && D % (16 * NW) == 0 && SG % 2 == 0,
-                  "d = 64 or 128, 32-column multiples per workgroup");
+    static_assert(RPL % 8 == 0 && (D == 32 || D == 64 || D == 128) && NC % 32 == 0 &&
+                      NT % 64 == 0 && NT <= 1024 && D % (16 * NW) == 0 && SG % 2 == 0,
+                  "d = 32, 64 or 128, 32-column multiples per workgroup");
     __shared__ __attribute__((aligned(16))) RFastSmem<D, NS, SG> sm;
     const int tid = threadIdx.x, w = mf::wave(), l = mf::lane();
-    const int bh = blockIdx.x / NS, cb = blockIdx.x % NS;
+    const int item = blockIdx.x / NS, cb = blockIdx.x % NS;
+    const int grp = item / gr.nbh, bh = item - grp * gr.nbh;
     const int col = cb * NC + tid / LPC, lcol = tid / LPC, part = tid % LPC, r0 = part * RPL;
     const int b = bh / H, h = bh % H;
-    const long dd = (long)D * D, nsegf = (T + SG - 1) / SG;
+    // this workgroup's tokens: tb .. T - 1
+    const long tb = (long)grp * gr.segs * SEGF;
+    const long T = tb + (long)gr.segs * SEGF < Tall ? tb + (long)gr.segs * SEGF : Tall;
+    const long dd = (long)D * D, nsegf = (T - tb + SG - 1) / SG;
     const long tstride = (long)H * D;  // elements between tokens
-    const long base0 = (long)b * T * tstride + (long)h * D;
-    const float* cbh = coef + (long)bh * T;
+    const long base0 = (long)b * Tall * tstride + (long)h * D;
+    const float* cbh = coef + (long)bh * Tall;
     bf16* st = state + (long)bh * dd;
 
     bf16x2 Sp[NP];  // rows r0 + 2p (low half) and r0 + 2p + 1 (high half)
+    if (gr.n > 1) {  // the group's start state from the chain pass
+        const bf16* cp = gr.ck + ((long)bh * gr.n + grp) * dd + (long)col * D + r0;
 #pragma unroll
-    for (int p = 0; p < NP; ++p)
-        Sp[p] = bf16x2{st[(long)(r0 + 2 * p) * D + col], st[(long)(r0 + 2 * p + 1) * D + col]};
+        for (int p = 0; p < NP; ++p) Sp[p] = bf16x2{cp[2 * p], cp[2 * p + 1]};
+    } else {
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+            Sp[p] = bf16x2{st[(long)(r0 + 2 * p) * D + col], st[(long)(r0 + 2 * p + 1) * D + col]};
+    }
 
     // o products of the last pair, fragments in registers
     constexpr int MT = D / 16 / NW, NK = NC / 32;
@@ -461,11 +491,11 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_fast_kernel(
     };
 
     SegRows<D, NC, NT, false, CKS, true, false, SG> rows;
-    rows.load(k, nullptr, v, cbh, nullptr, base0, tstride, 0, (int)(T < SG ? T : SG), cb * NC,
-              tid);
+    rows.load(k, nullptr, v, cbh, nullptr, base0, tstride, tb, (int)(T - tb < SG ? T - tb : SG),
+              cb * NC, tid);
     long P = 0;  // token pairs so far (selects the Sl buffers)
     for (long seg = 0; seg < nsegf; ++seg) {
-        const long t0 = seg * SG;
+        const long t0 = tb + seg * SG;
         const int n = (int)(T - t0 < SG ? T - t0 : SG);
         __syncthreads();  // the previous segment's rows read (its last o_reads)
         rows.store(sm.seg, n, tid);
@@ -487,6 +517,7 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_fast_kernel(
         }
     }
     if (pp >= 0) o_products();
+    if (gr.n > 1) return;  // the chain pass has written the final state
     // the final state back to the caller
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
@@ -495,87 +526,209 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_fast_kernel(
     }
 }
 
-// The checkpoint pass of the register-resident backward: the forward's state
-// update (as r_fast_kernel, same roundings) with no outputs but the state
-// before every SEGF-th token, stored column-major to ck.  Each lane's column
-// needs only its own rows of k and c k, so a segment runs without barriers
-// from staged rows (two barriers per segment, the next segment's reads in
-// flight meanwhile).
+// The chain pass: the recurrences without outputs (see RGroups; also the
+// checkpoint pass of the backward with one group).  Workgroups 0 .. nfwd - 1 run
+// the forward's state update (as r_fast_kernel, same roundings), storing the
+// state before every `every`-th segment of SEGF tokens column-major to ck, and
+// the final state to state_out if given; the others dL/dS backwards (as
+// r_bwd_fast_kernel, G <- g - k w1^T), storing it after each group but the last
+// to gck.  Each lane's column needs only its own rows of the staged tokens, so
+// a segment runs without barriers (two per segment, the next segment's reads
+// in flight meanwhile), a token's operands read from LDS during the token
+// before.  Bound by the token's dependent instructions (16 rows a lane: about
+// 60 with one wave per SIMD): 0.185 us per token at d = 128 and 0.13 at d = 64,
+// forward and backward chains side by side, against 0.26 for a forward chain
+// of 32 rows a lane whose operands were read in the token itself.
+template <int D, int NS>
+union RChainSmem {
+    SegLds<D, D / NS, false, true, true, false> fwd;
+    struct {
+        float kf[SEGF][D], gf[SEGF][D], cc[SEGF];
+    } bwd;
+};
+
 template <int D, int NS, int LPC>
-__global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_ckpt_kernel(
-    const bf16* __restrict__ k, const bf16* __restrict__ v, const float* __restrict__ coef,
-    const bf16* __restrict__ state, bf16* __restrict__ ck, int H, long T) {
+__global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_chain_kernel(
+    const bf16* __restrict__ k, const bf16* __restrict__ v, const bf16* __restrict__ dO,
+    const float* __restrict__ coef, const bf16* state, bf16* state_out, bf16* __restrict__ ck,
+    int every, float* __restrict__ gck, RGroups gr, int nfwd, int H, long T) {
     constexpr int NC = D / NS, NT = rfast_threads<D, NS, LPC>();
     constexpr int RPL = D / LPC, NP = RPL / 2;
-    static_assert(RPL % 8 == 0 && (D == 64 || D == 128) && NC % 32 == 0 && NT % 64 == 0 &&
-                      NT <= 1024,
-                  "d = 64 or 128, 32-column multiples per workgroup");
-    __shared__ __attribute__((aligned(16))) SegLds<D, NC, false, true, true, false> sm;
+    static_assert(RPL % 8 == 0 && (D == 32 || D == 64 || D == 128) && NC % 8 == 0 &&
+                      NT % 64 == 0 && NT <= 1024,
+                  "d = 32, 64 or 128, whole waves");
+    __shared__ __attribute__((aligned(16))) RChainSmem<D, NS> sm;
     const int tid = threadIdx.x;
-    const int bh = blockIdx.x / NS, cb = blockIdx.x % NS;
+    const bool rev = (int)blockIdx.x >= nfwd;
+    const int id = rev ? (int)blockIdx.x - nfwd : (int)blockIdx.x;
+    const int bh = id / NS, cb = id % NS;
     const int col = cb * NC + tid / LPC, lcol = tid / LPC, part = tid % LPC, r0 = part * RPL;
     const int b = bh / H, h = bh % H;
     const long dd = (long)D * D, nsegf = (T + SEGF - 1) / SEGF;
     const long tstride = (long)H * D;
     const long base0 = (long)b * T * tstride + (long)h * D;
     const float* cbh = coef + (long)bh * T;
+    if (rev) {
+        float G[RPL];
+#pragma unroll
+        for (int i = 0; i < RPL; ++i) G[i] = 0.f;
+        SegRows<D, NC, NT, true, false, false, false> rows;
+        typedef decltype(rows) Rows;
+        const long lo = gr.segs;  // the first group's dL/dS is the token loop's own
+        rows.load(k, dO, nullptr, cbh, nullptr, base0, tstride, (nsegf - 1) * SEGF,
+                  (int)(T - (nsegf - 1) * SEGF), 0, tid);
+        for (long seg = nsegf - 1; seg >= lo; --seg) {
+            const long t0 = seg * SEGF;
+            const int n = (int)(T - t0 < SEGF ? T - t0 : SEGF);
+#pragma unroll
+            for (int it = 0; it < Rows::IK; ++it) {
+                const int i = tid + it * NT, j = i / (D / Rows::VW), e0 = (i % (D / Rows::VW)) * Rows::VW;
+                if (i < Rows::NKP && j < n)
+#pragma unroll
+                    for (int e = 0; e < Rows::VW; ++e) {
+                        sm.bwd.kf[j][e0 + e] = (float)rows.kx[it][e];
+                        sm.bwd.gf[j][e0 + e] = (float)rows.gx[it][e];
+                    }
+            }
+            if (tid < n) sm.bwd.cc[tid] = rows.cs;
+            __syncthreads();
+            if (seg > lo)
+                rows.load(k, dO, nullptr, cbh, nullptr, base0, tstride, t0 - SEGF, SEGF, 0, tid);
+            struct Ops {
+                mf::floatx4 kf[RPL / 4], gf[RPL / 4];
+                float kc, c;
+            } oa, ob;
+            auto read = [&](Ops& x, int j) {
+                j = j < 0 ? 0 : j;
+#pragma unroll
+                for (int q = 0; q < RPL / 4; ++q) {
+                    x.kf[q] = *reinterpret_cast<const mf::floatx4*>(&sm.bwd.kf[j][r0 + 4 * q]);
+                    x.gf[q] = *reinterpret_cast<const mf::floatx4*>(&sm.bwd.gf[j][r0 + 4 * q]);
+                }
+                x.kc = sm.bwd.kf[j][col];
+                x.c = sm.bwd.cc[j];
+            };
+            auto token = [&](const Ops& x) {
+                float sa[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < RPL; ++i) {
+                    G[i] = fmaf(x.gf[i / 4][i % 4], x.kc, G[i]);
+                    sa[i & 3] = fmaf(G[i], x.kf[i / 4][i % 4], sa[i & 3]);
+                }
+                const float w1 = x.c * quad_sum<LPC>((sa[0] + sa[1]) + (sa[2] + sa[3]));
+#pragma unroll
+                for (int i = 0; i < RPL; ++i) G[i] = fmaf(-x.kf[i / 4][i % 4], w1, G[i]);
+            };
+            // pairs without a branch between them: a conditional second token
+            // has its reads moved next to their use
+            read(oa, n - 1);
+            for (int j = n - 1; j > 0; j -= 2) {
+                read(ob, j - 1);
+                __builtin_amdgcn_sched_barrier(0);
+                token(oa);
+                read(oa, j - 2);
+                __builtin_amdgcn_sched_barrier(0);
+                token(ob);
+            }
+            if (n & 1) token(oa);
+            if (seg % gr.segs == 0) {  // dL/dS after the group before
+                float* dst = gck + ((long)bh * gr.n + seg / gr.segs - 1) * dd + (long)col * D + r0;
+#pragma unroll
+                for (int i = 0; i < RPL / 4; ++i)
+                    *reinterpret_cast<mf::floatx4*>(dst + 4 * i) =
+                        mf::floatx4{G[4 * i], G[4 * i + 1], G[4 * i + 2], G[4 * i + 3]};
+            }
+            __syncthreads();  // the segment's rows read
+        }
+        return;
+    }
     const bf16* st = state + (long)bh * dd;
-
     bf16x2 S[NP];  // rows r0 + 2p (low half) and r0 + 2p + 1 (high half)
 #pragma unroll
     for (int p = 0; p < NP; ++p)
         S[p] = bf16x2{st[(long)(r0 + 2 * p) * D + col], st[(long)(r0 + 2 * p + 1) * D + col]};
+    const long nck = (nsegf + every - 1) / every;
     SegRows<D, NC, NT, false, true, true, false> rows;
     rows.load(k, nullptr, v, cbh, nullptr, base0, tstride, 0, (int)(T < SEGF ? T : SEGF), cb * NC,
               tid);
     for (long seg = 0; seg < nsegf; ++seg) {
         const long t0 = seg * SEGF;
         const int n = (int)(T - t0 < SEGF ? T - t0 : SEGF);
-        rows.store(sm, n, tid);
+        rows.store(sm.fwd, n, tid);
         __syncthreads();
         if (seg + 1 < nsegf) {
             const long t2 = t0 + SEGF;
             rows.load(k, nullptr, v, cbh, nullptr, base0, tstride, t2,
                       (int)(T - t2 < SEGF ? T - t2 : SEGF), cb * NC, tid);
         }
-        // the state before token t0, column-major [c][row]
-        bf16* dst = ck + ((long)bh * nsegf + seg) * dd + (long)col * D + r0;
-#pragma unroll
-        for (int q = 0; q < NP / 4; ++q)
-            *reinterpret_cast<bf16x8*>(dst + 8 * q) =
-                bf16x8{S[4 * q][0], S[4 * q][1], S[4 * q + 1][0], S[4 * q + 1][1],
-                       S[4 * q + 2][0], S[4 * q + 2][1], S[4 * q + 3][0], S[4 * q + 3][1]};
-        for (int j = 0; j < n; ++j) {
-            bf16x8 kq[NP / 4];
-            mf::floatx4 cq[RPL / 4];
+        if (seg % every == 0) {  // the state before token t0, column-major [c][row]
+            bf16* dst = ck + ((long)bh * nck + seg / every) * dd + (long)col * D + r0;
 #pragma unroll
             for (int q = 0; q < NP / 4; ++q)
-                kq[q] = *reinterpret_cast<const bf16x8*>(&sm.kb[j][r0 + 8 * q]);
+                *reinterpret_cast<bf16x8*>(dst + 8 * q) =
+                    bf16x8{S[4 * q][0], S[4 * q][1], S[4 * q + 1][0], S[4 * q + 1][1],
+                           S[4 * q + 2][0], S[4 * q + 2][1], S[4 * q + 3][0], S[4 * q + 3][1]};
+        }
+        struct Ops {
+            mf::int4v kq[NP / 4];
+            mf::floatx4 cq[RPL / 4];
+            bf16 vt;
+        } oa, ob;
+        auto read = [&](Ops& x, int j) {
+            j = j < n ? j : n - 1;
+#pragma unroll
+            for (int q = 0; q < NP / 4; ++q)
+                x.kq[q] = *reinterpret_cast<const mf::int4v*>(&sm.fwd.kb[j][r0 + 8 * q]);
 #pragma unroll
             for (int q = 0; q < RPL / 4; ++q)
-                cq[q] = *reinterpret_cast<const mf::floatx4*>(&sm.ckf[j][r0 + 4 * q]);
-            const float vt = to_f(sm.vb[j][lcol]);
+                x.cq[q] = *reinterpret_cast<const mf::floatx4*>(&sm.fwd.ckf[j][r0 + 4 * q]);
+            x.vt = sm.fwd.vb[j][lcol];
+        };
+        auto token = [&](const Ops& x) {
             float ua[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int p = 0; p < NP; ++p) {
-                const bf16x2 kp = bf16x2{kq[p / 4][2 * (p % 4)], kq[p / 4][2 * (p % 4) + 1]};
-                ua[p % 4] = __builtin_amdgcn_fdot2_f32_bf16(kp, S[p], ua[p % 4], false);
-            }
+            for (int p = 0; p < NP; ++p)
+                ua[p % 4] = __builtin_amdgcn_fdot2_f32_bf16(
+                    __builtin_bit_cast(bf16x2, (int)x.kq[p / 4][p % 4]), S[p], ua[p % 4], false);
             const float u = quad_sum<LPC>((ua[0] + ua[1]) + (ua[2] + ua[3]));
-            const float rc = vt - u;
+            const float rc = to_f(x.vt) - u;
 #pragma unroll
             for (int p = 0; p < NP; ++p) {
-                const float lo = fmaf(cq[p / 2][2 * (p % 2)], rc, (float)S[p][0]);
-                const float hi = fmaf(cq[p / 2][2 * (p % 2) + 1], rc, (float)S[p][1]);
+                // the pair as one opaque word: seen through, its halves become
+                // two more conversions that the next token unpacks
+                unsigned sp = __builtin_bit_cast(unsigned, S[p]);
+                asm("" : "+v"(sp));
+                const float lo = fmaf(x.cq[p / 2][2 * (p % 2)], rc,
+                                      __builtin_bit_cast(float, sp << 16));
+                const float hi = fmaf(x.cq[p / 2][2 * (p % 2) + 1], rc,
+                                      __builtin_bit_cast(float, sp & 0xffff0000u));
                 S[p] = bf16x2{(bf16)lo, (bf16)hi};
             }
+        };
+        read(oa, 0);
+        for (int j = 0; j + 1 < n; j += 2) {
+            read(ob, j + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            token(oa);
+            read(oa, j + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            token(ob);
         }
+        if (n & 1) token(oa);
         __syncthreads();  // the segment's rows read
+    }
+    if (state_out) {
+        bf16* so = state_out + (long)bh * dd;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            so[(long)(r0 + 2 * p) * D + col] = S[p][0];
+            so[(long)(r0 + 2 * p + 1) * D + col] = S[p][1];
+        }
     }
 }
 
 // ---------------------------------------------------------------------------
-// backward, register-resident (d = 64 or 128)
+// backward, register-resident (d = 32, 64 or 128)
 // ---------------------------------------------------------------------------
 // The reference BPTT (efla.cu:355-453) per token, last to first, with
 // G = dL/dS (after the token) in fp32 registers in the forward's column-owner
@@ -613,26 +766,30 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_bwd_fast_kern
     const bf16* __restrict__ dO, const bf16* __restrict__ k, const bf16* __restrict__ v,
     const float* __restrict__ coef, const float* __restrict__ dcoef, const bf16* __restrict__ ck,
     bf16* __restrict__ hist_all, bf16* __restrict__ grad_k, float* __restrict__ part_gk,
-    bf16* __restrict__ grad_v, bf16* __restrict__ grad_state, int H, long T) {
+    bf16* __restrict__ grad_v, bf16* __restrict__ grad_state, int H, long T, RGroups gr) {
     constexpr int NC = D / NS, NT = rfast_threads<D, NS, LPC>(), NW = NT / 64;
     constexpr int RPL = D / LPC, NP = RPL / 2, LDS = D + 8;
     constexpr int MT = D / 16 / NW, NK = NC / 32;
     constexpr bool CKS = RBwdSmem<D, NS>::CKS;
-    static_assert(RPL % 8 == 0 && (D == 64 || D == 128) && NC % 32 == 0 && NT % 64 == 0 &&
-                      NT <= 1024 && D % (16 * NW) == 0 && LPC % 4 == 0 && NW <= 16,
-                  "d = 64 or 128, 32-column multiples per workgroup, 4 or 8 lanes per column");
+    static_assert(RPL % 8 == 0 && (D == 32 || D == 64 || D == 128) && NC % 32 == 0 &&
+                      NT % 64 == 0 && NT <= 1024 && D % (16 * NW) == 0 && LPC % 4 == 0 &&
+                      NW <= 16,
+                  "d = 32, 64 or 128, 32-column multiples per workgroup, 4 or 8 lanes per column");
     __shared__ __attribute__((aligned(16))) RBwdSmem<D, NS> sm;
     const int tid = threadIdx.x, w = mf::wave(), l = mf::lane();
-    const int bh = blockIdx.x / NS, cb = blockIdx.x % NS;
+    const int item = blockIdx.x / NS, cb = blockIdx.x % NS;
+    const int grp = item / gr.nbh, bh = item - grp * gr.nbh;
     const int col = cb * NC + tid / LPC, lcol = tid / LPC, part = tid % LPC, r0 = part * RPL;
     const int g4 = l >> 4, j16 = l & 15;
     const int b = bh / H, h = bh % H;
     const long dd = (long)D * D, nsegf = (T + SEGF - 1) / SEGF;
+    // this workgroup's segments: s_lo .. s_hi - 1
+    const long s_lo = (long)grp * gr.segs, s_hi = s_lo + gr.segs < nsegf ? s_lo + gr.segs : nsegf;
     const long tstride = (long)H * D;
     const long base0 = (long)b * T * tstride + (long)h * D;
     const float* cbh = coef + (long)bh * T;
     const float* dcbh = dcoef + (long)bh * T;
-    bf16* hist = hist_all + (long)bh * (SEGF + 1) * dd;
+    bf16* hist = hist_all + (long)item * (SEGF + 1) * dd;
     auto col_ptr = [&](bf16* basep, long jj) { return basep + jj * dd + (long)col * D + r0; };
     auto load_col = [&](const bf16* src, bf16x2 (&dst)[NP]) {
 #pragma unroll
@@ -654,15 +811,21 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_bwd_fast_kern
     float G[RPL];
 #pragma unroll
     for (int i = 0; i < RPL; ++i) G[i] = 0.f;
+    if (s_hi < nsegf) {  // dL/dS after the group, from the chain pass
+        const float* gp = gr.gck + ((long)bh * gr.n + grp) * dd + (long)col * D + r0;
+#pragma unroll
+        for (int i = 0; i < RPL; ++i) G[i] = gp[i];
+    }
     const bf16x8 ones = bf16x8{(bf16)1.f, (bf16)1.f, (bf16)1.f, (bf16)1.f,
                                (bf16)1.f, (bf16)1.f, (bf16)1.f, (bf16)1.f};
 
     SegRows<D, NC, NT, true, CKS, CKS, true> rows;
     {
-        const long t0 = (nsegf - 1) * SEGF;
-        rows.load(k, dO, v, cbh, dcbh, base0, tstride, t0, (int)(T - t0), cb * NC, tid);
+        const long t0 = (s_hi - 1) * SEGF;
+        rows.load(k, dO, v, cbh, dcbh, base0, tstride, t0, (int)(T - t0 < SEGF ? T - t0 : SEGF),
+                  cb * NC, tid);
     }
-    for (long seg = nsegf - 1; seg >= 0; --seg) {
+    for (long seg = s_hi - 1; seg >= s_lo; --seg) {
         const long t0 = seg * SEGF, t1 = t0 + SEGF < T ? t0 + SEGF : T;
         const int n = (int)(t1 - t0);
         // ---- the segment's rows into LDS (the previous segment's last
@@ -734,7 +897,7 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_bwd_fast_kern
             load_col(col_ptr(hist, n), Sn);
             load_lane(n - 1, 0);
             // the next segment's rows: reads in flight during this reverse pass
-            if (seg > 0)
+            if (seg > s_lo)
                 rows.load(k, dO, v, cbh, dcbh, base0, tstride, t0 - SEGF, SEGF, cb * NC, tid);
             // token t0 + j: its (v and) state in vR[s], SpR[s]
             auto rtoken = [&](int j, int s) {
@@ -864,6 +1027,7 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_bwd_fast_kern
             }
         }
     }
+    if (s_lo > 0) return;
     // dL/dS_0 in the reference's [row][c] layout
     bf16* gs = grad_state + (long)bh * dd;
 #pragma unroll
@@ -891,57 +1055,120 @@ __global__ void __launch_bounds__(NTH) r_combine_kernel(const float* __restrict_
 // when B H would leave at least half of the CUs without one.
 // (Four workgroups of 32 columns, two per CU, measured slower at B H = 128:
 // forward 5.5 against 5.2 ms, backward 26.5 against 24.7 ms.)
-inline int r_split(size_t nbh) {
+inline int r_split(int d, size_t nbh) {
     const int ncu = device_cu_count();
-    return ncu > 0 && nbh * 2 <= (size_t)ncu ? 2 : 1;
+    return d > 32 && ncu > 0 && nbh * 2 <= (size_t)ncu ? 2 : 1;
 }
 
 template <int D, int NS, int LPC>
-void r_launch_fwd(bool checkpoints, int sg, const void* k, const void* v, const float* coef,
-                  void* state, void* out, float* part, long pstride, bf16* ck, int H, long T,
-                  size_t nbh, hipStream_t stream) {
-    const dim3 grid((unsigned)(nbh * NS)), block(rfast_threads<D, NS, LPC>());
-    if (checkpoints)
-        EFLA_LAUNCH("efla_r_checkpoint", (r_ckpt_kernel<D, NS, LPC>), grid, block, stream,
-                    (const bf16*)k, (const bf16*)v, coef, (const bf16*)state, ck, H, T);
-    else if (sg == 16)
+void r_launch_fwd(int sg, const void* k, const void* v, const float* coef, void* state, void* out,
+                  float* part, int H, long T, const RGroups& gr, hipStream_t stream) {
+    const dim3 grid((unsigned)((size_t)gr.nbh * gr.n * NS)), block(rfast_threads<D, NS, LPC>());
+    if (sg == 16)
         EFLA_LAUNCH("efla_r_forward", (r_fast_kernel<D, NS, LPC, 16>), grid, block, stream,
                     (const bf16*)k, (const bf16*)v, coef, (bf16*)state, (bf16*)out, part,
-                    H, T);
-    else if (sg == 64 && (NS > 1 || D == 64))  // the LDS of the other shapes holds 32 at most
-        EFLA_LAUNCH("efla_r_forward", (r_fast_kernel<D, NS, LPC, (NS > 1 || D == 64) ? 64 : 32>),
+                    H, T, gr);
+    else if (sg == 64 && (NS > 1 || D <= 64))  // the LDS of the other shapes holds 32 at most
+        EFLA_LAUNCH("efla_r_forward", (r_fast_kernel<D, NS, LPC, (NS > 1 || D <= 64) ? 64 : 32>),
                     grid, block, stream, (const bf16*)k, (const bf16*)v, coef, (bf16*)state,
-                    (bf16*)out, part, H, T);
+                    (bf16*)out, part, H, T, gr);
     else
         EFLA_LAUNCH("efla_r_forward", (r_fast_kernel<D, NS, LPC, 32>), grid, block, stream,
                     (const bf16*)k, (const bf16*)v, coef, (bf16*)state, (bf16*)out, part,
-                    H, T);
+                    H, T, gr);
 }
 
 template <int D, int NS, int LPC>
 void r_launch_bwd(const void* dO, const void* k, const void* v, const float* coef,
                   const float* dcoef, const bf16* ck, bf16* hist, void* grad_k, float* part,
-                  long pstride, void* grad_v, void* grad_state, int H, long T, size_t nbh,
+                  void* grad_v, void* grad_state, int H, long T, const RGroups& gr,
                   hipStream_t stream) {
-    EFLA_LAUNCH("efla_r_backward", (r_bwd_fast_kernel<D, NS, LPC>), dim3((unsigned)(nbh * NS)),
-                dim3(rfast_threads<D, NS, LPC>()), stream, (const bf16*)dO, (const bf16*)k,
-                (const bf16*)v, coef, dcoef, ck, hist, (bf16*)grad_k, part,
-                (bf16*)grad_v, (bf16*)grad_state, H, T);
+    EFLA_LAUNCH("efla_r_backward", (r_bwd_fast_kernel<D, NS, LPC>),
+                dim3((unsigned)((size_t)gr.nbh * gr.n * NS)), dim3(rfast_threads<D, NS, LPC>()),
+                stream, (const bf16*)dO, (const bf16*)k, (const bf16*)v, coef, dcoef, ck, hist,
+                (bf16*)grad_k, part, (bf16*)grad_v, (bf16*)grad_state, H, T, gr);
 }
 
-// the register-resident forward (checkpoints = false) or checkpoint pass for
-// head_dim d and split ns
-inline void r_fwd_fast(int d, int ns, bool checkpoints, int sg, const void* k, const void* v,
-                       const float* coef, void* state, void* out, float* part, long pstride,
-                       bf16* ck, int H, long T, size_t nbh, hipStream_t stream) {
-    if (d == 128 && ns == 1)
-        r_launch_fwd<128, 1, 4>(checkpoints, sg, k, v, coef, state, out, part, pstride, ck, H, T, nbh, stream);
-    else if (d == 128)
-        r_launch_fwd<128, 2, 8>(checkpoints, sg, k, v, coef, state, out, part, pstride, ck, H, T, nbh, stream);
-    else if (ns == 1)
-        r_launch_fwd<64, 1, 4>(checkpoints, sg, k, v, coef, state, out, part, pstride, ck, H, T, nbh, stream);
+// the chain pass: forward states to ck every `every` segments, and with gck
+// dL/dS after the groups
+template <int D, int NS, int LPC>
+void r_launch_chain(const void* k, const void* v, const void* dO, const float* coef,
+                    const void* state, void* state_out, bf16* ck, int every, float* gck, int H,
+                    long T, const RGroups& gr, hipStream_t stream) {
+    const int nfwd = gr.nbh * NS;
+    EFLA_LAUNCH("efla_r_chain", (r_chain_kernel<D, NS, LPC>),
+                dim3((unsigned)((size_t)nfwd * (gck ? 2 : 1))), dim3(rfast_threads<D, NS, LPC>()),
+                stream, (const bf16*)k, (const bf16*)v, (const bf16*)dO, coef, (const bf16*)state,
+                (bf16*)state_out, ck, every, gck, gr, nfwd, H, T);
+}
+
+// head_dim and split of the token loops -> their template arguments
+#define R_DISPATCH(FN, ...)                                        \
+    do {                                                           \
+        if (d == 128 && ns == 1) FN<128, 1, 4>(__VA_ARGS__);       \
+        else if (d == 128) FN<128, 2, 8>(__VA_ARGS__);             \
+        else if (d == 64 && ns == 1) FN<64, 1, 4>(__VA_ARGS__);    \
+        else if (d == 64) FN<64, 2, 8>(__VA_ARGS__);               \
+        else FN<32, 1, 4>(__VA_ARGS__);                            \
+    } while (0)
+
+// The chain pass keeps the token loops' lanes per column (the sums' order);
+// its columns spread over twice their workgroups while that leaves no CU with
+// two (D / NS columns of LPC lanes then put one wave on each SIMD).
+inline void r_chain(int d, int ns, const void* k, const void* v, const void* dO,
+                    const float* coef, const void* state, void* state_out, bf16* ck, int every,
+                    float* gck, int H, long T, const RGroups& gr, hipStream_t st) {
+    const int ncu = device_cu_count() > 0 ? device_cu_count() : 256;
+    if (ns > 1 && (long)gr.nbh * 4 * (gck ? 2 : 1) <= ncu) {
+        if (d == 128)
+            r_launch_chain<128, 4, 8>(k, v, dO, coef, state, state_out, ck, every, gck, H, T, gr, st);
+        else
+            r_launch_chain<64, 4, 8>(k, v, dO, coef, state, state_out, ck, every, gck, H, T, gr, st);
+        return;
+    }
+    R_DISPATCH(r_launch_chain, k, v, dO, coef, state, state_out, ck, every, gck, H, T, gr, st);
+}
+
+// Groups for the token loops: as many as the chip holds workgroups at once
+// (per CU one of the d = 128 kernels, two of d = 64, four of d = 32, by their
+// LDS), where the chain pass costs less than the groups save.  Measured (one
+// group / this, us; sequences x tokens x heads, d):
+//                              forward       backward
+//   2 x 2048 x 16, d = 128   1214 / 721    3937 / 1475
+//   4 x 1000 x 16, d = 128    600 / 511    2030 / 1258
+//   1 x  128 x 32, d = 128     89 / 59      265 / 110
+//   2 x 2048 x 16, d = 64     562 / 359    1941 / 568
+//   4 x 2048 x 32, d = 64     613 / 598    2137 / 1489   (forward: one group)
+//   1 x   40 x  1, d = 128     38 / 38       90 / 75     (forward: one group)
+// d = 32 against the LDS-resident kernels: 2 x 1000 x 8 1611 / 135 and
+// 7437 / 164; 4 x 2048 x 32 3797 / 367 and 17033 / 615.
+inline RGroups r_groups(int d, int ns, size_t nbh, size_t T, bool backward) {
+    RGroups gr{(int)nbh, 1, (int)((T + SEGF - 1) / SEGF), nullptr, nullptr};
+    const long ncu = device_cu_count() > 0 ? device_cu_count() : 256;
+    const long nseg = gr.segs, room = ncu * (d == 128 ? 1 : d == 64 ? 2 : 4) / ((long)nbh * ns);
+    if (room < 2 || nseg < 2 || (ns == 1 && d > 32)) return gr;
+    const long want = room < nseg ? room : nseg, segs = (nseg + want - 1) / want;
+    // us per token of the chain pass and of the forward's token loop; the
+    // backward has its checkpoint pass anyway
+    const double chain = d == 128 ? 0.20 : 0.14, loop = d == 128 ? 0.57 : 0.28;
+    if (!backward && T * chain + (double)(segs * SEGF) * loop + 10. > 0.95 * T * loop) return gr;
+    gr.segs = (int)segs;
+    gr.n = (int)((nseg + segs - 1) / segs);
+    return gr;
+}
+
+inline void r_coeff(int d, const void* k, float* c, float* dc, int H, long T, float beta,
+                    size_t ntok, hipStream_t stream) {
+    const dim3 cg((unsigned)((ntok * 16 + NTH - 1) / NTH));
+    if (d == 128)
+        EFLA_LAUNCH("efla_r_coeff", r_coeff_kernel<8>, cg, dim3(NTH), stream, (const bf16*)k, c,
+                    dc, H, T, beta, (long)ntok);
+    else if (d == 64)
+        EFLA_LAUNCH("efla_r_coeff", r_coeff_kernel<4>, cg, dim3(NTH), stream, (const bf16*)k, c,
+                    dc, H, T, beta, (long)ntok);
     else
-        r_launch_fwd<64, 2, 8>(checkpoints, sg, k, v, coef, state, out, part, pstride, ck, H, T, nbh, stream);
+        EFLA_LAUNCH("efla_r_coeff", r_coeff_kernel<2>, cg, dim3(NTH), stream, (const bf16*)k, c,
+                    dc, H, T, beta, (long)ntok);
 }
 
 // chunk_size as the forward's segment length: 16, 32 or 64 tokens staged in
@@ -1159,41 +1386,53 @@ extern "C" int efla_forward_hip(const void* k, const void* v, void* state, void*
     // its shared-memory limit; see the header)
     if (head_dim > (size_t)MAXD || nbh > (size_t)INT32_MAX) return kInvalidConfiguration;
     const dim3 grid((unsigned)nbh);
-    // the register-resident path: d = 64 / 128, k and v aligned for d / 8-byte
-    // row loads (the coefficient kernel's, the segment staging's) and output
-    // for 8-byte row pieces, at most 2^35 tokens
-    const bool fast = (head_dim == 128 || head_dim == 64) &&
+    // the register-resident path: d = 32 / 64 / 128, k and v aligned for d /
+    // 8-byte row loads (the coefficient kernel's, the segment staging's) and
+    // output for 8-byte row pieces, at most 2^35 tokens
+    const bool fast = (head_dim == 128 || head_dim == 64 || head_dim == 32) &&
                       (uintptr_t)k % (head_dim / 8) == 0 && (uintptr_t)v % (head_dim / 8) == 0 &&
                       (uintptr_t)output % 8 == 0 && nbh * seq_len <= ((size_t)1 << 35);
     if (fast) {
         // every token's coefficient first (the stream's workspace), then the
         // register-resident token loop; with the column split the fp32 row
         // sums (one zeroed buffer both halves add into) follow the
-        // coefficients in the workspace
+        // coefficients in the workspace, then the groups' start states
+        const int d = (int)head_dim, H = (int)num_heads;
+        const long T = (long)seq_len;
         const size_t ntok = nbh * seq_len;
-        const int ns = r_split(nbh);
+        const int ns = r_split(d, nbh);
         const size_t off_p = (ntok * sizeof(float) + 255) & ~(size_t)255;
-        const size_t need = ns > 1 ? off_p + elems * sizeof(float) : ntok * sizeof(float);
+        const size_t off_ck =
+            ns > 1 ? (off_p + elems * sizeof(float) + 255) & ~(size_t)255 : off_p;
+        RGroups gr = r_groups(d, ns, nbh, seq_len, false);
+        size_t need = off_ck;
+        if (gr.n > 1) {
+            need += nbh * gr.n * head_dim * head_dim * sizeof(bf16);
+            if (!workspace_available(need, stream)) {  // one group needs less
+                gr.n = 1;
+                gr.segs = (int)((seq_len + SEGF - 1) / SEGF);
+                need = off_ck;
+            }
+        }
         void* ws = nullptr;
         WsLease lease;
         int rc = workspace_acquire(need, stream, &ws, lease);
         if (rc != kSuccess) return rc;
+        float* coef = (float*)ws;
         float* part = ns > 1 ? (float*)((char*)ws + off_p) : nullptr;
         if (part) {
             rc = fill_zero(part, elems * sizeof(float), stream);
             if (rc != kSuccess) return rc;
         }
-        const dim3 cg((unsigned)((ntok * 16 + NTH - 1) / NTH));
-        if (head_dim == 128)
-            EFLA_LAUNCH("efla_r_coeff", r_coeff_kernel<8>, cg, dim3(NTH), stream, (const bf16*)k,
-                        (float*)ws, (float*)nullptr, (int)num_heads, (long)seq_len, beta,
-                        (long)ntok);
-        else
-            EFLA_LAUNCH("efla_r_coeff", r_coeff_kernel<4>, cg, dim3(NTH), stream, (const bf16*)k,
-                        (float*)ws, (float*)nullptr, (int)num_heads, (long)seq_len, beta,
-                        (long)ntok);
-        r_fwd_fast((int)head_dim, ns, false, r_segment(chunk_size), k, v, (const float*)ws, state,
-                   output, part, (long)elems, nullptr, (int)num_heads, (long)seq_len, nbh, stream);
+        r_coeff(d, k, coef, nullptr, H, T, beta, ntok, stream);
+        if (gr.n > 1) {
+            bf16* ck = (bf16*)((char*)ws + off_ck);
+            gr.ck = ck;
+            r_chain(d, ns, k, v, nullptr, coef, state, state, ck, gr.segs, nullptr, H, T, gr,
+                    stream);
+        }
+        const int sg = r_segment(chunk_size);
+        R_DISPATCH(r_launch_fwd, sg, k, v, coef, state, output, part, H, T, gr, stream);
         if (ns > 1) r_combine(part, (long)elems, 1, output, elems, stream);
     } else {
         EFLA_LAUNCH("efla_r_forward", r_forward_kernel, grid, dim3(NTH), stream, (const bf16*)k,
@@ -1217,66 +1456,60 @@ extern "C" int efla_backward_hip(const void* grad_output, const void* k, const v
     if (seq_len == 0) return fill_zero(grad_state, gsb, stream);
     if (!grad_output || !k || !v || !grad_k || !grad_v) return kInvalidValue;
     if (head_dim > (size_t)MAXD || nbh > (size_t)INT32_MAX) return kInvalidConfiguration;
-    // the register-resident path: d = 64 / 128, k, dO and v aligned for d / 8-byte
-    // row loads (the coefficient kernel's, the segment staging's) and grad_k
-    // for 8-byte row pieces, at most 2^35 tokens
+    // the register-resident path: d = 32 / 64 / 128, k, dO and v aligned for d /
+    // 8-byte row loads (the coefficient kernel's, the segment staging's) and
+    // grad_k for 8-byte row pieces, at most 2^35 tokens
     const size_t ra = head_dim / 8;
-    const bool fast = (head_dim == 128 || head_dim == 64) && (uintptr_t)k % ra == 0 &&
-                      (uintptr_t)grad_output % ra == 0 && (uintptr_t)v % ra == 0 &&
-                      (uintptr_t)grad_k % 8 == 0 && nbh * seq_len <= ((size_t)1 << 35);
+    const bool fast = (head_dim == 128 || head_dim == 64 || head_dim == 32) &&
+                      (uintptr_t)k % ra == 0 && (uintptr_t)grad_output % ra == 0 &&
+                      (uintptr_t)v % ra == 0 && (uintptr_t)grad_k % 8 == 0 &&
+                      nbh * seq_len <= ((size_t)1 << 35);
     if (fast) {
-        // workspace: checkpoints every SEGF tokens | one segment's states |
-        // c and dc/dlambda per token (all column-major states, bf16)
+        // workspace: checkpoints every SEGF tokens | c and dc/dlambda per token |
+        // with the column split grad_k's fp32 sums (one zeroed buffer) | per
+        // group one segment's states and dL/dS after it (column-major states)
+        const int d = (int)head_dim, H = (int)num_heads;
+        const long T = (long)seq_len;
         const size_t nsegf = (seq_len + SEGF - 1) / SEGF, ntok = nbh * seq_len;
-        size_t ck_elems, hist_elems;
-        if (!mul_ok(gse, nsegf, &ck_elems) || !mul_ok(gse, SEGF + 1, &hist_elems))
+        const int ns = r_split(d, nbh);
+        auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
+        size_t ck_elems, hist_elems, elems = 0;
+        if (!mul_ok(gse, nsegf, &ck_elems) || !mul_ok(gse, SEGF + 1, &hist_elems) ||
+            !mul_ok(ntok, head_dim, &elems))
             return kInvalidConfiguration;
-        const size_t off_hist = (ck_elems * 2 + 255) & ~(size_t)255;
-        const size_t off_c = (off_hist + hist_elems * 2 + 255) & ~(size_t)255;
-        const size_t off_dc = (off_c + ntok * 4 + 255) & ~(size_t)255;
-        // with the column split: grad_k's fp32 sums (one zeroed buffer)
-        const int ns = r_split(nbh);
-        size_t elems = 0;
-        if (!mul_ok(ntok, head_dim, &elems)) return kInvalidConfiguration;
-        const size_t off_p = (off_dc + ntok * 4 + 255) & ~(size_t)255;
-        const size_t need = ns > 1 ? off_p + elems * 4 : off_dc + ntok * 4 + 256;
+        const size_t off_c = up(ck_elems * 2);
+        const size_t off_dc = up(off_c + ntok * 4);
+        const size_t off_p = up(off_dc + ntok * 4);
+        const size_t off_hist = ns > 1 ? up(off_p + elems * 4) : off_p;
+        RGroups gr = r_groups(d, ns, nbh, seq_len, true);
+        auto size = [&] {
+            return up(off_hist + hist_elems * 2 * gr.n) + (gr.n > 1 ? gse * 4 * gr.n : 0);
+        };
+        if (gr.n > 1 && !workspace_available(size(), stream)) {  // one group needs less
+            gr.n = 1;
+            gr.segs = (int)nsegf;
+        }
         void* ws = nullptr;
         WsLease lease;
-        int rc = workspace_acquire(need, stream, &ws, lease);
+        int rc = workspace_acquire(size(), stream, &ws, lease);
         if (rc != kSuccess) return rc;
         bf16* ck = (bf16*)ws;
-        bf16* hist = (bf16*)((char*)ws + off_hist);
         float* coef = (float*)((char*)ws + off_c);
         float* dcoef = (float*)((char*)ws + off_dc);
         float* part = ns > 1 ? (float*)((char*)ws + off_p) : nullptr;
+        bf16* hist = (bf16*)((char*)ws + off_hist);
+        float* gck = gr.n > 1 ? (float*)((char*)ws + up(off_hist + hist_elems * 2 * gr.n)) : nullptr;
+        gr.ck = ck;
+        gr.gck = gck;
         if (part) {
             rc = fill_zero(part, elems * 4, stream);
             if (rc != kSuccess) return rc;
         }
-        const dim3 cg((unsigned)((ntok * 16 + NTH - 1) / NTH));
-        if (head_dim == 128)
-            EFLA_LAUNCH("efla_r_coeff", r_coeff_kernel<8>, cg, dim3(NTH), stream, (const bf16*)k,
-                        coef, dcoef, (int)num_heads, (long)seq_len, beta, (long)ntok);
-        else
-            EFLA_LAUNCH("efla_r_coeff", r_coeff_kernel<4>, cg, dim3(NTH), stream, (const bf16*)k,
-                        coef, dcoef, (int)num_heads, (long)seq_len, beta, (long)ntok);
-        r_fwd_fast((int)head_dim, ns, true, SEGF, k, v, coef, (void*)state, nullptr, nullptr, 0, ck,
-                   (int)num_heads, (long)seq_len, nbh, stream);
-        const int H = (int)num_heads;
-        const long T = (long)seq_len, ps = (long)elems;
-        if (head_dim == 128 && ns == 1)
-            r_launch_bwd<128, 1, 4>(grad_output, k, v, coef, dcoef, ck, hist, grad_k, part, ps,
-                                    grad_v, grad_state, H, T, nbh, stream);
-        else if (head_dim == 128)
-            r_launch_bwd<128, 2, 8>(grad_output, k, v, coef, dcoef, ck, hist, grad_k, part, ps,
-                                    grad_v, grad_state, H, T, nbh, stream);
-        else if (ns == 1)
-            r_launch_bwd<64, 1, 4>(grad_output, k, v, coef, dcoef, ck, hist, grad_k, part, ps,
-                                   grad_v, grad_state, H, T, nbh, stream);
-        else
-            r_launch_bwd<64, 2, 8>(grad_output, k, v, coef, dcoef, ck, hist, grad_k, part, ps,
-                                   grad_v, grad_state, H, T, nbh, stream);
-        if (ns > 1) r_combine(part, ps, 1, grad_k, elems, stream);
+        r_coeff(d, k, coef, dcoef, H, T, beta, ntok, stream);
+        r_chain(d, ns, k, v, grad_output, coef, state, nullptr, ck, 1, gck, H, T, gr, stream);
+        R_DISPATCH(r_launch_bwd, grad_output, k, v, coef, dcoef, ck, hist, grad_k, part, grad_v,
+                   grad_state, H, T, gr, stream);
+        if (ns > 1) r_combine(part, (long)elems, 1, grad_k, elems, stream);
         return (int)hipPeekAtLastError();
     }
     const size_t nseg = (seq_len + SEG - 1) / SEG;

@@ -48,7 +48,7 @@ extern "C" {
  *   S <- bf16(S + c k_t (v_t - S^T k_t)^T), o_t = S k_t   (requires d_k == d_v)
  * k, v, output: (B, T, H, d) bf16.  state: (B*H, d, d) bf16, read as S_0 and
  * overwritten with S_T.  chunk_size (ignored by the reference) is a tuning
- * hint: for d = 64 / 128 the number of tokens staged in LDS at once (16, 32 or
+ * hint: for d = 32 / 64 / 128 the number of tokens staged in LDS at once (16, 32 or
  * 64: the largest not above it, at least 16; 0 -> 32); the results do not
  * depend on it.  Validation order: B, H or d == 0 -> 1; T == 0 -> 0; any null
  * pointer -> 1; B*H or sizes overflowing -> 9.
@@ -57,7 +57,8 @@ extern "C" {
  * half the device's CU count (two workgroups per (b, h), each owning half of
  * the state's columns) 4 bytes per output element more: one fp32 buffer of
  * row sums both workgroups add into (cfg3's B=4, T=8192, H=32, d=128:
- * 0.54 GB).  `efla_rt_workspace_release_stream` frees a stream's share.
+ * 0.54 GB); with few (b, h), up to 1024 bf16 d*d start states of token groups.
+ * `efla_rt_workspace_release_stream` frees a stream's share.
  */
 int efla_forward_hip(const void* k, const void* v, void* state, void* output,
                      size_t batch_size, size_t seq_len, size_t num_heads, size_t head_dim,
@@ -72,7 +73,8 @@ int efla_forward_hip(const void* k, const void* v, void* state, void* output,
  * one bf16 d*d checkpoint per 32 tokens (64 on the LDS-resident path) and one
  * segment's states per (b, h), 8 bytes per (b, t, h) of coefficients, and with
  * the column split (as efla_forward_hip) 4 bytes per grad_k element for the
- * fp32 row sums.
+ * fp32 row sums; with few (b, h) (as efla_forward_hip) one segment's states and
+ * an fp32 d*d gradient per token group, at most 160 MB.
  */
 int efla_backward_hip(const void* grad_output, const void* k, const void* v, const void* state,
                       void* grad_k, void* grad_v, void* grad_state, size_t batch_size,

@@ -308,3 +308,37 @@ def test_reference_abi_nan_stays_in_its_head(oracle):
                     assert torch.equal(sa, sb), (name, bb, hh)
         assert not torch.isfinite(dirty[0][1, 11:, 1].float()).any()
         assert not torch.isfinite(dirty[1][1, 1].float()).all()
+
+
+# d = 32 on the register-resident kernels, and group edges of the chain pass:
+# one token past a segment, ragged last groups, more groups than segments.
+@pytest.mark.parametrize("B,T,H,d", [(2, 97, 3, 32), (1, 1000, 5, 32), (1, 33, 1, 32),
+                                     (1, 65, 1, 128), (1, 33, 2, 64), (3, 130, 21, 128),
+                                     (1, 1, 1, 32)])
+def test_token_groups_vs_oracle(oracle, B, T, H, d):
+    announce(f"efla_forward_hip / efla_backward_hip groups B={B} T={T} H={H} d={d}")
+    k, v, do, s0 = _inputs(oracle, 0x6209 + T + d, B, T, H, d, 0.2)
+    _fwd_bwd_vs_oracle(oracle, k, v, do, s0, B, T, H, d, 0.8, f"T={T}")
+
+
+@pytest.mark.parametrize("T,d", [(200, 128), (515, 128), (200, 64)])
+def test_token_groups_same_bits(oracle, T, d):
+    """128 (b, h) fill the chip with one group of tokens (d = 128; two for d =
+    64) each, two of them alone run in many groups: the same bits."""
+    from ceo_amd.efla import efla_backward, efla_forward
+
+    H = 128
+    announce(f"token groups, {H} heads against 2 alone, T={T} d={d}")
+    k, v, do, s0 = (_u16_to_dev(a) for a in _inputs(oracle, 77 + T, 1, T, H, d, 0.2))
+    few = slice(62, 64)
+    st, st2 = s0.clone(), s0[few].clone()
+    o = efla_forward(k, v, st, 0.7)
+    gk, gv, gs = efla_backward(do, k, v, s0, 0.7)
+    k2, v2, do2 = (t[:, :, few].contiguous() for t in (k, v, do))
+    o2 = efla_forward(k2, v2, st2, 0.7)
+    gk2, gv2, gs2 = efla_backward(do2, k2, v2, s0[few].contiguous(), 0.7)
+    torch.cuda.synchronize()
+    for n, a, b in (("o", o[:, :, few], o2), ("grad_k", gk[:, :, few], gk2),
+                    ("grad_v", gv[:, :, few], gv2), ("state", st[few], st2),
+                    ("grad_state", gs[few], gs2)):
+        assert torch.equal(a, b), n

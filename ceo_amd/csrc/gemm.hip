@@ -440,34 +440,108 @@ static bool direct_rows(const FastOp& o, long lines, long K) {
            aligned_to(o.p, 16);
 }
 
-// 8 waves (two per SIMD) measured faster than 4 at every config-4 shape
-template <typename T, int EPI, bool RAGGED>
-static void fast_kernel_launch(const FastOp& a, const FastOp& b, const gf::Opnd& A,
+// How a product is cut: output tiles of ts x ts, the contraction into ksplit
+// ranges of kper.
+struct Tiling {
+    int ts, ksplit;
+    long tiles, kper;
+};
+
+// The tile and the split of a product, by its estimated time.  Per 64-deep
+// k-iteration a 128-tile takes 0.71 us alone on its CU and 1.06 beside another,
+// a 256-tile 1.34 to 1.79 us as the chip fills; start and epilogue 4 and 6.5 us;
+// workgroups past the chip's room come in rounds.  A split writes and reads its
+// fp32 partials and launches the reduction.  Large products keep the 256-tile
+// (16384 x 1024 x 4096: 134 us against 155); those whose 256-tiles do not fill
+// the chip take the smaller one.  Measured (256-tile with its best split /
+// 128-tile with its best, us; m x k x n, forward):
+//    130 x 1024 x 4096  18.6 / 14.2     130 x 4096 x 1024  20.7 / 15.0
+//    400 x 1024 x 1024  17.5 / 12.7    1000 x 1024 x 4096  30.7 / 17.6
+//   1000 x 1024 x 1024  24.3 / 15.5    2500 x 4096 x 1024  46.3 / 38.0
+//   2500 x 1024 x 1024  27.5 / 16.2    6000 x 1024 x 1024  30.8 / 21.5
+//   6000 x 1024 x 4096  64.7 / 62.3   16384 x 1024 x 1024  36.1 / 42.0
+static double tiling_cost(int ts, long M, long N, long K, int ksplit, long kper, long cus) {
+    const double it = (double)((kper + gf::BK - 1) / gf::BK);
+    const long w = ((M + ts - 1) / ts) * ((N + ts - 1) / ts) * ksplit;
+    double t;
+    if (ts == 128) {
+        const double alone = it * 0.71 + 3.7, paired = it * 1.06 + 4.;
+        const long full = w / (2 * cus), rest = w % (2 * cus);
+        t = (double)full * paired + (rest == 0 ? 0. : rest <= cus ? alone : paired);
+    } else {
+        const long full = w / cus, rest = w % cus;
+        auto round = [&](double fill) { return it * (1.34 + 0.45 * fill) + 6.5; };
+        t = (double)full * round(1.) + (rest ? round((double)rest / (double)cus) : 0.);
+    }
+    if (ksplit > 1) t += 3. + (double)ksplit * (double)M * (double)N * 4. * 1.3 / 4.5e6;
+    return t;
+}
+
+static Tiling plan_tiling(long M, long N, long K, bool may_split) {
+    const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    Tiling best{};
+    double least = 0.;
+    for (int ts : {256, 128}) {
+        const long tiles = ((M + ts - 1) / ts) * ((N + ts - 1) / ts);
+        // at least 4 k-iterations to a split, no more workgroups than fit
+        const long slots = ts == 256 ? cus : 2 * cus;
+        const long most =
+            may_split ? std::max(1L, std::min({slots / tiles, K / (4 * gf::BK), 32L})) : 1;
+        for (long n = 1; n <= most; ++n) {
+            const long kper =
+                n == 1 ? K : ((K + n - 1) / n + gf::BK - 1) / gf::BK * gf::BK;
+            const int ksplit = (int)((K + kper - 1) / kper);
+            if (ksplit != n) continue;
+            const double t = tiling_cost(ts, M, N, K, ksplit, kper, cus);
+            if (best.ts == 0 || t < least) {
+                best = Tiling{ts, ksplit, tiles, kper};
+                least = t;
+            }
+        }
+    }
+    return best;
+}
+
+template <typename T, int EPI, bool RAGGED, int TS>
+static void fast_kernel_launch_ts(const FastOp& a, const FastOp& b, const gf::Opnd& A,
                                const gf::Opnd& B, long M, long N, long K,
                                const gf::EpiArgs<T>& ea, int ksplit, long kper, long tiles,
                                const char* name, hipStream_t st) {
-    // persistent: at most one workgroup per CU (the LDS allows no more)
+    // persistent: as many workgroups as the LDS holds (one or two per CU)
     const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
-    const long items = tiles * ksplit;
-    const dim3 grid((unsigned)(items < cus ? items : cus)), block(64 * 8);
+    const long items = tiles * ksplit, most = TS == 256 ? cus : 2 * cus;
+    const dim3 grid((unsigned)(items < most ? items : most)), block(64 * gf::tile_waves<TS>());
     // the GELU forms exist for the layouts their entry points have
     constexpr bool fwd = EPI != gf::EPI_DGELU, any = EPI != gf::EPI_DGELU && EPI != gf::EPI_GELU_AUX;
     if constexpr (any || !fwd)
         if (a.kc && b.kc)
-            EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, true, true, EPI, 8, RAGGED>), grid, block,
+            EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, true, true, EPI, TS, RAGGED>), grid, block,
                         st, A, B, M, N, K, ea, ksplit, kper);
     if constexpr (fwd)
         if (a.kc && !b.kc)
-            EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, true, false, EPI, 8, RAGGED>), grid, block,
+            EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, true, false, EPI, TS, RAGGED>), grid, block,
                         st, A, B, M, N, K, ea, ksplit, kper);
     if constexpr (any) {
         if (!a.kc && b.kc)
-            EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, false, true, EPI, 8, RAGGED>), grid, block,
+            EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, false, true, EPI, TS, RAGGED>), grid, block,
                         st, A, B, M, N, K, ea, ksplit, kper);
         if (!a.kc && !b.kc)
-            EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, false, false, EPI, 8, RAGGED>), grid,
+            EFLA_LAUNCH(name, (gf::gemm_fast_kernel<T, false, false, EPI, TS, RAGGED>), grid,
                         block, st, A, B, M, N, K, ea, ksplit, kper);
     }
+}
+
+template <typename T, int EPI, bool RAGGED>
+static void fast_kernel_launch(const FastOp& a, const FastOp& b, const gf::Opnd& A,
+                               const gf::Opnd& B, long M, long N, long K,
+                               const gf::EpiArgs<T>& ea, const Tiling& tl, const char* name,
+                               hipStream_t st) {
+    if (tl.ts == 128)
+        fast_kernel_launch_ts<T, EPI, RAGGED, 128>(a, b, A, B, M, N, K, ea, tl.ksplit, tl.kper,
+                                                   tl.tiles, name, st);
+    else
+        fast_kernel_launch_ts<T, EPI, RAGGED, 256>(a, b, A, B, M, N, K, ea, tl.ksplit, tl.kper,
+                                                   tl.tiles, name, st);
 }
 
 // Few-row products (gemm_skinny.hpp) up to this many rows, four 16-row tiles a
@@ -555,8 +629,7 @@ constexpr long kPadMinWork = (long)1 << 22;
 constexpr size_t kPadMaxBytes = (size_t)4 << 30;
 
 // Large-tile product, or -1 if it does not take the problem (the generic
-// kernel does).  Problems with fewer output tiles than the GPU has CUs
-// and a long contraction are split along k: fp32
+// kernel does).  Where the contraction is split (plan_tiling), fp32
 // partial tiles go to the stream's cached workspace and a second kernel adds
 // them in split order and runs the epilogue (plain epilogues only).
 // Workspace: [head_bytes for the caller (ea.cpart) | padded A | padded B |
@@ -576,20 +649,9 @@ static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
                            (!ea.aux || (ea.ldaux % 8 == 0 && aligned_to(ea.aux, 16)));
     const bool plain = !pa && !pb && K % 8 == 0 && out_whole;
     if (!plain && (double)M * (double)N * (double)K < (double)kPadMinWork) return -1;
-    const long tiles = ((M + gf::BM - 1) / gf::BM) * ((N + gf::BN - 1) / gf::BN);
-    if (tiles > 0x7FFFFFFFL / 64) return plain ? kInvalidConfiguration : -1;
-    int ksplit = 1;
-    const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
-    if ((EPI == gf::EPI_PLAIN || EPI == gf::EPI_RESID) && tiles < cus) {
-        const long want = cus / tiles;       // splits that fill every CU once
-        const long most = K / (4 * gf::BK);  // at least 4 k-iterations each
-        ksplit = (int)std::max(1L, std::min({want, most, 32L}));
-    }
-    long kper = K;
-    if (ksplit > 1) {
-        kper = ((K + ksplit - 1) / ksplit + gf::BK - 1) / gf::BK * gf::BK;
-        ksplit = (int)((K + kper - 1) / kper);
-    }
+    const Tiling tl = plan_tiling(M, N, K, EPI == gf::EPI_PLAIN || EPI == gf::EPI_RESID);
+    if (tl.tiles > 0x7FFFFFFFL / 64) return plain ? kInvalidConfiguration : -1;
+    const int ksplit = tl.ksplit;
     // scratch
     auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
     auto padded = [&](const FastOp& o, long lines, long& rows, long& cols) {
@@ -639,22 +701,20 @@ static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
     const bool ragged = !out_whole;
     if (ksplit == 1) {
         if (ragged)
-            fast_kernel_launch<T, EPI, true>(a, b, A, B, M, N, K, ep, 1, K, tiles, name, st);
+            fast_kernel_launch<T, EPI, true>(a, b, A, B, M, N, K, ep, tl, name, st);
         else
-            fast_kernel_launch<T, EPI, false>(a, b, A, B, M, N, K, ep, 1, K, tiles, name, st);
+            fast_kernel_launch<T, EPI, false>(a, b, A, B, M, N, K, ep, tl, name, st);
         return (int)hipPeekAtLastError();
     }
     if constexpr (EPI == gf::EPI_PLAIN || EPI == gf::EPI_RESID) {
         ep.part = (float*)(ws + up(head_bytes) + ba + bb);
         const long g = std::min(4096L, (M * ((N + 3) / 4) + 255) / 256);
         if (ragged) {
-            fast_kernel_launch<T, gf::EPI_PARTIAL, true>(a, b, A, B, M, N, K, ep, ksplit, kper,
-                                                         tiles, name, st);
+            fast_kernel_launch<T, gf::EPI_PARTIAL, true>(a, b, A, B, M, N, K, ep, tl, name, st);
             EFLA_LAUNCH("gemm_splitk_reduce", (gf::gemm_splitk_reduce<T, true>),
                         dim3((unsigned)g), dim3(256), st, ep, M, N, ksplit);
         } else {
-            fast_kernel_launch<T, gf::EPI_PARTIAL, false>(a, b, A, B, M, N, K, ep, ksplit, kper,
-                                                          tiles, name, st);
+            fast_kernel_launch<T, gf::EPI_PARTIAL, false>(a, b, A, B, M, N, K, ep, tl, name, st);
             EFLA_LAUNCH("gemm_splitk_reduce", (gf::gemm_splitk_reduce<T, false>),
                         dim3((unsigned)g), dim3(256), st, ep, M, N, ksplit);
         }
@@ -932,9 +992,10 @@ extern "C" int gemm_gelu_backward_hip(const void* grad_c, const void* a, const v
                 gf::EpiArgs<bf16> ea = epi<bf16>(grad_pre, (long)k, nullptr, 1.f, 0.f, nullptr, 0,
                                                  (void*)pre, (long)k);
                 // grad_pre's column sums from the epilogue: one fp32 row per
-                // 128 output rows, then their sum (whole 16-byte pieces only)
+                // half tile of output rows, then their sum (whole 16-byte pieces only)
                 WsLease lease;
-                const long prow = ((long)m + 127) / 128;
+                const Tiling tl = plan_tiling((long)m, (long)k, (long)n, false);
+                const long prow = ((long)m + tl.ts / 2 - 1) / (tl.ts / 2);
                 const bool sums = grad_pre_bias && k % 8 == 0;
                 done = fast_launch<bf16, gf::EPI_DGELU>(
                     fa, fb, (long)m, (long)k, (long)n, ea, "gemm_gelu_bwd_da", stream,

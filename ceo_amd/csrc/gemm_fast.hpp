@@ -6,14 +6,14 @@
 // ("line-contiguous", LC).  The four combinations cover the forward product
 // (A KC, B LC), dA = dC B^T (both KC) and dB = A^T dC (both LC).
 //
-// Workgroup tile 256 x 256 x 64.  The library launches eight waves (two per
-// SIMD), each owning 128 x 64 of the output as 4 x 2 tiles of
-// v_mfma_f32_32x32x16; the kernel also compiles for four waves of 128 x 128
-// (4 x 4 tiles).
+// Workgroup tile 256 x 256 x 64: eight waves (two per SIMD), each owning
+// 128 x 64 of the output as 4 x 2 tiles of v_mfma_f32_32x32x16; or, for
+// products with too few such tiles, 128 x 128 x 64: four waves of 64 x 64, two
+// workgroups to a CU.
 // The product is formed transposed, C^T = B^T A^T: B's fragments are the MFMA
 // A operand (rows n) and A's the B operand (columns m), so each lane ends up
 // holding 4 consecutive n of one output row m and writes 8-byte row pieces.
-// Per k-iteration each operand tile (256 lines x 64 k, 32 KB) is copied
+// Per k-iteration each operand tile (TS lines x 64 k) is copied
 // straight from global memory into LDS (global_load_lds_dwordx4, 16 bytes per
 // lane, no VGPR staging) one iteration ahead, double-buffered; all of an
 // iteration's copies are issued at its start, and the MFMA operand fragments
@@ -23,7 +23,7 @@
 // of bank conflicts:
 //   KC tile [line][k]  (128 B rows):  chunk c of line L at c ^ ((L >> 1) & 7)
 //     read with one 16-byte ds_read per lane (lanes 0-15 = 16 lines, one chunk)
-//   LC tile [k][line]  (512 B rows):  chunk c of row k at c ^ (4 (k & 3))
+//   LC tile [k][line]  (2 TS B rows): chunk c of row k at c ^ (4 (k & 3))
 //     read with two ds_read_b64_tr_b16 per lane (4 k rows x 32 lines per half wave)
 // A k-tail (K not a multiple of 64) runs one last iteration through registers
 // with the missing k zeroed.  Rows and columns past M or N are clamped on load
@@ -54,8 +54,16 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 typedef __attribute__((__vector_size__(4 * sizeof(short)))) short short4v;
 typedef __attribute__((address_space(3))) short4v lds_short4v;
 
-constexpr int BM = 256, BN = 256, BK = 64, NT = 256;
-constexpr int TILE_BYTES = 256 * 64 * 2;  // one operand tile
+constexpr int BK = 64;
+// a tile of TS lines (TS = 256 or 128): bytes of one operand tile, waves
+template <int TS>
+constexpr int tile_bytes() {
+    return TS * BK * 2;
+}
+template <int TS>
+constexpr int tile_waves() {
+    return TS / 32;
+}
 
 template <typename T>
 __device__ __forceinline__ floatx16 mma32(bf16x8 a, bf16x8 b, floatx16 c) {
@@ -70,13 +78,14 @@ __device__ __forceinline__ floatx16 mma32(bf16x8 a, bf16x8 b, floatx16 c) {
 __device__ __forceinline__ unsigned kc_off(int line, int chunk) {
     return (unsigned)(line * 128 + ((chunk ^ ((line >> 1) & 7)) << 4));
 }
+template <int TS>
 __device__ __forceinline__ unsigned lc_off(int krow, int line) {  // line = element column
-    return (unsigned)(krow * 512 + (((line >> 3) ^ ((krow & 3) << 2)) << 4) + ((line & 7) << 1));
+    return (unsigned)(krow * (2 * TS) + (((line >> 3) ^ ((krow & 3) << 2)) << 4) + ((line & 7) << 1));
 }
 
 // One 32-line x 16-k MFMA operand (lane l: line l & 31, k = 8 (l >> 5) .. + 7)
 // from a tile, k step ks (0..3), lines line0 .. line0 + 31.
-template <bool KC>
+template <bool KC, int TS>
 __device__ __forceinline__ bf16x8 frag(const char* tile, int line0, int ks, int l) {
     if constexpr (KC) {
         return *reinterpret_cast<const bf16x8*>(tile + kc_off(line0 + (l & 31), 2 * ks + (l >> 5)));
@@ -86,9 +95,9 @@ __device__ __forceinline__ bf16x8 frag(const char* tile, int line0, int ks, int 
         const int G = l >> 4, a = (l & 15) >> 2, b = l & 3;
         const int kr = 16 * ks + 8 * (G >> 1) + a;
         const int ln = line0 + 16 * (G & 1) + 4 * b;
-        const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4v*)(tile + lc_off(kr, ln)));
+        const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4v*)(tile + lc_off<TS>(kr, ln)));
         const short4v hi =
-            __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4v*)(tile + lc_off(kr + 4, ln)));
+            __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4v*)(tile + lc_off<TS>(kr + 4, ln)));
         const bf16x4 x = __builtin_bit_cast(bf16x4, lo), y = __builtin_bit_cast(bf16x4, hi);
         return bf16x8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
     }
@@ -102,19 +111,19 @@ struct Opnd {
     int nlines;        // M or N
 };
 
-// Direct copy of the tile (lines line0.., k k0..k0+63) into `tile` (LDS): 32
-// instructions of 64 16-byte chunks, 8 per wave.  The global side is
+// Direct copy of the tile (lines line0.., k k0..k0+63) into `tile` (LDS): TS / 8
+// instructions of 64 16-byte chunks, four per wave.  The global side is
 // permuted so the LDS side lands swizzled.  Offsets are 32-bit from a per-tile
 // scalar base (the host checks 256 * ld * 2 < 2^31).
-// Instruction q (of the tile's 32) goes to wave q % NW; a call issues this
-// wave's instructions numbered i0 .. i1 - 1 among its own.
-template <bool KC, int NW>
+// Instruction q goes to wave q % NW.
+template <bool KC, int TS>
 __device__ __forceinline__ void copy_tile(const Opnd& op, int line0, long k0, char* tile, int w,
-                                          int l, int i0 = 0, int i1 = 32 / NW) {
+                                          int l) {
+    constexpr int NW = tile_waves<TS>(), CR = TS / 8;  // chunks per row (line-contiguous)
     const char* base = KC ? op.base + ((long)line0 * op.ld + k0) * 2
                           : op.base + (k0 * op.ld + line0) * 2;
 #pragma unroll
-    for (int i = i0; i < i1; ++i) {
+    for (int i = 0; i < TS / 8 / NW; ++i) {
         const int q = NW * i + w;
         const int P = 64 * q + l;  // physical 16-byte chunk of the tile
         unsigned off;
@@ -123,7 +132,7 @@ __device__ __forceinline__ void copy_tile(const Opnd& op, int line0, long k0, ch
             const int gl = min(line, op.nlines - 1 - line0);
             off = (unsigned)(gl * op.ld + 8 * c) * 2u;
         } else {
-            const int kr = P >> 5, c = (P & 31) ^ ((kr & 3) << 2);
+            const int kr = P / CR, c = (P % CR) ^ ((kr & 3) << 2);
             const int gc = min(8 * c, op.nlines - 8 - line0);  // nlines % 8 == 0
             off = (unsigned)(kr * op.ld + gc) * 2u;
         }
@@ -134,11 +143,12 @@ __device__ __forceinline__ void copy_tile(const Opnd& op, int line0, long k0, ch
 // The k-tail tile through registers: k >= K reads as zero.  A k-contiguous
 // operand's row is zero between K and the next multiple of 8 (K % 8 == 0, or
 // rows padded by pad_rows_kernel), so its pieces are read whole.
-template <bool KC, int NTH>
+template <bool KC, int TS>
 __device__ __forceinline__ void copy_tile_tail(const Opnd& op, int line0, long k0, long K,
                                                char* tile, int tid) {
+    constexpr int NTH = 64 * tile_waves<TS>(), CR = TS / 8;
 #pragma unroll 4
-    for (int i = 0; i < 2048 / NTH; ++i) {
+    for (int i = 0; i < 8 * TS / NTH; ++i) {
         const int P = NTH * i + tid;
         bf16x8 x{};
         unsigned dst;
@@ -149,11 +159,11 @@ __device__ __forceinline__ void copy_tile_tail(const Opnd& op, int line0, long k
                 x = *reinterpret_cast<const bf16x8*>(op.base + ((long)gl * op.ld + k0 + 8 * c) * 2);
             dst = kc_off(line, c);
         } else {
-            const int kr = P >> 5, c = P & 31;
+            const int kr = P / CR, c = P % CR;
             const int gc = min(line0 + 8 * c, op.nlines - 8);
             if (k0 + kr < K)
                 x = *reinterpret_cast<const bf16x8*>(op.base + ((k0 + kr) * op.ld + gc) * 2);
-            dst = (unsigned)(kr * 512 + ((c ^ ((kr & 3) << 2)) << 4));
+            dst = (unsigned)(kr * (2 * TS) + ((c ^ ((kr & 3) << 2)) << 4));
         }
         *reinterpret_cast<bf16x8*>(tile + dst) = x;
     }
@@ -175,8 +185,8 @@ struct EpiArgs {
     T* aux;  // GELU_AUX: pre-activation out; DGELU: pre-activation in
     long ldaux;
     float* part;   // PARTIAL: fp32 partial sums [split][M][N rounded up to 8]
-    float* cpart;  // DGELU: column sums of the output, one fp32 row per 128 output
-                   // rows ([M / 128][N]), or NULL
+    float* cpart;  // DGELU: column sums of the output, one fp32 row per TS / 2 output
+                   // rows, or NULL
 };
 
 // W elements at p (element-aligned), the first cnt of them if cnt < W; those
@@ -231,7 +241,7 @@ __device__ __forceinline__ void epilogue4(const EpiArgs<T>& ea, long m, long n, 
 }
 
 // --- epilogue staged through LDS ---------------------------------------------
-// Each wave finishes its own 128 x (32 TNI) block of the output through a
+// Each wave finishes its own (32 TMJ) x (32 TNI) block of the output through a
 // private slice of the free LDS buffer (32 rows x 32 TNI columns of fp32,
 // 4 KB TNI), one 32-row m tile at a time: it writes alpha acc there in the
 // MFMA layout, reads it back as 8-element row pieces and finishes the
@@ -248,8 +258,8 @@ __device__ __forceinline__ unsigned ep_off(int row, int col) {  // col % 4 == 0
     return (unsigned)(row * (128 * TNI) + (((col >> 2) ^ (row & 15)) << 4));
 }
 
-template <typename T, int EPI, int TNI, bool AHEAD, bool RAGGED>
-__device__ __forceinline__ void epilogue_wave(const EpiArgs<T>& ea, const floatx16 (&acc)[TNI][4],
+template <typename T, int EPI, int TNI, int TMJ, bool AHEAD, bool RAGGED>
+__device__ __forceinline__ void epilogue_wave(const EpiArgs<T>& ea, const floatx16 (&acc)[TNI][TMJ],
                                               int split, long mw, long nw, long M, long N, int l,
                                               char* wp) {
     constexpr int WC = 32 * TNI;  // columns of the wave's block
@@ -288,7 +298,7 @@ __device__ __forceinline__ void epilogue_wave(const EpiArgs<T>& ea, const floatx
     t8 inp[2][NP];
     if (AHEAD && rd && mw < M) fetch(0, inp[0]);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < TMJ; ++j) {
         const long r0 = mw + 32 * j;
         if (r0 >= M) break;  // uniform over the wave
 #pragma unroll
@@ -302,7 +312,7 @@ __device__ __forceinline__ void epilogue_wave(const EpiArgs<T>& ea, const floatx
                     v[e] = (EPI == EPI_PARTIAL ? 1.f : ea.alpha) * acc[i][j][4 * qd + e];
                 *reinterpret_cast<mf::floatx4*>(wp + ep_off<TNI>(l & 31, col)) = v;
             }
-        if (AHEAD && rd && j + 1 < 4 && r0 + 32 < M) fetch(j + 1, inp[(j + 1) & 1]);
+        if (AHEAD && rd && j + 1 < TMJ && r0 + 32 < M) fetch(j + 1, inp[(j + 1) & 1]);
         if (!AHEAD && rd) fetch(j, inp[j & 1]);
 #pragma unroll
         for (int s = 0; s < NP; ++s) {
@@ -362,14 +372,14 @@ __device__ __forceinline__ void epilogue_wave(const EpiArgs<T>& ea, const floatx
     if constexpr (EPI == EPI_DGELU) {
         if (ea.cpart && mw < M) {
             // the lanes sharing a piece index hold different rows: sum them
-            // (fixed order), then one fp32 row of the wave's 128 rows
+            // (fixed order), then one fp32 row of the wave's rows
 #pragma unroll
             for (int e = 0; e < 8; ++e)
 #pragma unroll
                 for (int off = WC / 8; off < 64; off <<= 1) csum[e] += __shfl_xor(csum[e], off);
             const long n = nw + 8 * l;
             if (l < WC / 8 && n < N) {
-                float* dst = ea.cpart + (mw / 128) * N + n;
+                float* dst = ea.cpart + (mw / (32 * TMJ)) * N + n;
                 *reinterpret_cast<mf::floatx4*>(dst) = mf::floatx4{csum[0], csum[1], csum[2], csum[3]};
                 *reinterpret_cast<mf::floatx4*>(dst + 4) =
                     mf::floatx4{csum[4], csum[5], csum[6], csum[7]};
@@ -379,9 +389,9 @@ __device__ __forceinline__ void epilogue_wave(const EpiArgs<T>& ea, const floatx
 }
 
 // --- the kernel --------------------------------------------------------------
-// NW waves: 2 along m, NW / 2 along n; a wave owns 128 (m) x 512 / NW (n) of
-// the output (4 x 4 tiles of 32 x 32 for NW = 4, 4 x 2 for NW = 8, which puts
-// two waves on each SIMD).
+// NW = TS / 32 waves, 2 along m, NW / 2 along n; a wave owns TS / 2 (m) x 64 (n)
+// of the output: TS = 256 has eight waves (two per SIMD) of 4 x 2 tiles of
+// 32 x 32, TS = 128 four of 2 x 2, two such workgroups to a CU.
 //
 // Persistent: workgroup b takes work items b, b + gridDim.x, ... (an item is
 // an output tile, or a (tile, k-split) pair with ksplit > 1).  The LDS double
@@ -397,12 +407,12 @@ struct Item {
     long kbeg, klen;
 };
 
-template <typename T, bool AKC, bool BKC, int EPI, int NW, bool RAGGED>
-__global__ void __launch_bounds__(64 * NW) gemm_fast_kernel(Opnd A, Opnd B, long M, long N,
+template <typename T, bool AKC, bool BKC, int EPI, int TS, bool RAGGED>
+__global__ void __launch_bounds__(64 * tile_waves<TS>(), 2) gemm_fast_kernel(Opnd A, Opnd B, long M, long N,
                                                             long K, EpiArgs<T> ea, int ksplit,
                                                             long kper) {
-    constexpr int NTH = 64 * NW;
-    constexpr int TNI = 8 / NW * 2;  // 32-wide n tiles per wave: 4 (NW = 4) or 2 (NW = 8)
+    constexpr int BM = TS, BN = TS, TILE_BYTES = tile_bytes<TS>();
+    constexpr int TNI = 2, TMJ = TS / 64;  // 32 x 32 tiles per wave along n and m
     // two buffers of [A tile | B tile]; the epilogue stages the output through
     // the one the next item's first k-block is not in
     __shared__ __attribute__((aligned(1024))) char smem[4 * TILE_BYTES];
@@ -429,7 +439,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_fast_kernel(Opnd A, Opnd B, long
     };
 
     const int w = mf::wave(), l = mf::lane();
-    const int wm = (w & 1) * 128, wn = (w >> 1) * (32 * TNI);  // this wave's block
+    const int wm = (w & 1) * (TS / 2), wn = (w >> 1) * (32 * TNI);  // this wave's block
     // buffer b: A at smem + 2b * TILE_BYTES, B right after it
     auto As = [&](int b) { return smem + 2 * b * TILE_BYTES; };
     auto Bs = [&](int b) { return smem + (2 * b + 1) * TILE_BYTES; };
@@ -440,11 +450,11 @@ __global__ void __launch_bounds__(64 * NW) gemm_fast_kernel(Opnd A, Opnd B, long
     decode(it, cur);
     // the first item's first k-block
     if (cur.klen >= BK) {
-        copy_tile<AKC, NW>(A, cur.m0, cur.kbeg, As(0), w, l);
-        copy_tile<BKC, NW>(B, cur.n0, cur.kbeg, Bs(0), w, l);
+        copy_tile<AKC, TS>(A, cur.m0, cur.kbeg, As(0), w, l);
+        copy_tile<BKC, TS>(B, cur.n0, cur.kbeg, Bs(0), w, l);
     } else {
-        copy_tile_tail<AKC, NTH>(A, cur.m0, cur.kbeg, K, As(0), threadIdx.x);
-        copy_tile_tail<BKC, NTH>(B, cur.n0, cur.kbeg, K, Bs(0), threadIdx.x);
+        copy_tile_tail<AKC, TS>(A, cur.m0, cur.kbeg, K, As(0), threadIdx.x);
+        copy_tile_tail<BKC, TS>(B, cur.n0, cur.kbeg, K, Bs(0), threadIdx.x);
     }
     mf::dma_wait();
     __syncthreads();
@@ -454,11 +464,11 @@ __global__ void __launch_bounds__(64 * NW) gemm_fast_kernel(Opnd A, Opnd B, long
         const bool more = nitn < nitems;
         Item nxt = cur;
         if (more) decode(nitn, nxt);
-        floatx16 acc[TNI][4];  // [n tile][m tile]
+        floatx16 acc[TNI][TMJ];  // [n tile][m tile]
 #pragma unroll
         for (int i = 0; i < TNI; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < TMJ; ++j)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
         const long nfull = cur.klen / BK;  // whole k-iterations (direct copies)
@@ -477,14 +487,14 @@ __global__ void __launch_bounds__(64 * NW) gemm_fast_kernel(Opnd A, Opnd B, long
             const long k0 = own ? cur.kbeg + (kt + 1) * BK : nxt.kbeg;
             const bool direct = own ? kt + 1 < nfull : nxt.klen >= BK;
             if (fetch && !direct) {
-                copy_tile_tail<AKC, NTH>(A, src.m0, k0, K, As(buf ^ 1), threadIdx.x);
-                copy_tile_tail<BKC, NTH>(B, src.n0, k0, K, Bs(buf ^ 1), threadIdx.x);
+                copy_tile_tail<AKC, TS>(A, src.m0, k0, K, As(buf ^ 1), threadIdx.x);
+                copy_tile_tail<BKC, TS>(B, src.n0, k0, K, Bs(buf ^ 1), threadIdx.x);
             }
             const char* at = As(buf);
             const char* bt = Bs(buf);
             // fragments double-buffered in registers: k step ks + 1 is read
             // while the MFMAs of k step ks run
-            bf16x8 fb[2][TNI], fa[2][4];
+            bf16x8 fb[2][TNI], fa[2][TMJ];
             // the iteration's reads, copies and MFMAs issue at raised wave
             // priority, the wait for the next block at the normal one: a wave
             // still computing wins the SIMD's issue slots over its partner
@@ -493,16 +503,16 @@ __global__ void __launch_bounds__(64 * NW) gemm_fast_kernel(Opnd A, Opnd B, long
             __builtin_amdgcn_s_setprio(1);
             if (act) {
 #pragma unroll
-                for (int i = 0; i < TNI; ++i) fb[0][i] = frag<BKC>(bt, wn + 32 * i, 0, l);
+                for (int i = 0; i < TNI; ++i) fb[0][i] = frag<BKC, TS>(bt, wn + 32 * i, 0, l);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) fa[0][j] = frag<AKC>(at, wm + 32 * j, 0, l);
+                for (int j = 0; j < TMJ; ++j) fa[0][j] = frag<AKC, TS>(at, wm + 32 * j, 0, l);
             }
             // the next block's copies all go out now, a whole iteration ahead
             // of the wait (the buffer they fill was last read in the previous
             // iteration, which every wave has finished)
             if (fetch && direct) {
-                copy_tile<AKC, NW>(A, src.m0, k0, As(buf ^ 1), w, l);
-                copy_tile<BKC, NW>(B, src.n0, k0, Bs(buf ^ 1), w, l);
+                copy_tile<AKC, TS>(A, src.m0, k0, As(buf ^ 1), w, l);
+                copy_tile<BKC, TS>(B, src.n0, k0, Bs(buf ^ 1), w, l);
             }
             if (act) {
 #pragma unroll
@@ -511,20 +521,20 @@ __global__ void __launch_bounds__(64 * NW) gemm_fast_kernel(Opnd A, Opnd B, long
                     if (ks + 1 < BK / 16) {
 #pragma unroll
                         for (int i = 0; i < TNI; ++i)
-                            fb[c ^ 1][i] = frag<BKC>(bt, wn + 32 * i, ks + 1, l);
+                            fb[c ^ 1][i] = frag<BKC, TS>(bt, wn + 32 * i, ks + 1, l);
 #pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            fa[c ^ 1][j] = frag<AKC>(at, wm + 32 * j, ks + 1, l);
+                        for (int j = 0; j < TMJ; ++j)
+                            fa[c ^ 1][j] = frag<AKC, TS>(at, wm + 32 * j, ks + 1, l);
                     }
 #pragma unroll
                     for (int i = 0; i < TNI; ++i)
 #pragma unroll
-                        for (int j = 0; j < 4; ++j)
+                        for (int j = 0; j < TMJ; ++j)
                             acc[i][j] = mma32<T>(fb[c][i], fa[c][j], acc[i][j]);
                     if (ks + 1 < BK / 16) {
                         // one LDS read between consecutive MFMAs
-                        constexpr int NR = TNI * (BKC ? 1 : 2) + 4 * (AKC ? 1 : 2);
-                        constexpr int NM = 4 * TNI;
+                        constexpr int NR = TNI * (BKC ? 1 : 2) + TMJ * (AKC ? 1 : 2);
+                        constexpr int NM = TMJ * TNI;
                         constexpr int R = NR < NM ? NR : NM;
 #pragma unroll
                         for (int r = 0; r < R; ++r) {
@@ -549,7 +559,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_fast_kernel(Opnd A, Opnd B, long
         {
             const int le = mf::tid_in((int)it) & 63;
             char* wp = smem + 2 * (buf ^ 1) * TILE_BYTES + (4096 * TNI) * w;
-            epilogue_wave<T, EPI, TNI, AKC && BKC, RAGGED>(ea, acc, cur.split, (long)cur.m0 + wm,
+            epilogue_wave<T, EPI, TNI, TMJ, AKC && BKC, RAGGED>(ea, acc, cur.split, (long)cur.m0 + wm,
                                                     (long)cur.n0 + wn, M, N, le, wp);
         }
         __syncthreads();  // the next item's first copies refill the buffer

@@ -473,7 +473,7 @@ def test_token_stride_rejects_other_layouts():
 # A few tokens from a carried state: around the longest that the step kernel
 # takes, the smallest problem, each state shape, fused projection rows.  Its
 # state stays in fp32 throughout: S_T to 1e-5 (K + T fp32 sums of 128 terms);
-# the bf16 output is rounded once, to 2^-9.
+# the bf16 output is rounded once (8 significant bits: at most 2^-8).
 @pytest.mark.parametrize("T", [1, 2, 5, 6, 7])
 @pytest.mark.parametrize("dtype,K,V", [(torch.bfloat16, 64, 64), (torch.bfloat16, 64, 256),
                                        (torch.bfloat16, 128, 128), (torch.bfloat16, 128, 64),
@@ -496,7 +496,7 @@ def test_steps_from_carried_state(oracle, dtype, K, V, T):
     eo, es = rel_l2(o, ro), rel_l2(st, rst)
     print(f"  rel-L2 o {eo:.2e} S_T {es:.2e}", flush=True)
     steps = T <= 6
-    assert eo <= (1e-5 if dtype == torch.float32 else 2.0 ** -9 if steps else TOL[dtype])
+    assert eo <= (1e-5 if dtype == torch.float32 else 2.0 ** -8 if steps else TOL[dtype])
     assert es <= (1e-5 if dtype == torch.float32 or steps else TOL[dtype])
     assert torch.equal(s0, torch.from_numpy(S0).cuda())
     if dtype == torch.bfloat16:

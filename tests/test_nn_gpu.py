@@ -622,7 +622,7 @@ def test_gemm_odd_shapes_large_tile(m, k, n):
     errs["dgelu"] = 0.5 * off(dpre, gl)
     errs["dpre_bias"] = off(pb, dpre.double().sum(0))
     print("  rel-L2:", {n_: f"{v:.2e}" for n_, v in errs.items()}, flush=True)
-    assert all(v <= 2.0 ** -9 for v in errs.values()), errs
+    assert all(v <= 2.0 ** -8 for v in errs.values()), errs
 
 
 def test_gemm_odd_shape_ignores_what_surrounds_it():
@@ -649,7 +649,7 @@ def test_gemm_odd_shape_ignores_what_surrounds_it():
                 out = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
                 nn.gemm_ex(a, b, out, trans_a=ta, trans_b=tb)
                 ref = (a.double().T if ta else a.double()) @ (b.double().T if tb else b.double())
-                assert ((out.double() - ref).norm() / ref.norm()).item() <= 2.0 ** -9
+                assert ((out.double() - ref).norm() / ref.norm()).item() <= 2.0 ** -8
 
 
 # few rows (the kernel that streams the weights once): row counts around the
@@ -682,7 +682,47 @@ def test_gemm_few_rows(m, k, n, dt):
         errs["pre"] = off(pre, A @ B + bias.double())
         errs["gelu"] = off(act, torch.nn.functional.gelu(pre.double(), approximate="tanh"))
     print("  rel-L2:", {n_: f"{v:.2e}" for n_, v in errs.items()}, flush=True)
-    assert all(v <= 2.0 ** -9 for v in errs.values()), errs
+    assert all(v <= 2.0 ** -8 for v in errs.values()), errs
     if m <= 64:  # a row does not depend on how many others there are
         assert torch.equal(nn.gemm_forward(a[:1].contiguous(), b, bias),
                            nn.gemm_forward(a, b, bias)[:1])
+
+
+# the smaller tile of the large-tile kernel: around its 128-line edges, with and
+# without a split contraction, every layout and epilogue.  Bound as above: one
+# bf16 rounding of an fp32 sum.
+@pytest.mark.parametrize("m,k,n", [(127, 1024, 128), (129, 64, 136), (256, 72, 264),
+                                   (400, 4096, 1024), (1000, 512, 2048)])
+def test_gemm_small_tile(m, k, n):
+    from ceo_amd import nn
+
+    announce(f"gemm 128-tile {m}x{k}x{n}")
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+
+    def r(*s):
+        return torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+
+    def off(got, ref):
+        return ((got.double() - ref).norm() / ref.norm()).item()
+
+    a, b, dc, bias, u = r(m, k), r(k, n), r(m, n), r(n), r(m, k)
+    A, B, D = a.double(), b.double(), dc.double()
+    errs = {"fwd": off(nn.gemm_forward(a, b, bias), A @ B + bias.double())}
+    da, db, _ = nn.gemm_backward(dc, a, b)
+    errs.update(da=off(da, D @ B.T), db=off(db, A.T @ D))
+    out = nn.gemm_ex(a, b, torch.empty_like(dc), bias=bias, c=dc, beta=1.0)
+    errs["resid"] = off(out, A @ B + bias.double() + D)
+    at, bt = a.T.contiguous(), b.T.contiguous()
+    errs["tt"] = off(nn.gemm_ex(at, bt, torch.empty_like(dc), trans_a=True, trans_b=True), A @ B)
+    pre, act = nn.gemm_gelu_forward(a, b, bias)
+    errs["pre"] = off(pre, A @ B + bias.double())
+    errs["gelu"] = off(act, torch.nn.functional.gelu(pre.double(), approximate="tanh"))
+    pb = torch.empty(k, dtype=torch.bfloat16, device="cuda")
+    dpre, _, _ = nn.gemm_gelu_backward(dc, a, b, u, need_b=False, out_pre_bias=pb)
+    x = u.double().requires_grad_(True)
+    (gl,) = torch.autograd.grad(torch.nn.functional.gelu(x, approximate="tanh"), x, da.double())
+    # the product is rounded twice here (to bf16, and after GELU')
+    errs["dgelu"] = 0.5 * off(dpre, gl)
+    errs["dpre_bias"] = off(pb, dpre.double().sum(0))
+    print("  rel-L2:", {n_: f"{v:.2e}" for n_, v in errs.items()}, flush=True)
+    assert all(v <= 2.0 ** -8 for v in errs.values()), errs

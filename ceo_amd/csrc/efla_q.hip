@@ -40,8 +40,14 @@
 namespace efla {
 namespace q {
 
-constexpr int NTH = 256;  // threads per workgroup
-constexpr int NW = 4;     // waves per workgroup
+// The fp32 kernels run 16 waves per workgroup, one 16 x 16 tile of a 64 x 64
+// product each: a tile is a chain of 16 dependent fp32 MFMAs with scalar LDS
+// operands, and small fp32 problems have few workgroups, so their time is these
+// chains' latency.  With four waves of four tiles each, one after the other, the
+// forward and backward of 2 x 256 tokens, 4 heads, d = 64 took 234 us (its seven
+// kernels 237 us together under a trace); with sixteen 175 us (126 us).
+constexpr int NTH = 1024;  // threads per workgroup
+constexpr int NW = 16;     // waves per workgroup
 constexpr int LDF = 68;   // row stride of the 64x64 fp32 LDS matrices
 
 template <typename T>
@@ -139,8 +145,7 @@ __global__ void __launch_bounds__(1024) chunk_offsets_kernel(const int32_t* __re
 // Ends with a workgroup barrier.
 // ---------------------------------------------------------------------------
 template <typename MT, int K, typename TK>
-__device__ void compute_T(const TK* Ks, int ldk, const float* bs, float* Gs, float* Ts,
-                          float* Ysc) {
+__device__ void compute_T(const TK* Ks, int ldk, const float* bs, float* Gs, float* Ts) {
     block_gemm<MT, 64, 64, K, NW>(view_k(Ks, ldk), view_k(Ks, ldk), SkipUpper{},
                                   [&](int r, int c, floatx4 acc) {
 #pragma unroll
@@ -149,46 +154,35 @@ __device__ void compute_T(const TK* Ks, int ldk, const float* bs, float* Gs, flo
     for (int i = threadIdx.x; i < 64 * LDF; i += NTH) Ts[i] = 0.f;
     __syncthreads();
     const int w = wave_id(), l = lane_id();
-    if (l < 16) {
+    if (w < 4 && l < 16) {
         const int base = 16 * w, c = l;
         float x[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            float s = (i == c) ? 1.f : 0.f;
-            const float bi = bs[base + i];
+            float s = 0.f;
 #pragma unroll
-            for (int j = 0; j < i; ++j) s -= bi * Gs[(base + i) * LDF + base + j] * x[j];
-            x[i] = s;
+            for (int j = 0; j < i; ++j) s += Gs[(base + i) * LDF + base + j] * x[j];
+            x[i] = (i == c ? 1.f : 0.f) - bs[base + i] * s;
         }
 #pragma unroll
         for (int i = 0; i < 16; ++i) Ts[(base + i) * LDF + base + c] = x[i];
     }
     __syncthreads();
-    const int r = l >> 2, c0 = 4 * (l & 3);
-    float* Y = Ysc + w * 16 * 17;
+    const int r = l & 15, g = l >> 4;
     for (int d = 1; d < 4; ++d) {
-        const int I = w + d, J = w;
         if (w < 4 - d) {
-            float y[4] = {0.f, 0.f, 0.f, 0.f};
+            const int I = w + d, J = w;
             const float bi = bs[16 * I + r];
-            for (int m = 16 * J; m < 16 * I; ++m) {
-                const float a = bi * Gs[(16 * I + r) * LDF + m];
+            floatx4 y = {0.f, 0.f, 0.f, 0.f}, t = {0.f, 0.f, 0.f, 0.f};
+            for (int m = 16 * J; m < 16 * I; m += 4)
+                y = Mfma<float>::mma(bi * Gs[(16 * I + r) * LDF + m + g],
+                                     Ts[(m + g) * LDF + 16 * J + r], y);
+            // y's rows 4 g + i are the next product's contraction index
 #pragma unroll
-                for (int qq = 0; qq < 4; ++qq) y[qq] += a * Ts[m * LDF + 16 * J + c0 + qq];
-            }
+            for (int i = 0; i < 4; ++i)
+                t = Mfma<float>::mma(Ts[(16 * I + r) * LDF + 16 * I + 4 * g + i], y[i], t);
 #pragma unroll
-            for (int qq = 0; qq < 4; ++qq) Y[r * 17 + c0 + qq] = y[qq];
-        }
-        __syncthreads();
-        if (w < 4 - d) {
-            float t[4] = {0.f, 0.f, 0.f, 0.f};
-            for (int m = 0; m < 16; ++m) {
-                const float a = Ts[(16 * I + r) * LDF + 16 * I + m];
-#pragma unroll
-                for (int qq = 0; qq < 4; ++qq) t[qq] += a * Y[m * 17 + c0 + qq];
-            }
-#pragma unroll
-            for (int qq = 0; qq < 4; ++qq) Ts[(16 * I + r) * LDF + 16 * J + c0 + qq] = -t[qq];
+            for (int i = 0; i < 4; ++i) Ts[(16 * I + 4 * g + i) * LDF + 16 * J + r] = -t[i];
         }
         __syncthreads();
     }
@@ -202,13 +196,15 @@ __device__ __forceinline__ void chunk_coeffs(const T* Ks, int ldk, const T* __re
                                              float* dcls, float* dcbs, float* bco_out) {
     const int t = threadIdx.x >> 2, part = threadIdx.x & 3;
     float s = 0.f;
-    for (int d = part; d < K; d += 4) {
-        const float x = to_f(Ks[t * ldk + d]);
-        s += x * x;
+    if (t < 64) {
+        for (int d = part; d < K; d += 4) {
+            const float x = to_f(Ks[t * ldk + d]);
+            s += x * x;
+        }
+        s += __shfl_xor(s, 1);
+        s += __shfl_xor(s, 2);
     }
-    s += __shfl_xor(s, 1);
-    s += __shfl_xor(s, 2);
-    if (part == 0) {
+    if (t < 64 && part == 0) {
         float c = 0.f, dcl = 0.f, dcb = 0.f;
         if (t < len) {
             efla_coeff(s, to_f(beta[(bos + t) * H + h]), c, dcl, dcb);
@@ -236,7 +232,6 @@ __global__ void __launch_bounds__(NTH) fwd_prep_kernel(const T* __restrict__ k,
     __shared__ __attribute__((aligned(16))) T Vs[64 * LDV];
     __shared__ __attribute__((aligned(16))) float Gs[64 * LDF];
     __shared__ __attribute__((aligned(16))) float Ts[64 * LDF];
-    __shared__ float Ysc[4 * 16 * 17];
     __shared__ float bs[64];
     const int slot = blockIdx.x, h = blockIdx.y;
     long bos;
@@ -246,7 +241,7 @@ __global__ void __launch_bounds__(NTH) fwd_prep_kernel(const T* __restrict__ k,
     load_rows<T, 64, V, NTH>(Vs, LDV, v + (bos * H + h) * V, (long)H * V, len);
     __syncthreads();
     chunk_coeffs<T, K>(Ks, LDK, beta, bos, H, h, len, bs, nullptr, nullptr, bco);
-    compute_T<T, K>(Ks, LDK, bs, Gs, Ts, Ysc);
+    compute_T<T, K>(Ks, LDK, bs, Gs, Ts);
     T* Wb = Wout + (bos * H + h) * K;
     T* Ub = Uout + (bos * H + h) * V;
     block_gemm<T, 64, K, 64, NW>(view_k((const float*)Ts, LDF), view_t((const T*)Ks, LDK, nullptr, bs),
@@ -259,11 +254,27 @@ __global__ void __launch_bounds__(NTH) fwd_prep_kernel(const T* __restrict__ k,
                                  });
 }
 
+// A thread's 16-byte piece of a 64 x 64 fp32 tile (1024 threads): rows past the
+// end read as zero.
+struct Piece64 {
+    floatx4 x;
+    __device__ __forceinline__ void load(const float* __restrict__ src, long ld, int rows) {
+        const int r = threadIdx.x >> 4, c = 4 * (threadIdx.x & 15);
+        x = r < rows ? *reinterpret_cast<const floatx4*>(src + r * ld + c)
+                     : floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    __device__ __forceinline__ void store(float* dst) const {
+        const int r = threadIdx.x >> 4, c = 4 * (threadIdx.x & 15);
+        *reinterpret_cast<floatx4*>(dst + r * LDF + c) = x;
+    }
+};
+
 // ---------------------------------------------------------------------------
 // forward: state scan.  grid (N*H, V/VS).  One workgroup carries S[:, slice]
-// (K x VS, fp32) through all chunks of its sequence in MFMA accumulators:
-// wave w owns key rows [w*K/4, (w+1)*K/4).  Per chunk it stores the chunk
-// start state (bf16/fp32; transposed [v][k] when HT, else [k][v]) and Vn.
+// (64 x 64, fp32) through all chunks of its sequence in MFMA accumulators: wave
+// w owns the 16 x 16 tile (w & 3, w >> 2).  Per chunk it stores the chunk
+// start state (transposed [v][k] when HT, else [k][v]) and Vn; the next chunk's
+// rows are loaded into registers meanwhile.
 // ---------------------------------------------------------------------------
 template <typename T, int K, int V, int VS, bool HT>
 __global__ void __launch_bounds__(NTH) fwd_state_kernel(const T* __restrict__ k,
@@ -273,92 +284,65 @@ __global__ void __launch_bounds__(NTH) fwd_state_kernel(const T* __restrict__ k,
                                                         float* __restrict__ ST,
                                                         T* __restrict__ hout,
                                                         T* __restrict__ Vnout) {
-    constexpr int P = pad<T>();
-    constexpr int LDW = K + P, LDKT = 64 + P, LDST = K + P, LDU = VS + P, LDVN = 64 + P;
-    __shared__ __attribute__((aligned(16))) T Ws[64 * LDW];
-    __shared__ __attribute__((aligned(16))) T KTs[K * LDKT];
-    __shared__ __attribute__((aligned(16))) T STs[VS * LDST];
-    __shared__ __attribute__((aligned(16))) T Us[64 * LDU];
-    __shared__ __attribute__((aligned(16))) T VnT[VS * LDVN];
-    constexpr int RT = K / 64;  // 16-row tiles per wave
-    constexpr int CT = VS / 16;
+    static_assert(__is_same(T, float) && K == 64 && VS == 64, "fp32, 64 x 64 state slices");
+    __shared__ __attribute__((aligned(16))) float Ws[64 * LDF];
+    __shared__ __attribute__((aligned(16))) float Ks[64 * LDF];
+    __shared__ __attribute__((aligned(16))) float Us[64 * LDF];
+    __shared__ __attribute__((aligned(16))) float STs[64 * LDF];  // S transposed [v][k]
+    __shared__ __attribute__((aligned(16))) float VnT[64 * LDF];  // Vn transposed [v][token]
     const int seq = blockIdx.x / H, h = blockIdx.x % H, v0 = blockIdx.y * VS;
     const int w = wave_id(), lane = lane_id();
+    const int row = 16 * (w & 3) + 4 * (lane >> 4), col = 16 * (w >> 2) + (lane & 15);
     long sbos, slen;
     int slot0;
     seq_bounds(si, seq, sbos, slen, slot0);
     const int nch = (int)((slen + BT - 1) / BT);
-    const long sbase = ((long)seq * H + h) * K * V;
-    floatx4 S[RT][CT];
+    const long sbase = ((long)seq * H + h) * K * V + (long)row * V + v0 + col;
+    floatx4 S;
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            const int row = w * (K / 4) + rt * 16 + 4 * (lane >> 4);
-            const int col = v0 + ct * 16 + (lane & 15);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                S[rt][ct][i] = S0 ? S0[sbase + (long)(row + i) * V + col] : 0.f;
-        }
+    for (int i = 0; i < 4; ++i) S[i] = S0 ? S0[sbase + (long)i * V] : 0.f;
+    Piece64 pw, pk, pu;
+    auto fetch = [&](int n) {
+        const long bos = sbos + (long)n * BT;
+        const int len = (int)min((long)BT, slen - (long)n * BT);
+        pw.load(W + (bos * H + h) * K, (long)H * K, len);
+        pk.load(k + (bos * H + h) * K, (long)H * K, len);
+        pu.load(U + (bos * H + h) * V + v0, (long)H * V, len);
+    };
+    if (nch > 0) fetch(0);
     for (int n = 0; n < nch; ++n) {
         const long bos = sbos + (long)n * BT;
         const int len = (int)min((long)BT, slen - (long)n * BT);
         const long slot = slot0 + n;
-        load_rows<T, 64, K, NTH>(Ws, LDW, W + (bos * H + h) * K, (long)H * K, len);
-        load_rows_t<T, 64, K, NTH>(KTs, LDKT, k + (bos * H + h) * K, (long)H * K, len);
-        load_rows<T, 64, VS, NTH>(Us, LDU, U + (bos * H + h) * V + v0, (long)H * V, len);
+        pw.store(Ws);
+        pk.store(Ks);
+        pu.store(Us);
+        if (n + 1 < nch) fetch(n + 1);
         T* hb = hout + (slot * H + h) * (long)K * V;
+        store_frag_t(STs, LDF, row, col, S);
+        if (HT) {
+            *reinterpret_cast<floatx4*>(hb + (long)(v0 + col) * K + row) = S;
+        } else {
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct) {
-                const int row = w * (K / 4) + rt * 16 + 4 * (lane >> 4);
-                const int col = ct * 16 + (lane & 15);
-                store_frag_t(STs, LDST, row, col, S[rt][ct]);
-                if (HT) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        hb[(long)(v0 + col) * K + row + i] = from_f<T>(S[rt][ct][i]);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        hb[(long)(row + i) * V + v0 + col] = from_f<T>(S[rt][ct][i]);
-                }
-            }
-        __syncthreads();
-        T* vnb = Vnout + (bos * H + h) * V + v0;
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-            acc = tile_mma<T, K>(acc, view_k((const T*)Ws, LDW), 16 * w,
-                                 view_k((const T*)STs, LDST), ct * 16, lane);
-            const int r = 16 * w + 4 * (lane >> 4), c = ct * 16 + (lane & 15);
-            floatx4 vn;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) vn[i] = to_f(Us[(r + i) * LDU + c]) - acc[i];
-            store_frag(vnb, (long)H * V, r, c, vn, len);
-            store_frag_t(VnT, LDVN, r, c, vn);
+            for (int i = 0; i < 4; ++i) hb[(long)(row + i) * V + v0 + col] = S[i];
         }
         __syncthreads();
+        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+        acc = tile_mma<T, K>(acc, view_k((const T*)Ws, LDF), 16 * (w & 3),
+                             view_k((const T*)STs, LDF), 16 * (w >> 2), lane);
+        floatx4 vn;
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct)
-                S[rt][ct] = tile_mma<T, 64>(S[rt][ct], view_k((const T*)KTs, LDKT),
-                                            w * (K / 4) + rt * 16, view_k((const T*)VnT, LDVN),
-                                            ct * 16, lane);
+        for (int i = 0; i < 4; ++i) vn[i] = Us[(row + i) * LDF + col] - acc[i];
+        store_frag(Vnout + (bos * H + h) * V + v0, (long)H * V, row, col, vn, len);
+        store_frag_t(VnT, LDF, row, col, vn);
+        __syncthreads();
+        S = tile_mma<T, 64>(S, view_t((const T*)Ks, LDF), 16 * (w & 3),
+                            view_k((const T*)VnT, LDF), 16 * (w >> 2), lane);
         __syncthreads();
     }
     if (ST) {
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct) {
-                const int row = w * (K / 4) + rt * 16 + 4 * (lane >> 4);
-                const int col = v0 + ct * 16 + (lane & 15);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) ST[sbase + (long)(row + i) * V + col] = S[rt][ct][i];
-            }
+        for (int i = 0; i < 4; ++i) ST[sbase + (long)i * V] = S[i];
     }
 }
 
@@ -446,8 +430,9 @@ __global__ void __launch_bounds__(NTH) bwd_dvloc_kernel(const T* __restrict__ q,
 }
 
 // ---------------------------------------------------------------------------
-// backward: reverse state scan.  grid (N*H, V/VS).  dS (K x VS) in MFMA
-// accumulators; per chunk (last to first):
+// backward: reverse state scan.  grid (N*H, V/VS).  dS (64 x 64) in MFMA
+// accumulators, tiles and prefetch as in the forward's; per chunk (last to
+// first):
 //   dh_n = dS                         (gradient of the chunk's end state)
 //   dVn  = dv_local + K dS
 //   dS  += Q^T dO - W^T dVn
@@ -458,87 +443,70 @@ __global__ void __launch_bounds__(NTH) bwd_state_kernel(
     const T* __restrict__ dO, const T* __restrict__ dVloc, SeqInfo si, int H,
     const float* __restrict__ dST, float* __restrict__ dS0, T* __restrict__ dhout,
     T* __restrict__ dVnout) {
-    constexpr int P = pad<T>();
-    constexpr int LDK = K + P, LDA = 128 + P, LDB = 128 + P, LDS = K + P, LDV = VS + P;
-    __shared__ __attribute__((aligned(16))) T Ks[64 * LDK];
-    __shared__ __attribute__((aligned(16))) T AT[K * LDA];   // [Q^T | W^T]
-    __shared__ __attribute__((aligned(16))) T BTs[VS * LDB]; // [dO ; -dVn] as [v][token]
-    __shared__ __attribute__((aligned(16))) T dSTs[VS * LDS];
-    __shared__ __attribute__((aligned(16))) T dVl[64 * LDV];
-    constexpr int RT = K / 64, CT = VS / 16;
+    static_assert(__is_same(T, float) && K == 64 && VS == 64, "fp32, 64 x 64 state slices");
+    __shared__ __attribute__((aligned(16))) float Ks[64 * LDF];
+    __shared__ __attribute__((aligned(16))) float Qs[64 * LDF];
+    __shared__ __attribute__((aligned(16))) float Ws[64 * LDF];
+    __shared__ __attribute__((aligned(16))) float dOs[64 * LDF];
+    __shared__ __attribute__((aligned(16))) float dVl[64 * LDF];
+    __shared__ __attribute__((aligned(16))) float dSTs[64 * LDF];  // dS transposed [v][k]
+    __shared__ __attribute__((aligned(16))) float nVT[64 * LDF];   // -dVn transposed [v][token]
     const int seq = blockIdx.x / H, h = blockIdx.x % H, v0 = blockIdx.y * VS;
     const int w = wave_id(), lane = lane_id();
+    const int row = 16 * (w & 3) + 4 * (lane >> 4), col = 16 * (w >> 2) + (lane & 15);
     long sbos, slen;
     int slot0;
     seq_bounds(si, seq, sbos, slen, slot0);
     const int nch = (int)((slen + BT - 1) / BT);
-    const long sbase = ((long)seq * H + h) * K * V;
-    floatx4 dS[RT][CT];
+    const long sbase = ((long)seq * H + h) * K * V + (long)row * V + v0 + col;
+    floatx4 dS;
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            const int row = w * (K / 4) + rt * 16 + 4 * (lane >> 4);
-            const int col = v0 + ct * 16 + (lane & 15);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                dS[rt][ct][i] = dST ? dST[sbase + (long)(row + i) * V + col] : 0.f;
-        }
+    for (int i = 0; i < 4; ++i) dS[i] = dST ? dST[sbase + (long)i * V] : 0.f;
+    Piece64 pk, pq, pw, po, pv;
+    auto fetch = [&](int n) {
+        const long bos = sbos + (long)n * BT;
+        const int len = (int)min((long)BT, slen - (long)n * BT);
+        pk.load(k + (bos * H + h) * K, (long)H * K, len);
+        pq.load(q + (bos * H + h) * K, (long)H * K, len);
+        pw.load(W + (bos * H + h) * K, (long)H * K, len);
+        po.load(dO + (bos * H + h) * V + v0, (long)H * V, len);
+        pv.load(dVloc + (bos * H + h) * V + v0, (long)H * V, len);
+    };
+    if (nch > 0) fetch(nch - 1);
     for (int n = nch - 1; n >= 0; --n) {
         const long bos = sbos + (long)n * BT;
         const int len = (int)min((long)BT, slen - (long)n * BT);
         const long slot = slot0 + n;
-        load_rows<T, 64, K, NTH>(Ks, LDK, k + (bos * H + h) * K, (long)H * K, len);
-        load_rows_t<T, 64, K, NTH>(AT, LDA, q + (bos * H + h) * K, (long)H * K, len);
-        load_rows_t<T, 64, K, NTH>(AT + 64, LDA, W + (bos * H + h) * K, (long)H * K, len);
-        load_rows_t<T, 64, VS, NTH>(BTs, LDB, dO + (bos * H + h) * V + v0, (long)H * V, len);
-        load_rows<T, 64, VS, NTH>(dVl, LDV, dVloc + (bos * H + h) * V + v0, (long)H * V, len);
+        pk.store(Ks);
+        pq.store(Qs);
+        pw.store(Ws);
+        po.store(dOs);
+        pv.store(dVl);
+        if (n > 0) fetch(n - 1);
         T* dhb = dhout + (slot * H + h) * (long)K * V;
+        store_frag_t(dSTs, LDF, row, col, dS);
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct) {
-                const int row = w * (K / 4) + rt * 16 + 4 * (lane >> 4);
-                const int col = ct * 16 + (lane & 15);
-                store_frag_t(dSTs, LDS, row, col, dS[rt][ct]);
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    dhb[(long)(row + i) * V + v0 + col] = from_f<T>(dS[rt][ct][i]);
-            }
+        for (int i = 0; i < 4; ++i) dhb[(long)(row + i) * V + v0 + col] = dS[i];
         __syncthreads();
-        T* dvnb = dVnout + (bos * H + h) * V + v0;
+        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+        acc = tile_mma<T, K>(acc, view_k((const T*)Ks, LDF), 16 * (w & 3),
+                             view_k((const T*)dSTs, LDF), 16 * (w >> 2), lane);
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-            acc = tile_mma<T, K>(acc, view_k((const T*)Ks, LDK), 16 * w,
-                                 view_k((const T*)dSTs, LDS), ct * 16, lane);
-            const int r = 16 * w + 4 * (lane >> 4), c = ct * 16 + (lane & 15);
+        for (int i = 0; i < 4; ++i) acc[i] += dVl[(row + i) * LDF + col];
+        store_frag(dVnout + (bos * H + h) * V + v0, (long)H * V, row, col, acc, len);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[i] += to_f(dVl[(r + i) * LDV + c]);
-            store_frag(dvnb, (long)H * V, r, c, acc, len);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) BTs[c * LDB + 64 + r + i] = from_f<T>(-acc[i]);
-        }
+        for (int i = 0; i < 4; ++i) nVT[col * LDF + row + i] = -acc[i];
+        // Q^T dO needs no dVn: before the barrier
+        dS = tile_mma<T, 64>(dS, view_t((const T*)Qs, LDF), 16 * (w & 3),
+                             view_t((const T*)dOs, LDF), 16 * (w >> 2), lane);
         __syncthreads();
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct)
-                dS[rt][ct] = tile_mma<T, 128>(dS[rt][ct], view_k((const T*)AT, LDA),
-                                              w * (K / 4) + rt * 16, view_k((const T*)BTs, LDB),
-                                              ct * 16, lane);
+        dS = tile_mma<T, 64>(dS, view_t((const T*)Ws, LDF), 16 * (w & 3),
+                             view_k((const T*)nVT, LDF), 16 * (w >> 2), lane);
         __syncthreads();
     }
     if (dS0) {
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct) {
-                const int row = w * (K / 4) + rt * 16 + 4 * (lane >> 4);
-                const int col = v0 + ct * 16 + (lane & 15);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) dS0[sbase + (long)(row + i) * V + col] = dS[rt][ct][i];
-            }
+        for (int i = 0; i < 4; ++i) dS0[sbase + (long)i * V] = dS[i];
     }
 }
 
@@ -579,13 +547,14 @@ __global__ void __launch_bounds__(NTH) bwd_dqkw_kernel(
     const int w = wave_id(), lane = lane_id();
     constexpr int TNK = K / 16;
     constexpr int TPW = 4 * TNK / NW;  // 64 x K tiles per wave
-    floatx4 aq[TPW], ak[TPW], aw[TPW], am[4];
+    constexpr int TM = 16 / NW;  // 64 x 64 tiles per wave
+    floatx4 aq[TPW], ak[TPW], aw[TPW], am[TM];
 #pragma unroll
     for (int j = 0; j < TPW; ++j)
 #pragma unroll
         for (int i = 0; i < 4; ++i) aq[j][i] = ak[j][i] = aw[j][i] = 0.f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < TM; ++j)
 #pragma unroll
         for (int i = 0; i < 4; ++i) am[j][i] = 0.f;
     const long hbase = ((long)slot * H + h) * K * V;
@@ -598,7 +567,7 @@ __global__ void __launch_bounds__(NTH) bwd_dqkw_kernel(
         load_rows<T, K, 64, NTH>(dhs, LD64, dhst + hbase + v0, V, K);
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < TM; ++j) {
             const int t = w + NW * j, tm = t / 4, tn = t % 4;
             am[j] = tile_mma<T, 64>(am[j], view_k((const T*)dOs, LD64), tm * 16,
                                     view_k((const T*)Vns, LD64), tn * 16, lane);
@@ -619,7 +588,7 @@ __global__ void __launch_bounds__(NTH) bwd_dqkw_kernel(
     for (int i = threadIdx.x; i < 2 * SZ_A; i += NTH) smem[i] = from_f<T>(0.f);
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < TM; ++j) {
         const int t = w + NW * j, tm = t / 4, tn = t % 4;
         const int r = tm * 16 + 4 * (lane >> 4), c = tn * 16 + (lane & 15);
 #pragma unroll
@@ -687,7 +656,6 @@ __global__ void __launch_bounds__(NTH) bwd_wy_kernel(
     __shared__ __attribute__((aligned(16))) float Ts[64 * LDF];
     __shared__ __attribute__((aligned(16))) float As[64 * LDF];
     __shared__ __attribute__((aligned(16))) float Xs[64 * LDF];
-    __shared__ float Ysc[4 * 16 * 17];
     __shared__ float bs[64], dcls[64], dcbs[64], dbs[64];
     const int slot = blockIdx.x, h = blockIdx.y;
     long bos;
@@ -699,12 +667,13 @@ __global__ void __launch_bounds__(NTH) bwd_wy_kernel(
     if (threadIdx.x < 64) dbs[threadIdx.x] = 0.f;
     __syncthreads();
     chunk_coeffs<T, K>(Ks, LDK, beta, bos, H, h, len, bs, dcls, dcbs, nullptr);
-    compute_T<T, K>(Ks, LDK, bs, Gs, Ts, Ysc);
+    compute_T<T, K>(Ks, LDK, bs, Gs, Ts);
 
-    // dT (all 16 tiles, 4 per wave) and dv, tile by tile over V
-    floatx4 dT[4];
+    // dT (all 16 tiles) and dv, tile by tile over V
+    constexpr int TM = 16 / NW;
+    floatx4 dT[TM];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < TM; ++j) {
         const int t = w + NW * j, tm = t / 4, tn = t % 4;
         floatx4 acc = {0.f, 0.f, 0.f, 0.f};
         dT[j] = tile_mma<T, K>(acc, view_k((const T*)dWs, LDK), tm * 16,
@@ -717,7 +686,7 @@ __global__ void __launch_bounds__(NTH) bwd_wy_kernel(
         load_rows<T, 64, 64, NTH>(dUt, LD64, dUg + (bos * H + h) * V + v0, (long)H * V, len);
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < TM; ++j) {
             const int t = w + NW * j, tm = t / 4, tn = t % 4;
             dT[j] = tile_mma<T, 64>(dT[j], view_k((const T*)dUt, LD64), tm * 16,
                                     view_k((const T*)Vt, LD64, (const float*)bs), tn * 16, lane);
@@ -737,7 +706,7 @@ __global__ void __launch_bounds__(NTH) bwd_wy_kernel(
         __syncthreads();
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < TM; ++j) {
         const int t = w + NW * j, tm = t / 4, tn = t % 4;
         const int r = tm * 16 + 4 * (lane >> 4), c = tn * 16 + (lane & 15);
 #pragma unroll
@@ -1062,14 +1031,14 @@ static int run_fwd(const Problem& p, const T* q, const T* k, const T* v, const T
         EFLA_LAUNCH("efla_q_fwd_scan", (fast::scan_o_kernel<K, V>),
                     dim3(p.N * si.nseg * H * (V / fast::VS)), dim3(fast::NTS), st, q, k, v, w.Tc,
                     w.bc, si, H, start, ST, o, w.h, w.Pc, p.ld);
-        return (int)hipPeekAtLastError();
+    } else {
+        EFLA_LAUNCH("efla_q_fwd_prep", (fwd_prep_kernel<T, K, V>), dim3(p.slots, H), dim3(NTH),
+                    st, k, v, beta, si, H, w.bco, w.W, w.U);
+        EFLA_LAUNCH("efla_q_fwd_state", (fwd_state_kernel<T, K, V, VS, true>),
+                    dim3(p.N * H, V / VS), dim3(NTH), st, k, w.W, w.U, si, H, S0, ST, w.h, w.Vn);
+        EFLA_LAUNCH("efla_q_fwd_o", (fwd_o_kernel<T, K, V, VO>), dim3(p.slots, H, V / VO),
+                    dim3(NTH), st, q, k, w.h, w.Vn, si, H, o);
     }
-    EFLA_LAUNCH("efla_q_fwd_prep", (fwd_prep_kernel<T, K, V>), dim3(p.slots, H), dim3(NTH), st,
-                k, v, beta, si, H, w.bco, w.W, w.U);
-    EFLA_LAUNCH("efla_q_fwd_state", (fwd_state_kernel<T, K, V, VS, true>),
-                dim3(p.N * H, V / VS), dim3(NTH), st, k, w.W, w.U, si, H, S0, ST, w.h, w.Vn);
-    EFLA_LAUNCH("efla_q_fwd_o", (fwd_o_kernel<T, K, V, VO>), dim3(p.slots, H, V / VO),
-                dim3(NTH), st, q, k, w.h, w.Vn, si, H, o);
     return (int)hipPeekAtLastError();
 }
 
@@ -1137,24 +1106,24 @@ static int run_bwd(const Problem& p, const T* q, const T* k, const T* v, const T
                         (const float*)w.bc, (const float*)w.dcc, (const bf16*)nullptr, w.h, w.dh,
                         si, H, nitems, dq, dk, dv, dbeta, p.ld);
         }
-        return (int)hipPeekAtLastError();
-    } else if (!reuse) {
-        EFLA_LAUNCH("efla_q_bwd_re_prep", (fwd_prep_kernel<T, K, V>), dim3(p.slots, H),
-                    dim3(NTH), st, k, v, beta, si, H, w.bco, w.W, w.U);
+    } else {
+        if (!reuse)
+            EFLA_LAUNCH("efla_q_bwd_re_prep", (fwd_prep_kernel<T, K, V>), dim3(p.slots, H),
+                        dim3(NTH), st, k, v, beta, si, H, w.bco, w.W, w.U);
+        // the generic forward keeps its states transposed for its output kernel,
+        // so this path recomputes them whatever reuse_states says
+        EFLA_LAUNCH("efla_q_bwd_re_state", (fwd_state_kernel<T, K, V, VS, false>),
+                    dim3(p.N * H, V / VS), dim3(NTH), st, k, w.W, w.U, si, H, S0,
+                    (float*)nullptr, w.h, w.Vn);
+        EFLA_LAUNCH("efla_q_bwd_dvloc", (bwd_dvloc_kernel<T, K, V, VO>),
+                    dim3(p.slots, H, V / VO), dim3(NTH), st, q, k, dO, si, H, w.dvloc);
+        EFLA_LAUNCH("efla_q_bwd_state", (bwd_state_kernel<T, K, V, VS>), dim3(p.N * H, V / VS),
+                    dim3(NTH), st, q, k, w.W, dO, w.dvloc, si, H, dST, dS0, w.dh, w.dVn);
+        EFLA_LAUNCH("efla_q_bwd_dqkw", (bwd_dqkw_kernel<T, K, V>), dim3(p.slots, H), dim3(NTH),
+                    st, q, k, dO, w.Vn, w.dVn, w.h, w.dh, si, H, dq, w.dKp, w.dW);
+        EFLA_LAUNCH("efla_q_bwd_wy", (bwd_wy_kernel<T, K, V>), dim3(p.slots, H), dim3(NTH), st, k,
+                    v, beta, w.dW, w.dVn, w.dKp, si, H, dk, dv, dbeta);
     }
-    // the generic forward keeps its states transposed for its output kernel,
-    // so this path recomputes them whatever reuse_states says
-    EFLA_LAUNCH("efla_q_bwd_re_state", (fwd_state_kernel<T, K, V, VS, false>),
-                dim3(p.N * H, V / VS), dim3(NTH), st, k, w.W, w.U, si, H, S0, (float*)nullptr,
-                w.h, w.Vn);
-    EFLA_LAUNCH("efla_q_bwd_dvloc", (bwd_dvloc_kernel<T, K, V, VO>), dim3(p.slots, H, V / VO),
-                dim3(NTH), st, q, k, dO, si, H, w.dvloc);
-    EFLA_LAUNCH("efla_q_bwd_state", (bwd_state_kernel<T, K, V, VS>), dim3(p.N * H, V / VS),
-                dim3(NTH), st, q, k, w.W, dO, w.dvloc, si, H, dST, dS0, w.dh, w.dVn);
-    EFLA_LAUNCH("efla_q_bwd_dqkw", (bwd_dqkw_kernel<T, K, V>), dim3(p.slots, H), dim3(NTH), st,
-                q, k, dO, w.Vn, w.dVn, w.h, w.dh, si, H, dq, w.dKp, w.dW);
-    EFLA_LAUNCH("efla_q_bwd_wy", (bwd_wy_kernel<T, K, V>), dim3(p.slots, H), dim3(NTH), st, k,
-                v, beta, w.dW, w.dVn, w.dKp, si, H, dk, dv, dbeta);
     return (int)hipPeekAtLastError();
 }
 

@@ -59,6 +59,12 @@ def test_fp32_ragged_with_states(oracle):
     _case(oracle, 11, 2, 200, 3, 64, 64, torch.float32, s0=True, dst=True)
 
 
+# around the edges of a 16-token tile of the fp32 kernels and of a chunk
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 48, 63, 64, 65, 129])
+def test_fp32_short_sequences(oracle, T):
+    _case(oracle, 300 + T, 2, T, 3, 64, 64, torch.float32, s0=True, dst=True)
+
+
 @pytest.mark.parametrize("K,V", [(64, 64), (128, 128), (128, 256), (64, 128), (128, 64),
                                  (64, 256)])
 def test_bf16_shapes(oracle, K, V):

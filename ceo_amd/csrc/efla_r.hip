@@ -357,8 +357,9 @@ struct RFastSmem {
 };
 
 // SG: tokens staged per segment (chunk_size's tuning hint; the results do not
-// depend on it)
-template <int D, int NS, int LPC, int SG>
+// depend on it).  GR: token groups (gr.n > 1); a form of its own, since the
+// shortest calls feel the few instructions more.
+template <int D, int NS, int LPC, int SG, bool GR>
 __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_fast_kernel(
     const bf16* __restrict__ k, const bf16* __restrict__ v, const float* __restrict__ coef,
     bf16* __restrict__ state, bf16* __restrict__ out, float* __restrict__ part_out,
@@ -372,12 +373,12 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_fast_kernel(
     __shared__ __attribute__((aligned(16))) RFastSmem<D, NS, SG> sm;
     const int tid = threadIdx.x, w = mf::wave(), l = mf::lane();
     const int item = blockIdx.x / NS, cb = blockIdx.x % NS;
-    const int grp = item / gr.nbh, bh = item - grp * gr.nbh;
+    const int grp = GR ? item / gr.nbh : 0, bh = item - grp * gr.nbh;
     const int col = cb * NC + tid / LPC, lcol = tid / LPC, part = tid % LPC, r0 = part * RPL;
     const int b = bh / H, h = bh % H;
     // this workgroup's tokens: tb .. T - 1
-    const long tb = (long)grp * gr.segs * SEGF;
-    const long T = tb + (long)gr.segs * SEGF < Tall ? tb + (long)gr.segs * SEGF : Tall;
+    const long tb = GR ? (long)grp * gr.segs * SEGF : 0;
+    const long T = GR && tb + (long)gr.segs * SEGF < Tall ? tb + (long)gr.segs * SEGF : Tall;
     const long dd = (long)D * D, nsegf = (T - tb + SG - 1) / SG;
     const long tstride = (long)H * D;  // elements between tokens
     const long base0 = (long)b * Tall * tstride + (long)h * D;
@@ -385,7 +386,7 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_fast_kernel(
     bf16* st = state + (long)bh * dd;
 
     bf16x2 Sp[NP];  // rows r0 + 2p (low half) and r0 + 2p + 1 (high half)
-    if (gr.n > 1) {  // the group's start state from the chain pass
+    if constexpr (GR) {  // the group's start state from the chain pass
         const bf16* cp = gr.ck + ((long)bh * gr.n + grp) * dd + (long)col * D + r0;
 #pragma unroll
         for (int p = 0; p < NP; ++p) Sp[p] = bf16x2{cp[2 * p], cp[2 * p + 1]};
@@ -517,7 +518,7 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_fast_kernel(
         }
     }
     if (pp >= 0) o_products();
-    if (gr.n > 1) return;  // the chain pass has written the final state
+    if constexpr (GR) return;  // the chain pass has written the final state
     // the final state back to the caller
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
@@ -669,6 +670,7 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_chain_kernel(
                     bf16x8{S[4 * q][0], S[4 * q][1], S[4 * q + 1][0], S[4 * q + 1][1],
                            S[4 * q + 2][0], S[4 * q + 2][1], S[4 * q + 3][0], S[4 * q + 3][1]};
         }
+        if (!state_out && seg + 1 == nsegf) break;  // no start state is left to form
         struct Ops {
             mf::int4v kq[NP / 4];
             mf::floatx4 cq[RPL / 4];
@@ -761,7 +763,7 @@ struct RBwdSmem {
     float gks[NS > 1 ? 2 : 1][NS > 1 ? SEGF : 1][NS > 1 ? D : 1];
 };
 
-template <int D, int NS, int LPC>
+template <int D, int NS, int LPC, bool GR>
 __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_bwd_fast_kernel(
     const bf16* __restrict__ dO, const bf16* __restrict__ k, const bf16* __restrict__ v,
     const float* __restrict__ coef, const float* __restrict__ dcoef, const bf16* __restrict__ ck,
@@ -778,13 +780,14 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_bwd_fast_kern
     __shared__ __attribute__((aligned(16))) RBwdSmem<D, NS> sm;
     const int tid = threadIdx.x, w = mf::wave(), l = mf::lane();
     const int item = blockIdx.x / NS, cb = blockIdx.x % NS;
-    const int grp = item / gr.nbh, bh = item - grp * gr.nbh;
+    const int grp = GR ? item / gr.nbh : 0, bh = item - grp * gr.nbh;
     const int col = cb * NC + tid / LPC, lcol = tid / LPC, part = tid % LPC, r0 = part * RPL;
     const int g4 = l >> 4, j16 = l & 15;
     const int b = bh / H, h = bh % H;
     const long dd = (long)D * D, nsegf = (T + SEGF - 1) / SEGF;
     // this workgroup's segments: s_lo .. s_hi - 1
-    const long s_lo = (long)grp * gr.segs, s_hi = s_lo + gr.segs < nsegf ? s_lo + gr.segs : nsegf;
+    const long s_lo = GR ? (long)grp * gr.segs : 0;
+    const long s_hi = GR && s_lo + gr.segs < nsegf ? s_lo + gr.segs : nsegf;
     const long tstride = (long)H * D;
     const long base0 = (long)b * T * tstride + (long)h * D;
     const float* cbh = coef + (long)bh * T;
@@ -811,7 +814,7 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_bwd_fast_kern
     float G[RPL];
 #pragma unroll
     for (int i = 0; i < RPL; ++i) G[i] = 0.f;
-    if (s_hi < nsegf) {  // dL/dS after the group, from the chain pass
+    if (GR && s_hi < nsegf) {  // dL/dS after the group, from the chain pass
         const float* gp = gr.gck + ((long)bh * gr.n + grp) * dd + (long)col * D + r0;
 #pragma unroll
         for (int i = 0; i < RPL; ++i) G[i] = gp[i];
@@ -1027,7 +1030,7 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_bwd_fast_kern
             }
         }
     }
-    if (s_lo > 0) return;
+    if (GR && s_lo > 0) return;
     // dL/dS_0 in the reference's [row][c] layout
     bf16* gs = grad_state + (long)bh * dd;
 #pragma unroll
@@ -1064,18 +1067,15 @@ template <int D, int NS, int LPC>
 void r_launch_fwd(int sg, const void* k, const void* v, const float* coef, void* state, void* out,
                   float* part, int H, long T, const RGroups& gr, hipStream_t stream) {
     const dim3 grid((unsigned)((size_t)gr.nbh * gr.n * NS)), block(rfast_threads<D, NS, LPC>());
-    if (sg == 16)
-        EFLA_LAUNCH("efla_r_forward", (r_fast_kernel<D, NS, LPC, 16>), grid, block, stream,
-                    (const bf16*)k, (const bf16*)v, coef, (bf16*)state, (bf16*)out, part,
-                    H, T, gr);
+#define R_FWD(SG, GR)                                                                          \
+    EFLA_LAUNCH("efla_r_forward", (r_fast_kernel<D, NS, LPC, SG, GR>), grid, block, stream,    \
+                (const bf16*)k, (const bf16*)v, coef, (bf16*)state, (bf16*)out, part, H, T, gr)
+    if (gr.n > 1) R_FWD(((NS > 1 || D <= 64) ? 64 : 32), true);
+    else if (sg == 16) R_FWD(16, false);
     else if (sg == 64 && (NS > 1 || D <= 64))  // the LDS of the other shapes holds 32 at most
-        EFLA_LAUNCH("efla_r_forward", (r_fast_kernel<D, NS, LPC, (NS > 1 || D <= 64) ? 64 : 32>),
-                    grid, block, stream, (const bf16*)k, (const bf16*)v, coef, (bf16*)state,
-                    (bf16*)out, part, H, T, gr);
-    else
-        EFLA_LAUNCH("efla_r_forward", (r_fast_kernel<D, NS, LPC, 32>), grid, block, stream,
-                    (const bf16*)k, (const bf16*)v, coef, (bf16*)state, (bf16*)out, part,
-                    H, T, gr);
+        R_FWD(((NS > 1 || D <= 64) ? 64 : 32), false);
+    else R_FWD(32, false);
+#undef R_FWD
 }
 
 template <int D, int NS, int LPC>
@@ -1083,10 +1083,15 @@ void r_launch_bwd(const void* dO, const void* k, const void* v, const float* coe
                   const float* dcoef, const bf16* ck, bf16* hist, void* grad_k, float* part,
                   void* grad_v, void* grad_state, int H, long T, const RGroups& gr,
                   hipStream_t stream) {
-    EFLA_LAUNCH("efla_r_backward", (r_bwd_fast_kernel<D, NS, LPC>),
-                dim3((unsigned)((size_t)gr.nbh * gr.n * NS)), dim3(rfast_threads<D, NS, LPC>()),
-                stream, (const bf16*)dO, (const bf16*)k, (const bf16*)v, coef, dcoef, ck, hist,
-                (bf16*)grad_k, part, (bf16*)grad_v, (bf16*)grad_state, H, T, gr);
+    const dim3 grid((unsigned)((size_t)gr.nbh * gr.n * NS)), block(rfast_threads<D, NS, LPC>());
+    if (gr.n > 1)
+        EFLA_LAUNCH("efla_r_backward", (r_bwd_fast_kernel<D, NS, LPC, true>), grid, block, stream,
+                    (const bf16*)dO, (const bf16*)k, (const bf16*)v, coef, dcoef, ck, hist,
+                    (bf16*)grad_k, part, (bf16*)grad_v, (bf16*)grad_state, H, T, gr);
+    else
+        EFLA_LAUNCH("efla_r_backward", (r_bwd_fast_kernel<D, NS, LPC, false>), grid, block, stream,
+                    (const bf16*)dO, (const bf16*)k, (const bf16*)v, coef, dcoef, ck, hist,
+                    (bf16*)grad_k, part, (bf16*)grad_v, (bf16*)grad_state, H, T, gr);
 }
 
 // the chain pass: forward states to ck every `every` segments, and with gck

@@ -132,7 +132,7 @@ __device__ __forceinline__ void copy_tile(const Opnd& op, int line0, long k0, ch
             const int gl = min(line, op.nlines - 1 - line0);
             off = (unsigned)(gl * op.ld + 8 * c) * 2u;
         } else {
-            const int kr = P / CR, c = (P % CR) ^ ((kr & 3) << 2);
+            const int kr = (int)((unsigned)P / CR), c = (int)((unsigned)P % CR) ^ ((kr & 3) << 2);
             const int gc = min(8 * c, op.nlines - 8 - line0);  // nlines % 8 == 0
             off = (unsigned)(kr * op.ld + gc) * 2u;
         }
@@ -159,7 +159,7 @@ __device__ __forceinline__ void copy_tile_tail(const Opnd& op, int line0, long k
                 x = *reinterpret_cast<const bf16x8*>(op.base + ((long)gl * op.ld + k0 + 8 * c) * 2);
             dst = kc_off(line, c);
         } else {
-            const int kr = P / CR, c = P % CR;
+            const int kr = (int)((unsigned)P / CR), c = (int)((unsigned)P % CR);
             const int gc = min(line0 + 8 * c, op.nlines - 8);
             if (k0 + kr < K)
                 x = *reinterpret_cast<const bf16x8*>(op.base + ((k0 + kr) * op.ld + gc) * 2);
@@ -408,9 +408,8 @@ struct Item {
 };
 
 template <typename T, bool AKC, bool BKC, int EPI, int TS, bool RAGGED>
-__global__ void __launch_bounds__(64 * tile_waves<TS>(), 2) gemm_fast_kernel(Opnd A, Opnd B, long M, long N,
-                                                            long K, EpiArgs<T> ea, int ksplit,
-                                                            long kper) {
+__global__ void __launch_bounds__(64 * tile_waves<TS>(), TS == 128 ? 2 : 1)
+gemm_fast_kernel(Opnd A, Opnd B, long M, long N, long K, EpiArgs<T> ea, int ksplit, long kper) {
     constexpr int BM = TS, BN = TS, TILE_BYTES = tile_bytes<TS>();
     constexpr int TNI = 2, TMJ = TS / 64;  // 32 x 32 tiles per wave along n and m
     // two buffers of [A tile | B tile]; the epilogue stages the output through

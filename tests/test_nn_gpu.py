@@ -579,7 +579,7 @@ def test_gemm_gelu_config4_mlp():
 # odd contractions, strides and alignments on the large-tile kernel: operands
 # read in place (dB of an odd row count), padded copies, outputs whose rows end
 # in a partial 8-element piece or start off a 16-byte boundary, with and
-# without split-K.  Bound: the product is rounded once to bf16 (2^-9 at most,
+# without split-K.  Bound: the product is rounded once to bf16 (2^-8 at most,
 # relative) after an fp32 sum, the residual forms round nothing else.
 _ODD = [(333, 519, 1031), (900, 64, 2316), (257, 2316, 264), (1250, 1000, 24), (65, 4097, 320)]
 

@@ -155,14 +155,16 @@ def gemm_ex(a, b, out, bias=None, c=None, alpha: float = 1.0, beta: float = 0.0,
     rows are contiguous (views of column blocks allowed); ``c`` may be ``out``
     itself.  Writes into ``out`` and returns it."""
     m, n = out.shape
-    k = a.shape[0] if trans_a else a.shape[1]
-    if (a.shape[1] if trans_a else a.shape[0]) != m:
+    ra, ca = a.shape[:2]
+    rb, cb = b.shape[:2]
+    k = ra if trans_a else ca
+    if (ca if trans_a else ra) != m:
         raise ValueError("gemm_ex: op(a) rows differ from out rows")
-    if (b.shape[1] if trans_b else b.shape[0]) != k or \
-            (b.shape[0] if trans_b else b.shape[1]) != n:
+    if (cb if trans_b else rb) != k or (rb if trans_b else cb) != n:
         raise ValueError("gemm_ex: op(b) must be k x n")
+    dt = out.dtype
     for t, nme in ((a, "a"), (b, "b"), (out, "out")):
-        if not t.is_cuda or t.dtype != out.dtype:
+        if not t.is_cuda or t.dtype != dt:
             raise ValueError(f"{nme} must be a device tensor of out's dtype")
     if bias is not None:
         _require(bias, "bias", out.dtype, out.device)

@@ -15,10 +15,15 @@
 // holding 4 consecutive n of one output row m and writes 8-byte row pieces.
 // Per k-iteration each operand tile (TS lines x 64 k) is copied
 // straight from global memory into LDS (global_load_lds_dwordx4, 16 bytes per
-// lane, no VGPR staging) one iteration ahead, double-buffered; all of an
-// iteration's copies are issued at its start, and the MFMA operand fragments
-// are double-buffered in registers with the LDS reads of k step ks + 1
-// interleaved between the MFMAs of k step ks.  Both LDS
+// lane, no VGPR staging) one iteration ahead, double-buffered, and the MFMA
+// operand fragments are double-buffered in registers with the LDS reads of k
+// step ks + 1 interleaved between the MFMAs of k step ks.  The wait for the
+// next block stands before the iteration's last k step: that step's operands
+// are in registers, so its MFMAs cover the next block's first fragment reads
+// and the issue of the block after (with the wait at the iteration's end both
+// waves of a SIMD sat out those reads: 16384 x 4096 x 1024 121 -> 117 us, the
+// 16384 x 1024 x 32000 product's gradients 990 and 1026 -> 945 and 979).
+// Both LDS
 // layouts are XOR-swizzled in 16-byte chunks so the fragment reads are free
 // of bank conflicts:
 //   KC tile [line][k]  (128 B rows):  chunk c of line L at c ^ ((L >> 1) & 7)
@@ -395,9 +400,10 @@ __device__ __forceinline__ void epilogue_wave(const EpiArgs<T>& ea, const floatx
 //
 // Persistent: workgroup b takes work items b, b + gridDim.x, ... (an item is
 // an output tile, or a (tile, k-split) pair with ksplit > 1).  The LDS double
-// buffer runs across items: the last k-iteration of an item copies the next
-// item's first k-block, so an item starts with its first block in place and
-// the previous item's epilogue stores drain behind the next main loop.
+// buffer runs across items: the next item's first k-block is copied during an
+// item's last k-iteration, so an item starts with its first block in place and
+// the previous item's epilogue stores drain behind the next main loop; the
+// other buffer stages the epilogue before it takes the second block.
 //
 // ksplit > 1 (EPI_PARTIAL): the contraction is cut into ksplit ranges of
 // kper (a multiple of 64) and item (tile, split) writes its fp32 partial tile
@@ -424,20 +430,21 @@ gemm_fast_kernel(Opnd A, Opnd B, long M, long N, long K, EpiArgs<T> ea, int kspl
     auto decode = [&](long it, Item& I) {
         long id = it;
         if (nitems % 8 == 0) id = (id % 8) * (nitems / 8) + id / 8;
-        I.split = (int)(id % ksplit);
+        I.split = __builtin_amdgcn_readfirstlane((int)(id % ksplit));
         const long pid = id / ksplit;
         constexpr long GROUP = 8;
         const long group_span = GROUP * tn_n;
         const long gi = pid / group_span;
         const long first_m = gi * GROUP;
         const long gsize = (tm_n - first_m) < GROUP ? (tm_n - first_m) : GROUP;
-        I.m0 = (int)((first_m + (pid % group_span) % gsize) * BM);
-        I.n0 = (int)(((pid % group_span) / gsize) * BN);
+        // (divisions run on the vector unit: back to scalar registers)
+        I.m0 = __builtin_amdgcn_readfirstlane((int)((first_m + (pid % group_span) % gsize) * BM));
+        I.n0 = __builtin_amdgcn_readfirstlane((int)(((pid % group_span) / gsize) * BN));
         I.kbeg = (long)I.split * kper;
         I.klen = (K - I.kbeg) < kper ? (K - I.kbeg) : kper;
     };
 
-    const int w = mf::wave(), l = mf::lane();
+    const int w = mf::wave();
     const int wm = (w & 1) * (TS / 2), wn = (w >> 1) * (32 * TNI);  // this wave's block
     // buffer b: A at smem + 2b * TILE_BYTES, B right after it
     auto As = [&](int b) { return smem + 2 * b * TILE_BYTES; };
@@ -445,24 +452,41 @@ gemm_fast_kernel(Opnd A, Opnd B, long M, long N, long K, EpiArgs<T> ea, int kspl
 
     long it = blockIdx.x;
     if (it >= nitems) return;  // uniform over the workgroup
-    Item cur;
-    decode(it, cur);
-    // the first item's first k-block
-    if (cur.klen >= BK) {
-        copy_tile<AKC, TS>(A, cur.m0, cur.kbeg, As(0), w, l);
-        copy_tile<BKC, TS>(B, cur.n0, cur.kbeg, Bs(0), w, l);
-    } else {
-        copy_tile_tail<AKC, TS>(A, cur.m0, cur.kbeg, K, As(0), threadIdx.x);
-        copy_tile_tail<BKC, TS>(B, cur.n0, cur.kbeg, K, Bs(0), threadIdx.x);
-    }
+    // the next k-block to copy: block fkt of item fi, through this workgroup's
+    // items in order; whole blocks by direct copies, a k-tail through registers
+    long fit = it, fkt = 0;
+    bool fmore = true;
+    Item fi;
+    decode(fit, fi);
+    auto fetch = [&](int b, int l) {
+        if (!fmore) return;
+        const long k0 = fi.kbeg + fkt * BK;
+        if (fi.klen - fkt * BK >= BK) {
+            copy_tile<AKC, TS>(A, fi.m0, k0, As(b), w, l);
+            copy_tile<BKC, TS>(B, fi.n0, k0, Bs(b), w, l);
+        } else {
+            copy_tile_tail<AKC, TS>(A, fi.m0, k0, K, As(b), 64 * w + l);
+            copy_tile_tail<BKC, TS>(B, fi.n0, k0, K, Bs(b), 64 * w + l);
+        }
+        if (++fkt * BK >= fi.klen) {
+            fkt = 0;
+            fit += gridDim.x;
+            fmore = fit < nitems;
+            if (fmore) decode(fit, fi);
+        }
+    };
+    Item cur = fi;
+    fetch(0, mf::lane());
     mf::dma_wait();
     __syncthreads();
     int buf = 0;
     for (;;) {
-        const long nitn = it + gridDim.x;
-        const bool more = nitn < nitems;
-        Item nxt = cur;
-        if (more) decode(nitn, nxt);
+        // Buffer `buf` holds the item's first k-block, the other one is free.
+        // The lane index is re-derived per item (mf::tid_in), for the main
+        // loop and again for the epilogue: the addresses each forms from it
+        // then do not stay live across the other.
+        const int l = mf::tid_in((int)it) & 63;
+        fetch(buf ^ 1, l);  // the item's second block or the next item's first
         floatx16 acc[TNI][TMJ];  // [n tile][m tile]
 #pragma unroll
         for (int i = 0; i < TNI; ++i)
@@ -470,101 +494,84 @@ gemm_fast_kernel(Opnd A, Opnd B, long M, long N, long K, EpiArgs<T> ea, int kspl
             for (int j = 0; j < TMJ; ++j)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-        const long nfull = cur.klen / BK;  // whole k-iterations (direct copies)
         const long niter = (cur.klen + BK - 1) / BK;
         // on an edge tile a wave whose rows are all past M, or columns all
         // past N, holds no output: it only copies (the N = 3088 projection's
         // last tile column is 16 wide and 6 of its 8 waves sit idle)
         const bool act = cur.m0 + wm < M && cur.n0 + wn < N;
-        for (long kt = 0; kt < niter; ++kt) {
-            // what the other buffer receives: this item's next k-block, or
-            // the next item's first; whole blocks by direct copies, a k-tail
-            // block through registers
-            const bool own = kt + 1 < niter;
-            const bool fetch = own || more;
-            const Item& src = own ? cur : nxt;
-            const long k0 = own ? cur.kbeg + (kt + 1) * BK : nxt.kbeg;
-            const bool direct = own ? kt + 1 < nfull : nxt.klen >= BK;
-            if (fetch && !direct) {
-                copy_tile_tail<AKC, TS>(A, src.m0, k0, K, As(buf ^ 1), threadIdx.x);
-                copy_tile_tail<BKC, TS>(B, src.n0, k0, K, Bs(buf ^ 1), threadIdx.x);
+        // fragments double-buffered in registers: k step ks + 1 is read while
+        // the MFMAs of k step ks run, across the iterations too
+        constexpr int KS = BK / 16;
+        bf16x8 fb[2][TNI], fa[2][TMJ];
+        auto read = [&](int c, int b, int ks) {
+#pragma unroll
+            for (int i = 0; i < TNI; ++i) fb[c][i] = frag<BKC, TS>(Bs(b), wn + 32 * i, ks, l);
+#pragma unroll
+            for (int j = 0; j < TMJ; ++j) fa[c][j] = frag<AKC, TS>(As(b), wm + 32 * j, ks, l);
+        };
+        auto mma_step = [&](int c) {
+#pragma unroll
+            for (int i = 0; i < TNI; ++i)
+#pragma unroll
+                for (int j = 0; j < TMJ; ++j)
+                    acc[i][j] = mma32<T>(fb[c][i], fa[c][j], acc[i][j]);
+            // one LDS read between consecutive MFMAs
+            constexpr int NR = TNI * (BKC ? 1 : 2) + TMJ * (AKC ? 1 : 2);
+            constexpr int NM = TMJ * TNI;
+            constexpr int R = NR < NM ? NR : NM;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
             }
-            const char* at = As(buf);
-            const char* bt = Bs(buf);
-            // fragments double-buffered in registers: k step ks + 1 is read
-            // while the MFMAs of k step ks run
-            bf16x8 fb[2][TNI], fa[2][TMJ];
+            if constexpr (NM > R) __builtin_amdgcn_sched_group_barrier(0x008, NM - R, 0);
+            if constexpr (NR > R) __builtin_amdgcn_sched_group_barrier(0x100, NR - R, 0);
+        };
+        if (act) read(0, buf, 0);
+        for (long kt = 0; kt < niter; ++kt) {
             // the iteration's reads, copies and MFMAs issue at raised wave
             // priority, the wait for the next block at the normal one: a wave
             // still computing wins the SIMD's issue slots over its partner
-            // that has reached the end of the iteration (-1 to -4 % on the
-            // config-4 products, measured)
+            // that has reached the wait (-1 to -4 % on products of 16384 rows,
+            // measured)
             __builtin_amdgcn_s_setprio(1);
             if (act) {
 #pragma unroll
-                for (int i = 0; i < TNI; ++i) fb[0][i] = frag<BKC, TS>(bt, wn + 32 * i, 0, l);
-#pragma unroll
-                for (int j = 0; j < TMJ; ++j) fa[0][j] = frag<AKC, TS>(at, wm + 32 * j, 0, l);
-            }
-            // the next block's copies all go out now, a whole iteration ahead
-            // of the wait (the buffer they fill was last read in the previous
-            // iteration, which every wave has finished)
-            if (fetch && direct) {
-                copy_tile<AKC, TS>(A, src.m0, k0, As(buf ^ 1), w, l);
-                copy_tile<BKC, TS>(B, src.n0, k0, Bs(buf ^ 1), w, l);
-            }
-            if (act) {
-#pragma unroll
-                for (int ks = 0; ks < BK / 16; ++ks) {
-                    const int c = ks & 1;
-                    if (ks + 1 < BK / 16) {
-#pragma unroll
-                        for (int i = 0; i < TNI; ++i)
-                            fb[c ^ 1][i] = frag<BKC, TS>(bt, wn + 32 * i, ks + 1, l);
-#pragma unroll
-                        for (int j = 0; j < TMJ; ++j)
-                            fa[c ^ 1][j] = frag<AKC, TS>(at, wm + 32 * j, ks + 1, l);
-                    }
-#pragma unroll
-                    for (int i = 0; i < TNI; ++i)
-#pragma unroll
-                        for (int j = 0; j < TMJ; ++j)
-                            acc[i][j] = mma32<T>(fb[c][i], fa[c][j], acc[i][j]);
-                    if (ks + 1 < BK / 16) {
-                        // one LDS read between consecutive MFMAs
-                        constexpr int NR = TNI * (BKC ? 1 : 2) + TMJ * (AKC ? 1 : 2);
-                        constexpr int NM = TMJ * TNI;
-                        constexpr int R = NR < NM ? NR : NM;
-#pragma unroll
-                        for (int r = 0; r < R; ++r) {
-                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-                            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
-                        }
-                        if constexpr (NM > R) __builtin_amdgcn_sched_group_barrier(0x008, NM - R, 0);
-                        if constexpr (NR > R) __builtin_amdgcn_sched_group_barrier(0x100, NR - R, 0);
-                    }
+                for (int ks = 0; ks + 1 < KS; ++ks) {
+                    read((ks + 1) & 1, buf, ks + 1);
+                    mma_step(ks & 1);
                 }
             }
+            // the wait for the next block stands before the last k step: its
+            // operands are in registers, so the matrix cores go on right after
+            // the barrier while the next block's first fragments arrive
             __builtin_amdgcn_s_setprio(0);
             mf::dma_wait();
             __syncthreads();
+            __builtin_amdgcn_s_setprio(1);
+            // every wave has read buffer `buf`: it takes the block after the
+            // next, a whole iteration ahead of its wait (after an item's last
+            // iteration the epilogue stages through it first)
+            if (kt + 1 < niter) fetch(buf, l);
+            if (act) {
+                read(KS & 1, buf ^ 1, 0);  // after the last iteration: not used
+                mma_step((KS - 1) & 1);
+            }
             buf ^= 1;
         }
+        __builtin_amdgcn_s_setprio(0);
         // lane l holds, for tile (i, j), output row m = m0 + wm + 32 j + (l & 31)
         // and columns n = n0 + wn + 32 i + 8 q + 4 (l >> 5) + e in acc[i][j][4 q + e].
-        // The lane index is re-derived per item (mf::tid_in): the epilogue's
-        // lane-dependent addresses are then not hoisted out of the item loop,
-        // where they would stay live across the main loop.
         {
-            const int le = mf::tid_in((int)it) & 63;
+            const int le = mf::tid_in(~(int)it) & 63;
             char* wp = smem + 2 * (buf ^ 1) * TILE_BYTES + (4096 * TNI) * w;
             epilogue_wave<T, EPI, TNI, TMJ, AKC && BKC, RAGGED>(ea, acc, cur.split, (long)cur.m0 + wm,
                                                     (long)cur.n0 + wn, M, N, le, wp);
         }
-        __syncthreads();  // the next item's first copies refill the buffer
-        if (!more) break;
-        it = nitn;
-        cur = nxt;
+        it += gridDim.x;
+        if (it >= nitems) break;
+        __syncthreads();  // the staged output is read: the buffer takes its block
+        decode(it, cur);
     }
 }
 

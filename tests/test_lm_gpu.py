@@ -98,3 +98,51 @@ def test_cross_entropy_uniform_logits():
     loss = cross_entropy_forward(torch.zeros(B, V, dtype=torch.bfloat16, device="cuda"),
                                  torch.arange(B, dtype=torch.int32, device="cuda"), 0.3)
     assert abs(loss.sum().item() - np.log(V)) < 1e-5
+
+
+# Masked and extreme logits in the row-in-registers path: every kind of piece
+# count, threads whose whole part is masked (-inf) or holds bf16's lowest
+# value, a target at a piece's first and last element, a row with one finite
+# logit.  Loss: fp32 sums of V terms, 1e-5 as above; the gradient is rounded
+# to bf16 (2^-8) after fp32 exponentials of differences up to 60 (60 2^-22).
+@pytest.mark.parametrize("V", [8, 1000, 8192, 8200, 32000, 65536])
+def test_cross_entropy_masked_and_extreme(V):
+    from ceo_amd.nn import cross_entropy_forward, cross_entropy_forward_backward
+
+    announce(f"cross_entropy masked V={V}")
+    g = torch.Generator().manual_seed(V)
+    z = (torch.randn(6, V, generator=g) * 6).to(torch.bfloat16)
+    t = torch.tensor([0, V - 1, 7, V // 2, 3, 5], dtype=torch.int32)
+    z[0, V // 2:] = float("-inf")
+    z[1, :V - 8] = float("-inf")
+    z[2, 1::2] = torch.finfo(torch.bfloat16).min
+    z[3] = float("-inf")
+    z[3, V // 2] = 2.0
+    z[4, :] = -3.0
+    loss, grad = cross_entropy_forward_backward(z.cuda(), t.cuda())
+    assert torch.equal(loss, cross_entropy_forward(z.cuda(), t.cuda()))
+    torch.cuda.synchronize()
+    lp = torch.log_softmax(z.double(), -1)
+    ref = -lp.gather(1, t.long()[:, None])[:, 0] / 6
+    rg = lp.exp()
+    rg[torch.arange(6), t.long()] -= 1
+    loss, grad = loss.cpu().double(), grad.cpu().double() * 6
+    # lp[t] near 0 is the difference of two numbers of about 20
+    both = torch.isfinite(ref)
+    assert torch.equal(torch.isinf(loss), ~both)
+    err = ((loss - ref).abs() / ref.abs().clamp(min=1))[both].max().item()
+    eg = ((grad - rg).abs() - (2.0 ** -8 + 60 * 2.0 ** -22) * rg.abs()).max().item()
+    print(f"  loss {err:.2e} grad beyond the bound {eg:.2e}", flush=True)
+    assert err <= 1e-5 and eg <= 1e-5  # p_t - 1: fp32's 2^-22 of 1
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_cross_entropy_row_with_inf_or_nan(bad):
+    from ceo_amd.nn import cross_entropy_forward_backward
+
+    z = torch.zeros(3, 1000, dtype=torch.bfloat16)
+    z[1, 500] = bad
+    t = torch.tensor([1, 1, 1], dtype=torch.int32)
+    loss, grad = cross_entropy_forward_backward(z.cuda(), t.cuda())
+    assert loss.isnan().tolist() == [False, True, False]
+    assert grad.isnan().all(1).tolist() == [False, True, False] and not grad[0].isnan().any()

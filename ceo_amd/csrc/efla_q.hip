@@ -988,7 +988,7 @@ static void seg_forward(const Problem& p, const SeqInfo& si, const bf16* k, cons
                 dim3(p.N * (p.nseg - 1) * p.H * ((V + K) / fast::VS)), dim3(fast::NT), st, k, v,
                 Tc, bc, si, p.H, S0, (bf16*)nullptr, p.ld, seg);
     EFLA_LAUNCH("efla_q_seg_combine", (fast::seg_combine_kernel<K, V, false>),
-                dim3(p.N * p.H * (V / 16)), dim3(256), st, seg, p.nseg, p.H, S0);
+                dim3(p.N * p.H * (V / 16)), dim3(fast::comb_threads<K>()), st, seg, p.nseg, p.H, S0);
 }
 // ... and backwards
 template <int K, int V, bool PS>
@@ -1000,7 +1000,7 @@ static void seg_backward(const Problem& p, const SeqInfo& si, const bf16* q, con
                 dim3(fast::dh_threads<K>()), st, q, k, dO, Tc, bc, Pc, si, p.H, dST,
                 (float*)nullptr, (bf16*)nullptr, p.ld, seg);
     EFLA_LAUNCH("efla_q_seg_combine", (fast::seg_combine_kernel<K, V, true>),
-                dim3(p.N * p.H * (V / 16)), dim3(256), st, seg, p.nseg, p.H, dST);
+                dim3(p.N * p.H * (V / 16)), dim3(fast::comb_threads<K>()), st, seg, p.nseg, p.H, dST);
 }
 
 static int build_offsets(const Problem& p, const int32_t* cu, int32_t* cu_s, int32_t* coff,

@@ -116,68 +116,71 @@ __device__ __forceinline__ void seg_store(const SegOut& seg, int seq, int h, int
 // segment j, or nseg - 1 - j for REV): X[0] = S0 (or 0), X[1] is in place (the
 // first pass ran segment 0 from S0), X[j + 1] += M[j] X[j].  All in fp32 (fp32
 // MFMA): a workgroup carries 16 state columns of one (sequence, head) through
-// the segments, its four waves a quarter of the rows each; the column block
-// sits in LDS between segments, the next segment's M rows and X are loaded
-// during the current product.  nseg - 2 dependent products of K x K x 16,
-// about 2 us each (K = 128; 1 us for K = 64).
+// the segments, each wave 16 of the rows; the column block sits in LDS between
+// segments.  nseg - 2 dependent products of K x K x 16: their M rows and X are
+// requested kAhead segments early, so a step costs its product and not a trip
+// to memory (8 segments, K = V = 128, 16 heads: 25.0 us with one segment
+// requested after the product before, half the waves and every XCD reading every
+// M; 20.5 us now).
+constexpr int kAhead = 4;
+template <int K>
+constexpr int comb_threads() {
+    return 4 * K;
+}
 template <int K, int V, bool REV>
-__global__ void __launch_bounds__(256) seg_combine_kernel(SegOut seg, int nseg, int H,
-                                                          const float* __restrict__ S0) {
-    constexpr int RT = K / 64;  // 16-row tiles per wave
-    __shared__ float X[2][K][16 + 1];
+__global__ void __launch_bounds__(comb_threads<K>()) seg_combine_kernel(
+    SegOut seg, int nseg, int H, const float* __restrict__ S0) {
+    __shared__ __attribute__((aligned(16))) float X[2][16][K + 4];  // [column][row]
     const int w = mf::wave(), l = mf::lane(), g = l >> 4, r = l & 15;
-    constexpr int NC = V / 16;
-    const int col = (int)(blockIdx.x % NC) * 16 + r;
-    const int bh = blockIdx.x / NC, seq = bh / H, h = bh % H;
+    // the workgroups of one (sequence, head) a multiple of B H apart: on one
+    // XCD where that is a multiple of 8, so its L2 is the only one to read M
+    const int nbh = gridDim.x / (V / 16), bh = blockIdx.x % nbh;
+    const int col = (int)(blockIdx.x / nbh) * 16 + r, seq = bh / H, h = bh % H;
     auto at = [&](int j) {
         return (long)(seq * nseg + (REV ? nseg - 1 - j : j)) * H + h;
     };
+    floatx4 m[kAhead][K / 16], c[kAhead];
+    auto fetch = [&](int j, floatx4 (&mj)[K / 16], floatx4& cj) {  // M[j]'s rows and X[j + 1]
+        const float* mp = seg.M + at(j) * K * K + (long)(16 * w + r) * K + 4 * g;
+#pragma unroll
+        for (int i = 0; i < K / 16; ++i) mj[i] = *reinterpret_cast<const floatx4*>(mp + 16 * i);
+        const float* xp = seg.X + at(j + 1) * K * V + (long)(16 * w + 4 * g) * V + col;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) cj[e] = xp[(long)e * V];
+    };
+#pragma unroll
+    for (int d = 0; d < kAhead; ++d)
+        if (d + 2 < nseg) fetch(d + 1, m[d], c[d]);
     // X[0]
     float* x0 = seg.X + at(0) * K * V + col;
     const float* s0 = S0 ? S0 + (long)bh * K * V + col : nullptr;
-    for (int row = threadIdx.x >> 4; row < K; row += 16)
+    for (int row = threadIdx.x >> 4; row < K; row += K / 4) {
         x0[(long)row * V] = s0 ? s0[(long)row * V] : 0.f;
-    floatx4 m[RT][K / 16], c[RT];
-    auto fetch = [&](int j) {  // M[j]'s rows and X[j + 1]
-#pragma unroll
-        for (int t = 0; t < RT; ++t) {
-            const int row0 = 16 * (w + 4 * t);
-            const float* mp = seg.M + at(j) * K * K + (long)(row0 + r) * K + 4 * g;
-#pragma unroll
-            for (int i = 0; i < K / 16; ++i) m[t][i] = *reinterpret_cast<const floatx4*>(mp + 16 * i);
-            const float* xp = seg.X + at(j + 1) * K * V + (long)(row0 + 4 * g) * V + col;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) c[t][e] = xp[(long)e * V];
-        }
-    };
-    if (nseg > 2) fetch(1);
-    for (int row = threadIdx.x >> 4; row < K; row += 16)
-        X[1][row][r] = seg.X[at(1) * K * V + (long)row * V + col];
+        X[1][r][row] = seg.X[at(1) * K * V + (long)row * V + col];
+    }
     __syncthreads();
-    for (int j = 1; j + 1 < nseg; ++j) {
-        floatx4 a[RT];
+    for (int j0 = 1; j0 + 1 < nseg; j0 += kAhead) {
 #pragma unroll
-        for (int t = 0; t < RT; ++t) a[t] = c[t];
+        for (int d = 0; d < kAhead; ++d) {
+            const int j = j0 + d;
+            if (j + 1 < nseg) {  // uniform
+                floatx4 a = c[d], x[K / 16];
 #pragma unroll
-        for (int i = 0; i < K / 16; ++i)
+                for (int i = 0; i < K / 16; ++i)
+                    x[i] = *reinterpret_cast<const floatx4*>(&X[j & 1][r][16 * i + 4 * g]);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float xv = X[j & 1][16 * i + 4 * g + e][r];
+                for (int i = 0; i < K / 16; ++i)
 #pragma unroll
-                for (int t = 0; t < RT; ++t) a[t] = mma_f32(m[t][i][e], xv, a[t]);
-            }
-        if (j + 2 < nseg) fetch(j + 1);
+                    for (int e = 0; e < 4; ++e) a = mma_f32(m[d][i][e], x[i][e], a);
+                if (j + kAhead + 1 < nseg) fetch(j + kAhead, m[d], c[d]);
+                const int row0 = 16 * w + 4 * g;
+                float* xp = seg.X + at(j + 1) * K * V + (long)row0 * V + col;
 #pragma unroll
-        for (int t = 0; t < RT; ++t) {
-            const int row0 = 16 * (w + 4 * t) + 4 * g;
-            float* xp = seg.X + at(j + 1) * K * V + (long)row0 * V + col;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                xp[(long)e * V] = a[t][e];
-                X[(j + 1) & 1][row0 + e][r] = a[t][e];
+                for (int e = 0; e < 4; ++e) xp[(long)e * V] = a[e];
+                *reinterpret_cast<floatx4*>(&X[(j + 1) & 1][r][row0]) = a;
+                __syncthreads();
             }
         }
-        __syncthreads();
     }
 }
 

@@ -6,10 +6,11 @@
 //   backward: dA = dC B^T, dB = A^T dC, dbias = column sums of dC   (bf16)
 //
 // Matching bf16 / fp16 operands take the large-tile kernel of gemm_fast.hpp
-// (256 x 256 workgroup tiles of v_mfma_f32_32x32x16, operands copied straight
-// into LDS, persistent grid in XCD bands, split-K for short grids, fused
-// bias / residual / GELU epilogues), operands of odd strides or sizes from
-// padded copies.  Everything else -- fp32 and mixed dtypes, small odd shapes
+// (256 x 256 or 128 x 128 workgroup tiles of v_mfma_f32_32x32x16, operands
+// copied straight into LDS, persistent grid in XCD bands, split-K for short
+// grids, fused bias / residual / GELU epilogues), operands of odd strides or
+// sizes from padded copies; products of up to 64 rows the kernel of
+// gemm_skinny.hpp.  Everything else -- fp32 and mixed dtypes, small odd shapes
 // (kPadMinWork), and efla_rt_set_gemm_backend(1) -- runs the generic kernel
 // below.
 //

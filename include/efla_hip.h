@@ -362,11 +362,14 @@ int prism_backward_hip(const void* grad_output, const void* u, const void* v, co
 /* ========================================================================
  * GEMM (row-major)
  *
- * Hand-written MFMA kernels: bf16 / fp16 problems whose k, output columns
- * and strides are multiples of 8 elements (16-byte rows) run a 256 x 256 x 64
- * tile kernel; everything else (fp32, mixed dtypes, other shapes) a generic
- * 128 x 128 one (efla_rt_set_gemm_backend(1) forces it).  No vendor BLAS
- * is linked.
+ * Hand-written MFMA kernels.  bf16 / fp16 problems run a 256 x 256 x 64 or a
+ * 128 x 128 x 64 tile kernel, whichever is estimated faster, or, with up to 64
+ * rows, a kernel that streams the second operand once.  Operands whose rows are not whole 16-byte
+ * pieces (odd sizes, strides or alignments) are first copied into padded rows
+ * in the stream's workspace (at most 4 GiB; where that is not to be had, and
+ * for products below 2^22 multiply-adds, the generic kernel takes them).
+ * fp32 and mixed dtypes run the generic 128 x 128 kernel
+ * (efla_rt_set_gemm_backend(1) forces it).  No vendor BLAS is linked.
  * ======================================================================== */
 
 /* Replaces gemm_forward_cuda (kernels.h:211-223, gemm.cu:303-398):

@@ -18,10 +18,10 @@
 // T, W, U; parallel over chunks), state (serial over chunks, one workgroup
 // per (sequence, head, 64-wide value slice), S held in MFMA accumulators),
 // output (parallel over chunks).  Generic backward: it recomputes b, W, U and
-// the chunk states, then runs dv_local (tril(QK^T)^T dO), a reverse state
-// scan for dS, dq/dk/dw per chunk, and the WY backward that carries dW, dU
-// through T and b (including the dc/dlambda term of efla.cu:384-451 and
-// dbeta = dc * exp(-beta lambda)).  This file also holds the host side:
+// the chunk states where the forward did not leave them, then runs dv_local
+// (tril(QK^T)^T dO), a reverse state scan for dS, dq/dk/dw per chunk, and the
+// WY backward that carries dW, dU through T and b (including the dc/dlambda
+// term of efla.cu:384-451 and dbeta = dc * exp(-beta lambda)).  This file also holds the host side:
 // validation, workspace layout and the launches.
 #include <hip/hip_runtime.h>
 #include <stdlib.h>
@@ -273,10 +273,10 @@ struct Piece64 {
 // forward: state scan.  grid (N*H, V/VS).  One workgroup carries S[:, slice]
 // (64 x 64, fp32) through all chunks of its sequence in MFMA accumulators: wave
 // w owns the 16 x 16 tile (w & 3, w >> 2).  Per chunk it stores the chunk
-// start state (transposed [v][k] when HT, else [k][v]) and Vn; the next chunk's
-// rows are loaded into registers meanwhile.
+// start state (transposed, [v][k]) and Vn; the next chunk's rows are loaded into
+// registers meanwhile.
 // ---------------------------------------------------------------------------
-template <typename T, int K, int V, int VS, bool HT>
+template <typename T, int K, int V, int VS>
 __global__ void __launch_bounds__(NTH) fwd_state_kernel(const T* __restrict__ k,
                                                         const T* __restrict__ W,
                                                         const T* __restrict__ U, SeqInfo si,
@@ -320,12 +320,7 @@ __global__ void __launch_bounds__(NTH) fwd_state_kernel(const T* __restrict__ k,
         if (n + 1 < nch) fetch(n + 1);
         T* hb = hout + (slot * H + h) * (long)K * V;
         store_frag_t(STs, LDF, row, col, S);
-        if (HT) {
-            *reinterpret_cast<floatx4*>(hb + (long)(v0 + col) * K + row) = S;
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) hb[(long)(row + i) * V + v0 + col] = S[i];
-        }
+        *reinterpret_cast<floatx4*>(hb + (long)(v0 + col) * K + row) = S;
         __syncthreads();
         floatx4 acc = {0.f, 0.f, 0.f, 0.f};
         acc = tile_mma<T, K>(acc, view_k((const T*)Ws, LDF), 16 * (w & 3),
@@ -516,7 +511,8 @@ __global__ void __launch_bounds__(NTH) bwd_state_kernel(
 //   dq  = dO h^T + Dm K
 //   dk' = Dm^T Q + Vn dh^T
 //   dW  = -dVn h^T
-// h = chunk start state, dh = gradient of the chunk end state, both [k][v].
+// h = chunk start state, [v][k] as the state scan leaves it (for the forward's
+// output kernel too); dh = gradient of the chunk end state, [k][v].
 // ---------------------------------------------------------------------------
 template <typename T, int K, int V>
 __global__ void __launch_bounds__(NTH) bwd_dqkw_kernel(
@@ -563,7 +559,7 @@ __global__ void __launch_bounds__(NTH) bwd_dqkw_kernel(
         load_rows<T, 64, 64, NTH>(dOs, LD64, dO + (bos * H + h) * V + v0, (long)H * V, len);
         load_rows<T, 64, 64, NTH>(Vns, LD64, Vn + (bos * H + h) * V + v0, (long)H * V, len);
         load_rows<T, 64, 64, NTH>(dVns, LD64, dVn + (bos * H + h) * V + v0, (long)H * V, len);
-        load_rows<T, K, 64, NTH>(hs, LD64, hst + hbase + v0, V, K);
+        load_rows_t<T, 64, K, NTH>(hs, LD64, hst + hbase + (long)v0 * K, K, 64);
         load_rows<T, K, 64, NTH>(dhs, LD64, dhst + hbase + v0, V, K);
         __syncthreads();
 #pragma unroll
@@ -1034,7 +1030,7 @@ static int run_fwd(const Problem& p, const T* q, const T* k, const T* v, const T
     } else {
         EFLA_LAUNCH("efla_q_fwd_prep", (fwd_prep_kernel<T, K, V>), dim3(p.slots, H), dim3(NTH),
                     st, k, v, beta, si, H, w.bco, w.W, w.U);
-        EFLA_LAUNCH("efla_q_fwd_state", (fwd_state_kernel<T, K, V, VS, true>),
+        EFLA_LAUNCH("efla_q_fwd_state", (fwd_state_kernel<T, K, V, VS>),
                     dim3(p.N * H, V / VS), dim3(NTH), st, k, w.W, w.U, si, H, S0, ST, w.h, w.Vn);
         EFLA_LAUNCH("efla_q_fwd_o", (fwd_o_kernel<T, K, V, VO>), dim3(p.slots, H, V / VO),
                     dim3(NTH), st, q, k, w.h, w.Vn, si, H, o);
@@ -1110,11 +1106,14 @@ static int run_bwd(const Problem& p, const T* q, const T* k, const T* v, const T
         if (!reuse)
             EFLA_LAUNCH("efla_q_bwd_re_prep", (fwd_prep_kernel<T, K, V>), dim3(p.slots, H),
                         dim3(NTH), st, k, v, beta, si, H, w.bco, w.W, w.U);
-        // the generic forward keeps its states transposed for its output kernel,
-        // so this path recomputes them whatever reuse_states says
-        EFLA_LAUNCH("efla_q_bwd_re_state", (fwd_state_kernel<T, K, V, VS, false>),
-                    dim3(p.N * H, V / VS), dim3(NTH), st, k, w.W, w.U, si, H, S0,
-                    (float*)nullptr, w.h, w.Vn);
+        // The forward left the states and Vn in the workspace: the scan over them,
+        // serial in the chunks, need not run again (forward + backward, with it /
+        // without, us: 1 x 1024 x 1 head 255 / 202, 3 x 700 x 4 203 / 165,
+        // 8 x 1024 x 8 449 / 391).
+        if (!reuse_states)
+            EFLA_LAUNCH("efla_q_bwd_re_state", (fwd_state_kernel<T, K, V, VS>),
+                        dim3(p.N * H, V / VS), dim3(NTH), st, k, w.W, w.U, si, H, S0,
+                        (float*)nullptr, w.h, w.Vn);
         EFLA_LAUNCH("efla_q_bwd_dvloc", (bwd_dvloc_kernel<T, K, V, VO>),
                     dim3(p.slots, H, V / VO), dim3(NTH), st, q, k, dO, si, H, w.dvloc);
         EFLA_LAUNCH("efla_q_bwd_state", (bwd_state_kernel<T, K, V, VS>), dim3(p.N * H, V / VS),

@@ -145,8 +145,8 @@ size_t efla_chunk_bwd_workspace_size(size_t batch_size, size_t seq_len, size_t n
 #define EFLA_BWD_REUSE_FORWARD 1u
 /* With EFLA_BWD_REUSE_FORWARD only: the forward also ran with
  * EFLA_FWD_SAVE_STATES on this workspace, so the chunk states and P are read
- * from it too and the backward runs no forward recompute at all (bf16; the
- * fp32 path accepts the flag and recomputes the states). */
+ * (fp32: the states and Vn, which every forward on a caller's workspace leaves
+ * there) from it too and the backward runs no forward recompute at all. */
 #define EFLA_BWD_REUSE_STATES 2u
 
 /* Gradients of sum(output * grad_output) + sum(final_state * grad_final_state);

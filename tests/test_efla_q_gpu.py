@@ -269,6 +269,39 @@ def test_backward_reusing_forward_factors(oracle, dtype, K, V, states):
             assert rel_l2(a, b.float().cpu().numpy()) <= 1e-6, n
 
 
+# The fp32 backward reads the forward's chunk states and Vn where they were saved.
+# One workspace through several backwards, with and without a recompute of the
+# states in between, over packed sequences with an empty one, lone tokens and
+# whole and ragged chunks: the same sums each time (the bit-exact outputs), except
+# dk and dbeta, into which dL/dlambda and dL/dbeta come by LDS float atomics (2^-24
+# per term of a few hundred: 1e-6 as above).
+@pytest.mark.parametrize("lens", [(1,), (64, 0, 65), (130, 1, 63, 200)])
+def test_fp32_backward_from_saved_states(oracle, lens):
+    from ceo_amd.efla import chunk_efla_bwd, chunk_efla_fwd, new_workspace
+
+    announce(f"chunk_efla fp32 saved states lens={lens}")
+    H, K, V, T, N = 3, 64, 64, sum(lens), len(lens)
+    x = oracle.make_efla_inputs(77 + T, T, H, K, V, bf16=False)
+    g = {n: to_dev(a, torch.float32, (1, T, H, K) if n in "qk" else
+                   (1, T, H) if n == "beta" else (1, T, H, V)) for n, a in x.items()}
+    cu = torch.tensor(np.cumsum((0,) + lens), dtype=torch.int32).cuda()
+    gen = torch.Generator().manual_seed(6)
+    s0, dst = (0.1 * torch.randn(N, H, K, V, generator=gen).cuda() for _ in range(2))
+    args = (g["q"], g["k"], g["v"], g["beta"])
+    ref = chunk_efla_bwd(*args, g["do"], s0, dst, cu)
+    ws = new_workspace(g["q"], g["v"], cu)
+    chunk_efla_fwd(*args, s0, True, cu, workspace=ws, save_states=True)
+    for states in (True, True, False, True):
+        got = chunk_efla_bwd(*args, g["do"], s0, dst, cu, workspace=ws, reuse_forward=True,
+                             reuse_states=states)
+        torch.cuda.synchronize()
+        for a, b, n in zip(got, ref, ("dq", "dk", "dv", "dbeta", "dh0")):
+            if n in ("dk", "dbeta"):
+                assert rel_l2(a, b.cpu().numpy()) <= 1e-6, n
+            else:
+                assert torch.equal(a, b), n
+
+
 def test_packed_batch_runs_sequences_independently(oracle):
     """efla_pack_sequences output drives the varlen entries: each packed
     sequence's outputs and gradients equal a separate run on that sequence."""

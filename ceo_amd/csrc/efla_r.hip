@@ -740,8 +740,12 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_chain_kernel(
 //   grad_lambda = dc/dlambda * sum_c w2_c sw_c       (= sum_row k_row (g w2)_row)
 // where S / S_n are the states before / after the token.  Column sums are
 // lane-local (plus the lanes of the column); the row sum goes through LDS as
-// bf16 high and low parts of each fp32 summand (about 16 bits kept) and
-// 16x16x32 MFMAs against ones.
+// bf16 parts of each fp32 summand and 16x16x32 MFMAs against ones.  d = 64 and
+// 128 keep a high and a low part (about 16 bits).  d = 32 keeps three, cut and
+// not rounded, which together are the summand exactly: its sums were plain fp32
+// ones in the LDS-resident kernel, and a row whose terms cancel shows the
+// difference also in bf16 (backward with two parts / three: 2 x 1000 tokens, 8
+// heads 164 / 167 us; 4 x 2048, 32 heads 617 / 637).
 // Segments of SEGF tokens are taken last to first.  A segment's k, dO, c and
 // dc/dlambda (and c k in fp32 and this workgroup's v columns where LDS allows:
 // the split kernels) are staged in LDS by the whole workgroup at once, their
@@ -750,11 +754,17 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_chain_kernel(
 // without barriers (each lane's column needs only its own rows), every state
 // stored column-major to the workspace (hist), which the same lanes read back
 // in the reverse pass (one barrier per token, for the row sum).
+// x cut (towards zero) to its upper 8 significant bits
+__device__ __forceinline__ bf16 cut_bf16(float x) {
+    return __builtin_bit_cast(bf16, (unsigned short)(__builtin_bit_cast(unsigned, x) >> 16));
+}
+
 template <int D, int NS>
 struct RBwdSmem {
     static constexpr bool CKS = NS > 1;  // c k and v staged; else formed per row / read per lane
     bf16 Mh[2][(D / NS) * (D + 8)];      // the row sum's summands [c][row], high bf16 part
     bf16 Ml[2][(D / NS) * (D + 8)];      // low part
+    bf16 Mx[2][D == 32 ? D * (D + 8) : 8];  // d = 32: the rest
     SegLds<D, D / NS, true, CKS, CKS, true> seg;
     float gkv[2][D / NS];                // S_n^T dO per column
     float red[2][16];                    // grad_c partials per wave
@@ -950,18 +960,27 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_bwd_fast_kern
                 bf16* ml = sm.Ml[par] + lcol * LDS + r0;
 #pragma unroll
                 for (int i8 = 0; i8 < RPL / 8; ++i8) {
-                    bf16x8 hv, lv;
+                    bf16x8 hv, lv, xv;
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
                         const int ii = 8 * i8 + e;
                         const float sp = (float)SpR[s][ii / 2][ii % 2];
                         const float m = fmaf(G[ii], cw2, -(sp * w1));
-                        hv[e] = (bf16)m;
-                        lv[e] = (bf16)(m - (float)hv[e]);
+                        if constexpr (D == 32) {
+                            hv[e] = cut_bf16(m);
+                            const float m1 = m - (float)hv[e];
+                            lv[e] = cut_bf16(m1);
+                            xv[e] = cut_bf16(m1 - (float)lv[e]);
+                        } else {
+                            hv[e] = (bf16)m;
+                            lv[e] = (bf16)(m - (float)hv[e]);
+                        }
                         G[ii] = fmaf(-kf[ii], w1, G[ii]);
                     }
                     *reinterpret_cast<bf16x8*>(mh + 8 * i8) = hv;
                     *reinterpret_cast<bf16x8*>(ml + 8 * i8) = lv;
+                    if constexpr (D == 32)
+                        *reinterpret_cast<bf16x8*>(sm.Mx[par] + lcol * LDS + r0 + 8 * i8) = xv;
                 }
                 // grad_c = sum_c w2_c sw_c: one value per column, then per wave
                 const float gc = wave_sum_q4(part == 0 ? w2 * sw : 0.f);
@@ -979,10 +998,18 @@ __global__ void __launch_bounds__((rfast_threads<D, NS, LPC>())) r_bwd_fast_kern
                 for (int m = 0; m < MT; ++m) {
                     const int f0 = 16 * (MT * w + m);
                     mf::floatx4 acc = mf::zero4();
+                    if constexpr (D == 32) {  // (the small parts beside the high one)
+                        mf::floatx4 low = mf::mma(mf::frag_trc(l, sm.Mx[par], LDS, 0, f0), ones, acc);
+                        acc = mf::mma(mf::frag_trc(l, sm.Mh[par], LDS, 0, f0), ones, acc);
+                        low = mf::mma(mf::frag_trc(l, sm.Ml[par], LDS, 0, f0), ones, low);
 #pragma unroll
-                    for (int q = 0; q < NK; ++q) {
-                        acc = mf::mma(mf::frag_trc(l, sm.Mh[par], LDS, 32 * q, f0), ones, acc);
-                        acc = mf::mma(mf::frag_trc(l, sm.Ml[par], LDS, 32 * q, f0), ones, acc);
+                        for (int i = 0; i < 4; ++i) acc[i] += low[i];
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < NK; ++q) {
+                            acc = mf::mma(mf::frag_trc(l, sm.Mh[par], LDS, 32 * q, f0), ones, acc);
+                            acc = mf::mma(mf::frag_trc(l, sm.Ml[par], LDS, 32 * q, f0), ones, acc);
+                        }
                     }
                     // the 16 columns of acc are equal (B is ones); with the
                     // column split lanes 0..3 of each row group add one row each

@@ -342,3 +342,41 @@ def test_token_groups_same_bits(oracle, T, d):
                     ("grad_v", gv[:, :, few], gv2), ("state", st[few], st2),
                     ("grad_state", gs[few], gs2)):
         assert torch.equal(a, b), n
+
+
+def test_backward_d32_row_sums_keep_fp32(oracle):
+    """grad_k where every term of it cancels, at d = 32, whose row sums are fp32
+    sums of fp32 summands.  v = 0 and S^T k = 0 (k equal in pairs of rows, S
+    of opposite sign in them), so the state stays; S^T dO = 0 in the same way;
+    and S k = 0 by three columns with 3 * 6 + 5 * 2 - 7 * 4 = 0.  The last
+    token's grad_k is then - sum_c S[:, c] w1_c with w1 = c (dO . k) k: zero
+    but for the rounding of w1_c, of each product, and of the sum's three
+    terms, in all at most 5 * 2^-24 sum |S w1|; checked at 8 * 2^-24.  Summands
+    kept to 16 bits are off by up to 2^-18 each."""
+    from ceo_amd.efla import efla_backward
+
+    announce("efla_backward_hip d=32 cancelling row sums")
+    B, T, H, d = 2, 6, 96, 32
+    rng = np.random.default_rng(31)
+    k = np.repeat(rng.integers(1, 8, (B, H, d // 2)), 2, axis=-1).astype(np.float64) / 16
+    k[..., (0, 1)], k[..., (4, 5)], k[..., (8, 9)] = 3 / 16, 5 / 16, 7 / 16
+    do = np.zeros((B, T, H, d))
+    do[:, -1] = np.repeat(rng.integers(1, 100, (B, H, d // 2)), 2, axis=-1)
+    s = np.zeros((B, H, d, d))
+    sign = np.where(np.arange(d) % 2 == 0, 1.0, -1.0)
+    s[..., 0], s[..., 4], s[..., 8] = 6 * sign, 2 * sign, -4 * sign
+
+    def dev(a):
+        return torch.from_numpy(np.ascontiguousarray(a)).to(torch.bfloat16).cuda()
+
+    kt = dev(np.broadcast_to(k[:, None], (B, T, H, d)))
+    beta = 0.7
+    gk, gv, gs = efla_backward(dev(do), kt, torch.zeros_like(kt), dev(s.reshape(B * H, d, d)), beta)
+    torch.cuda.synchronize()
+    lam = (k ** 2).sum(-1)
+    w1 = ((1 - np.exp(-beta * lam)) / lam * (do[:, -1] * k).sum(-1))[..., None] * k
+    assert rel_l2(gv[:, -1], w1.astype(np.float32)) <= 2.0 ** -8
+    scale = np.einsum("bhrc,bhc->bhr", np.abs(s), np.abs(w1))
+    worst = float((gk[:, -1].double().cpu().numpy().__abs__() / scale).max())
+    print(f"  worst |grad_k| / sum |S w1| = {worst:.2e}", flush=True)
+    assert worst <= 8 * 2.0 ** -24

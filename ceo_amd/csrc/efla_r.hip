@@ -1420,10 +1420,10 @@ extern "C" int efla_forward_hip(const void* k, const void* v, void* state, void*
     const dim3 grid((unsigned)nbh);
     // the register-resident path: d = 32 / 64 / 128, k and v aligned for d /
     // 8-byte row loads (the coefficient kernel's, the segment staging's) and
-    // output for 8-byte row pieces, at most 2^35 tokens (d = 32: where its
-    // scratch is to be had, the LDS-resident kernel needs none)
+    // output for 8-byte row pieces, at most 2^35 tokens (d = 32: not in a capture,
+    // since the LDS-resident kernel needs no scratch)
     const bool fast = (head_dim == 128 || head_dim == 64 ||
-                       (head_dim == 32 && workspace_available(nbh * seq_len * 4 + 256, stream))) &&
+                       (head_dim == 32 && workspace_optional(stream))) &&
                       (uintptr_t)k % (head_dim / 8) == 0 && (uintptr_t)v % (head_dim / 8) == 0 &&
                       (uintptr_t)output % 8 == 0 && nbh * seq_len <= ((size_t)1 << 35);
     if (fast) {

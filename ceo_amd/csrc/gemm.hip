@@ -583,9 +583,11 @@ static void skinny_launch_rows(const FastOp& a, const FastOp& b, long M, long N,
     else skinny_launch_mt<T, EPI, 4>(a, b, M, N, K, kper, ea, name, st);
 }
 
+// plain: as in fast_launch
 template <typename T, int EPI>
 static int skinny_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
-                         const gf::EpiArgs<T>& ea, const char* name, hipStream_t st) {
+                         const gf::EpiArgs<T>& ea, bool plain, const char* name,
+                         hipStream_t st) {
     // a workgroup takes 2.5 ns (16 rows) to 4.7 ns (64 rows) per row of the
     // weights, a split's reduction about 4 us: split k over the idle CUs from
     // 2048 rows on, at least 512 rows to a workgroup
@@ -596,7 +598,8 @@ static int skinny_launch(const FastOp& a, const FastOp& b, long M, long N, long 
         const long kper = ks > 1 ? (K + ks * 32 - 1) / (ks * 32) * 32 : K;
         const int n = (int)((K + kper - 1) / kper);
         const size_t bytes = (size_t)n * M * up8(N) * sizeof(float);
-        if (K >= 2048 && n > 1 && workspace_available(bytes, st)) {
+        if (K >= 2048 && n > 1 &&
+            (plain ? workspace_available(bytes, st) : workspace_optional(st))) {
             void* ws = nullptr;
             WsLease lease;
             if (workspace_acquire(bytes, st, &ws, lease) == kSuccess) {
@@ -640,8 +643,6 @@ static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
                        const gf::EpiArgs<T>& ea, const char* name, hipStream_t st,
                        size_t head_bytes = 0, WsLease* head_lease = nullptr) {
     if (M < 1 || N < 1 || K < 1 || M > INT32_MAX / 2 || N > INT32_MAX / 2) return -1;
-    if constexpr (EPI != gf::EPI_DGELU)
-        if (skinny_ok(a, b, M, N, K)) return skinny_launch<T, EPI>(a, b, M, N, K, ea, name, st);
     const bool pa = !direct_rows(a, M, K), pb = !direct_rows(b, N, K);
     // whole 16-byte pieces everywhere: nothing but split-K partials needs scratch
     const bool out_whole = N % 8 == 0 && ea.ldd % 8 == 0 && aligned_to(ea.d, 16) &&
@@ -649,6 +650,9 @@ static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
                            (!ea.c || (ea.ldc % 8 == 0 && aligned_to(ea.c, 16))) &&
                            (!ea.aux || (ea.ldaux % 8 == 0 && aligned_to(ea.aux, 16)));
     const bool plain = !pa && !pb && K % 8 == 0 && out_whole;
+    if constexpr (EPI != gf::EPI_DGELU)
+        if (skinny_ok(a, b, M, N, K))
+            return skinny_launch<T, EPI>(a, b, M, N, K, ea, plain, name, st);
     if (!plain && (double)M * (double)N * (double)K < (double)kPadMinWork) return -1;
     const Tiling tl = plan_tiling(M, N, K, EPI == gf::EPI_PLAIN || EPI == gf::EPI_RESID);
     if (tl.tiles > 0x7FFFFFFFL / 64) return plain ? kInvalidConfiguration : -1;
@@ -674,7 +678,7 @@ static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
         void* p = nullptr;
         // a product that the generic kernel would take without scratch does
         // so where scratch is not to be had (a stream under capture, memory)
-        if (!plain && !workspace_available(need, st)) return -1;
+        if (!plain && !workspace_optional(st)) return -1;
         const int rc = workspace_acquire(need, st, &p, head_lease ? *head_lease : own);
         if (rc != kSuccess) {
             if (plain) return rc;

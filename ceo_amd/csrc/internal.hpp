@@ -102,6 +102,12 @@ int workspace_acquire(size_t bytes, hipStream_t stream, void** ptr, WsLease& lea
 // cannot grow there).  For callers that have a slower way without scratch.
 bool workspace_available(size_t bytes, hipStream_t stream, int slot = 0);
 
+// Whether a call that has a form without scratch may use the cached buffer: not
+// where it is being captured.  A graph keeps the buffer's address, and the buffer
+// is freed when a larger call on the stream grows it (or its workspace is
+// released), and belongs to the stream the graph may not be replayed on.
+bool workspace_optional(hipStream_t stream, int slot = 0);
+
 // Zero-fill through a kernel (no hipMemsetAsync, so the call is safe inside
 // stream capture).
 int fill_zero(void* ptr, size_t bytes, hipStream_t stream);

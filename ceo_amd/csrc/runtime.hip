@@ -358,6 +358,13 @@ bool workspace_available(size_t bytes, hipStream_t stream, int slot) {
         std::lock_guard<std::mutex> lk(e->mu);
         if (e->bytes >= bytes) return true;
     }
+    return workspace_optional(stream, slot);
+}
+
+bool workspace_optional(hipStream_t stream, int slot) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    if (ws_entry(dev, stream, slot)->owner.load() == std::this_thread::get_id()) return false;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &st) != hipSuccess) {
         (void)hipGetLastError();

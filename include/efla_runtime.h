@@ -64,7 +64,18 @@ int efla_rt_event_elapsed_ms(float* ms, hipEvent_t start, hipEvent_t stop);
  * caches per (device, stream): callers on different streams never share
  * scratch, and calls on one stream from several host threads take turns
  * while they queue their kernels.  A buffer grows (after its stream drains)
- * only when a larger problem arrives. */
+ * only when a larger problem arrives.
+ *
+ * Stream capture: a call that cannot do without scratch (the EFLA entries
+ * without a caller's workspace, efla_forward_hip with head_dim 64 / 128,
+ * efla_backward_hip, gradients summed over rows) is captured with its buffer's address, and
+ * only when the buffer is large enough already (run the same call on the
+ * stream first).  Such a graph is valid while no larger call on that stream
+ * grows the buffer and the workspace is not released, and must not run beside
+ * other library calls of that stream.  So is an aligned bf16 / fp16 product
+ * split along its contraction.  The others (odd sizes, strides or alignments;
+ * efla_forward_hip with other head_dim) are captured in forms without scratch
+ * and have no such condition. */
 /* Bytes currently held by the cached workspaces of the current device. */
 size_t efla_rt_workspace_bytes(void);
 /* Release the cached workspaces of the current device (synchronises it). */

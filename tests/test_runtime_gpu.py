@@ -228,3 +228,56 @@ def test_workspace_released_with_its_stream(L):
     assert all(rc == 0 for rc, _ in left)
     assert [b for _, b in left] == [(3 - j) * totals[0] for j in range(4)]
     assert runtime.workspace_bytes() == 0
+
+
+# Calls that have a form without scratch are captured in it, also where the
+# stream's workspace is large enough already: the graph stays valid when that
+# workspace is freed.  The memory it had is handed to a tensor of known values,
+# which the replays must leave alone.  Bounds: products are rounded once to bf16
+# (2^-8 at most); efla_forward's bf16 trajectory 2e-2 as in its own tests.
+@pytest.mark.parametrize("what", ["odd", "odd weight gradient", "few rows, split", "d=32"])
+def test_graphs_hold_no_scratch(what):
+    from ceo_amd import lib, nn
+    from ceo_amd.efla import efla_forward
+
+    announce(f"graph without scratch: {what}")
+    g = torch.Generator(device="cuda").manual_seed(3)
+
+    def r(*s, std=1.0):
+        return (torch.randn(*s, generator=g, device="cuda") * std).to(torch.bfloat16)
+
+    if what == "d=32":
+        k, v, s0 = r(2, 300, 4, 32, std=0.2), r(2, 300, 4, 32), r(8, 32, 32, std=0.2)
+
+        def call():
+            return efla_forward(k, v, s0.clone(), 0.5)
+        ref, tol = call().double(), 2e-2
+    else:
+        m, kk, n = (16, 4096, 1026) if what == "few rows, split" else (300, 331, 517)
+        a, b, dc = r(m, kk), r(kk, n), r(m, n)
+        if what == "odd weight gradient":
+            def call():
+                return nn.gemm_backward(dc, a, b, need_a=False)[1]
+            ref = a.double().T @ dc.double()
+        else:
+            def call():
+                return nn.gemm_forward(a, b)
+            ref = a.double() @ b.double()
+        tol = 2.0 ** -8
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        call()
+        assert lib().efla_rt_workspace_bytes() > 0
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            out = call()
+    assert lib().efla_rt_workspace_release_stream(stream.cuda_stream) == 0
+    held = torch.full((64 << 18,), 7.0, device="cuda")
+    for _ in range(4):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert ((out.double() - ref).norm() / ref.norm()).item() <= tol
+        assert bool((held == 7.0).all())
+        call()  # the program's own work in between

@@ -635,13 +635,16 @@ constexpr size_t kPadMaxBytes = (size_t)4 << 30;
 // Large-tile product, or -1 if it does not take the problem (the generic
 // kernel does).  Where the contraction is split (plan_tiling), fp32
 // partial tiles go to the stream's cached workspace and a second kernel adds
-// them in split order and runs the epilogue (plain epilogues only).
+// them in split order and runs the epilogue (plain epilogues only).  Where
+// the workspace is not to be had (a cold one under capture, memory), an aligned
+// product runs in one piece.
 // Workspace: [head_bytes for the caller (ea.cpart) | padded A | padded B |
 // partials]; with head_bytes the lease stays with the caller.
 template <typename T, int EPI>
 static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
                        const gf::EpiArgs<T>& ea, const char* name, hipStream_t st,
-                       size_t head_bytes = 0, WsLease* head_lease = nullptr) {
+                       size_t head_bytes = 0, WsLease* head_lease = nullptr,
+                       bool may_split = true) {
     if (M < 1 || N < 1 || K < 1 || M > INT32_MAX / 2 || N > INT32_MAX / 2) return -1;
     const bool pa = !direct_rows(a, M, K), pb = !direct_rows(b, N, K);
     // whole 16-byte pieces everywhere: nothing but split-K partials needs scratch
@@ -654,7 +657,8 @@ static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
         if (skinny_ok(a, b, M, N, K))
             return skinny_launch<T, EPI>(a, b, M, N, K, ea, plain, name, st);
     if (!plain && (double)M * (double)N * (double)K < (double)kPadMinWork) return -1;
-    const Tiling tl = plan_tiling(M, N, K, EPI == gf::EPI_PLAIN || EPI == gf::EPI_RESID);
+    const Tiling tl = plan_tiling(M, N, K, (EPI == gf::EPI_PLAIN || EPI == gf::EPI_RESID) &&
+                                               may_split);
     if (tl.tiles > 0x7FFFFFFFL / 64) return plain ? kInvalidConfiguration : -1;
     const int ksplit = tl.ksplit;
     // scratch
@@ -679,12 +683,15 @@ static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
         // a product that the generic kernel would take without scratch does
         // so where scratch is not to be had (a stream under capture, memory)
         if (!plain && !workspace_optional(st)) return -1;
-        const int rc = workspace_acquire(need, st, &p, head_lease ? *head_lease : own);
+        const bool split_only = plain && !head_bytes;  // scratch for the partials alone
+        int rc = kInvalidValue;
+        if (!split_only || workspace_available(need, st))
+            rc = workspace_acquire(need, st, &p, head_lease ? *head_lease : own);
         if (rc != kSuccess) {
-            if (plain) return rc;
+            if (plain && !split_only) return rc;
             (void)hipGetLastError();
             (head_lease ? *head_lease : own).release();
-            return -1;
+            return plain ? fast_launch<T, EPI>(a, b, M, N, K, ea, name, st, 0, nullptr, false) : -1;
         }
         ws = (char*)p;
     }

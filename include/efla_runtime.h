@@ -73,7 +73,8 @@ int efla_rt_event_elapsed_ms(float* ms, hipEvent_t start, hipEvent_t stop);
  * stream first).  Such a graph is valid while no larger call on that stream
  * grows the buffer and the workspace is not released, and must not run beside
  * other library calls of that stream.  So is an aligned bf16 / fp16 product
- * split along its contraction.  The others (odd sizes, strides or alignments;
+ * split along its contraction, which without a large enough buffer is captured
+ * in one piece (the same sum, other roundings).  The others (odd sizes, strides or alignments;
  * efla_forward_hip with other head_dim) are captured in forms without scratch
  * and have no such condition. */
 /* Bytes currently held by the cached workspaces of the current device. */

@@ -281,3 +281,30 @@ def test_graphs_hold_no_scratch(what):
         assert ((out.double() - ref).norm() / ref.norm()).item() <= tol
         assert bool((held == 7.0).all())
         call()  # the program's own work in between
+
+
+def test_split_product_captured_on_a_cold_stream():
+    """A product that is split along its contraction outside of a capture runs
+    in one piece where its stream has no workspace yet.  Both are fp32 sums
+    rounded once to bf16 (2^-8 at most)."""
+    from ceo_amd import lib, nn
+
+    announce("graph: split product, cold stream")
+    g = torch.Generator(device="cuda").manual_seed(4)
+    a, b = (torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+            for s in ((256, 8192), (8192, 256)))
+    few = a[:16].contiguous()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    assert lib().efla_rt_workspace_release_stream(stream.cuda_stream) == 0
+    refs = [x.double() @ b.double() for x in (a, few)]
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        outs = [nn.gemm_forward(x, b) for x in (a, few)]
+    for _ in range(3):
+        for o in outs:
+            o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for o, ref in zip(outs, refs):
+            assert ((o.double() - ref).norm() / ref.norm()).item() <= 2.0 ** -8
+        nn.gemm_forward(a, b)

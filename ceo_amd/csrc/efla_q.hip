@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 #include <stdlib.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "../../include/efla_hip.h"
@@ -1166,6 +1167,16 @@ static bool supported(int dtype, size_t K, size_t V) {
         if (p.K == 128 && p.V == 256) return FN<bf16, 128, 256>(__VA_ARGS__);   \
     } while (0)
 
+// The chunk slots and the scans' segments of a problem whose sizes are set, for the
+// calls and the size queries alike.
+static void set_layout(Problem* p, bool varlen, size_t seq_len, int dtype) {
+    p->varlen = varlen;
+    p->T = varlen ? 0 : (long)seq_len;
+    p->nt = varlen ? 0 : (int)((seq_len + BT - 1) / BT);
+    p->slots = varlen ? p->ntok / BT + p->N : (long)p->N * p->nt;
+    plan_segments(p, dtype);
+}
+
 // Validates the Mode Q arguments and fills `p`.  Returns kSuccess, or the
 // error code to return; *empty is set when there are no tokens to process.
 static int make_problem(const void* q, const void* k, const void* v, const void* beta,
@@ -1197,15 +1208,11 @@ static int make_problem(const void* q, const void* k, const void* v, const void*
     p->H = (int)H;
     p->K = (int)K;
     p->V = (int)V;
-    p->varlen = cu != nullptr;
-    p->T = p->varlen ? 0 : (long)seq_len;
-    p->nt = p->varlen ? 0 : (int)((seq_len + BT - 1) / BT);
-    p->slots = p->varlen ? (long)(ntok / BT + num_seqs) : (long)num_seqs * p->nt;
+    set_layout(p, cu != nullptr, seq_len, dtype);
     p->ld = TokLd{(long)(H * K), (long)(H * K), (long)(H * V), (long)(H * K), (long)(H * K),
                   (long)(H * V)};
     if ((size_t)p->N * H > (size_t)INT32_MAX || (size_t)p->slots > (size_t)INT32_MAX)
         return kInvalidConfiguration;
-    plan_segments(p, dtype);
     if (seq_len == 0) {
         *empty = true;
         return kSuccess;
@@ -1221,49 +1228,50 @@ using namespace efla;
 using namespace efla::q;
 
 // Workspace bound covering both the fixed-length and the packed layout of
-// batch_size * seq_len tokens in max(num_seqs, batch_size) sequences.
-static bool ws_problem(size_t batch, size_t seq_len, size_t num_seqs, size_t H, size_t K,
-                       size_t V, int dtype, Problem* p) {
-    if (H == 0 || K == 0 || V == 0 || !supported(dtype, K, V)) return false;
+// batch_size * seq_len tokens in max(num_seqs, batch_size) sequences: the larger
+// of the two, each planned and laid out as its calls do it (0: not supported).
+template <typename Carve>
+static size_t ws_size(size_t batch, size_t seq_len, size_t num_seqs, size_t H, size_t K, size_t V,
+                      int dtype, Carve carve) {
+    if (H == 0 || K == 0 || V == 0 || !supported(dtype, K, V)) return 0;
     size_t ntok;
-    if (!mul_ok(batch, seq_len, &ntok) || ntok > (size_t)INT32_MAX) return false;
+    if (!mul_ok(batch, seq_len, &ntok) || ntok > (size_t)INT32_MAX) return 0;
     const size_t N = num_seqs > batch ? num_seqs : batch;
-    if (N == 0 || N > (size_t)INT32_MAX / 2) return false;
-    p->ntok = (long)ntok;
-    p->N = (int)N;
-    p->H = (int)H;
-    p->K = (int)K;
-    p->V = (int)V;
-    p->varlen = false;
-    p->T = (long)seq_len;
-    p->nt = (int)((seq_len + BT - 1) / BT);
-    const size_t fixed = batch * (size_t)p->nt;
-    const size_t packed = ntok / BT + N;
-    p->slots = (long)(fixed > packed ? fixed : packed);
-    plan_segments(p, dtype);
-    return true;
+    if (N == 0 || N > (size_t)INT32_MAX / 2) return 0;
+    Problem p;
+    p.ntok = (long)ntok;
+    p.H = (int)H;
+    p.K = (int)K;
+    p.V = (int)V;
+    p.N = (int)N;
+    set_layout(&p, true, seq_len, dtype);
+    const size_t packed = carve(p);
+    if (batch == 0) return packed;
+    p.N = (int)batch;
+    set_layout(&p, false, seq_len, dtype);
+    return std::max(packed, carve(p));
 }
 
 extern "C" size_t efla_chunk_fwd_workspace_size(size_t batch_size, size_t seq_len,
                                                 size_t num_seqs, size_t num_heads,
                                                 size_t head_dim_k, size_t head_dim_v,
                                                 int dtype) {
-    Problem p;
-    if (!ws_problem(batch_size, seq_len, num_seqs, num_heads, head_dim_k, head_dim_v, dtype, &p))
-        return 0;
-    return dtype == kDtypeBF16 ? carve_fwd<bf16>(p, nullptr, nullptr, false)
-                               : carve_fwd<float>(p, nullptr, nullptr, false);
+    return ws_size(batch_size, seq_len, num_seqs, num_heads, head_dim_k, head_dim_v, dtype,
+                   [&](const Problem& p) {
+                       return dtype == kDtypeBF16 ? carve_fwd<bf16>(p, nullptr, nullptr, false)
+                                                  : carve_fwd<float>(p, nullptr, nullptr, false);
+                   });
 }
 
 extern "C" size_t efla_chunk_bwd_workspace_size(size_t batch_size, size_t seq_len,
                                                 size_t num_seqs, size_t num_heads,
                                                 size_t head_dim_k, size_t head_dim_v,
                                                 int dtype) {
-    Problem p;
-    if (!ws_problem(batch_size, seq_len, num_seqs, num_heads, head_dim_k, head_dim_v, dtype, &p))
-        return 0;
-    return dtype == kDtypeBF16 ? carve_bwd<bf16>(p, nullptr, nullptr)
-                               : carve_bwd<float>(p, nullptr, nullptr);
+    return ws_size(batch_size, seq_len, num_seqs, num_heads, head_dim_k, head_dim_v, dtype,
+                   [&](const Problem& p) {
+                       return dtype == kDtypeBF16 ? carve_bwd<bf16>(p, nullptr, nullptr)
+                                                  : carve_bwd<float>(p, nullptr, nullptr);
+                   });
 }
 
 // Token strides of the strided entry points (NULL: packed), in the order

@@ -74,9 +74,9 @@ int efla_rt_event_elapsed_ms(float* ms, hipEvent_t start, hipEvent_t stop);
  * grows the buffer and the workspace is not released, and must not run beside
  * other library calls of that stream.  So is an aligned bf16 / fp16 product
  * split along its contraction, which without a large enough buffer is captured
- * in one piece (the same sum, other roundings).  The others (odd sizes, strides or alignments;
- * efla_forward_hip with other head_dim) are captured in forms without scratch
- * and have no such condition. */
+ * in one piece (the same sum, other roundings).  The others (odd sizes, strides
+ * or alignments; efla_forward_hip with other head_dim) are captured in forms
+ * without scratch and have no such condition. */
 /* Bytes currently held by the cached workspaces of the current device. */
 size_t efla_rt_workspace_bytes(void);
 /* Release the cached workspaces of the current device (synchronises it). */

@@ -595,3 +595,38 @@ def test_segmented_scans_same_bits_every_way(oracle):
                         device="cuda:0")
     o3, _ = chunk_efla_fwd(*a4, s0, workspace=small)
     assert rel_l2(o3, o.float().cpu().numpy()) <= 2e-2
+
+
+# A workspace of exactly the queried size runs the plan that a call without one
+# runs, on both sides of a whole number of chunks: the same bits.  The longest
+# lie where the scratch that a plan may take ends (38016 x 16 heads: five segments
+# with the call's chunk count, four with one chunk more per sequence).
+@pytest.mark.parametrize("B,T,H,K,V", [(1, 4096, 2, 128, 128), (1, 4097, 2, 64, 64),
+                                       (1, 38016, 16, 128, 128), (1, 38015, 16, 128, 128),
+                                       (3, 45952, 4, 128, 128), (2, 33792, 8, 128, 128)])
+def test_queried_workspace_runs_the_same_plan(B, T, H, K, V):
+    from ceo_amd.efla import chunk_efla_bwd, chunk_efla_fwd, new_workspace, workspace_bytes
+
+    announce(f"queried workspace B={B} T={T} H={H} K={K} V={V}")
+    gen = torch.Generator(device="cuda").manual_seed(T)
+
+    def r(*s):
+        return torch.randn(*s, generator=gen, device="cuda")
+
+    bf = torch.bfloat16
+    k = r(B, T, H, K)
+    k = (k / k.norm(dim=-1, keepdim=True)).to(bf)
+    q, v, do = r(B, T, H, K).to(bf), r(B, T, H, V).to(bf), r(B, T, H, V).to(bf)
+    a4 = (q, k, v, torch.sigmoid(r(B, T, H)).to(bf))
+    s0 = r(B, H, K, V) * 0.1
+    o, st = chunk_efla_fwd(*a4, s0, True)
+    ws = torch.empty(workspace_bytes("fwd", B, T, H, K, V, bf), dtype=torch.uint8, device="cuda")
+    o2, st2 = chunk_efla_fwd(*a4, s0, True, workspace=ws)
+    assert torch.equal(o, o2) and torch.equal(st, st2)
+    ref = chunk_efla_bwd(*a4, do, s0)
+    ws = new_workspace(q, v)
+    o2, _ = chunk_efla_fwd(*a4, s0, workspace=ws, save_states=True)
+    assert torch.equal(o, o2)
+    got = chunk_efla_bwd(*a4, do, s0, workspace=ws, reuse_forward=True, reuse_states=True)
+    for a, b, n in zip(got, ref, ("dq", "dk", "dv", "dbeta", "dh0")):
+        assert torch.equal(a, b), n

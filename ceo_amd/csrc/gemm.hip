@@ -448,33 +448,54 @@ struct Tiling {
     long tiles, kper;
 };
 
-// The tile and the split of a product, by its estimated time.  Per 64-deep
-// k-iteration a 128-tile takes 0.71 us alone on its CU and 1.06 beside another,
-// a 256-tile 1.34 to 1.79 us as the chip fills; start and epilogue 4 and 6.5 us;
-// workgroups past the chip's room come in rounds.  A split writes and reads its
-// fp32 partials and launches the reduction.  Large products keep the 256-tile
-// (16384 x 1024 x 4096: 134 us against 155); those whose 256-tiles do not fill
-// the chip take the smaller one.  Measured (256-tile with its best split /
-// 128-tile with its best, us; m x k x n, forward):
-//    130 x 1024 x 4096  18.6 / 14.2     130 x 4096 x 1024  20.7 / 15.0
-//    400 x 1024 x 1024  17.5 / 12.7    1000 x 1024 x 4096  30.7 / 17.6
-//   1000 x 1024 x 1024  24.3 / 15.5    2500 x 4096 x 1024  46.3 / 38.0
-//   2500 x 1024 x 1024  27.5 / 16.2    6000 x 1024 x 1024  30.8 / 21.5
-//   6000 x 1024 x 4096  64.7 / 62.3   16384 x 1024 x 1024  36.1 / 42.0
+// The tile and the split of a product, by its estimated time (us).  Workgroups
+// come in rounds of what the chip holds, two 128-tiles or one 256-tile to a CU.
+// A 64-deep k iteration takes 0.87 / 1.53 us in a full round, 0.88 to 0.99 /
+// 1.25 to 1.39 in the last one, the more the fuller that is; start and epilogue
+// 3.2 to 4 / 6.6 to 7.4.  Small tiles whose count is no multiple of 8, and so
+// are not in bands of an XCD's own, take 9 % longer.  Below 119 ns per MB that
+// the XCDs' L2s have to fetch no product falls.  A split adds its reduction's
+// launch and chain, and its fp32 partials are written and read.
+//
+// The numbers are fitted to 2412 products timed with either tile and up to a
+// dozen splits: 65 to 16384 rows, 128 to 32000 columns, contractions of 64 to
+// 50000, each in the forward's and both gradients' layouts.  The choice is 0.4 %
+// over the best on average for the layers' sizes and 1.3 % for random ones (an
+// estimate with one time per iteration, cheaper partials and no L2 term: 1.4 and
+// 1.6 %, and up to 17 % over the 256-tile alone at contractions of 32000).
+// Measured, us (m x n x k: the 256-tile with its best split / the 128-tile):
+//   1024 x 1024 x 1024   23.8 / 13.6    4096 x  256 x  1024   23.7 / 13.7
+//   1024 x 1024 x 4096   31.2 / 24.7    1024 x 1024 x 16384   55.9 / 55.1
+//   2048 x 1024 x 16384  86.5 / 90.5    1024 x 3088 x 16384  122.6 / 127.1
+//   1024 x 1024 x 32000  85.7 / 95.5     256 x 1024 x 32000   47.1 / 41.6
+//   6000 x 3072 x  768   58.5 / 48.8   16384 x 1024 x  1024   36.1 / 42.0
 static double tiling_cost(int ts, long M, long N, long K, int ksplit, long kper, long cus) {
     const double it = (double)((kper + gf::BK - 1) / gf::BK);
-    const long w = ((M + ts - 1) / ts) * ((N + ts - 1) / ts) * ksplit;
-    double t;
+    const long tm = (M + ts - 1) / ts, tn = (N + ts - 1) / ts, w = tm * tn * ksplit;
+    const long room = ts == 128 ? 2 * cus : cus, full = (w + room - 1) / room - 1;
+    const double fill = (double)(w - full * room) / (double)room;  // of the last round
+    double t, start;
     if (ts == 128) {
-        const double alone = it * 0.71 + 3.7, paired = it * 1.06 + 4.;
-        const long full = w / (2 * cus), rest = w % (2 * cus);
-        t = (double)full * paired + (rest == 0 ? 0. : rest <= cus ? alone : paired);
+        const double both = std::max(0., 2. * fill - 1.);  // CUs with two workgroups
+        start = 3.2;
+        t = (double)full * (it * 0.87 + 4.) + it * (0.88 + 0.11 * both * both) + start;
+        if (w % 8 != 0 && full > 0) t *= 1.09;
     } else {
-        const long full = w / cus, rest = w % cus;
-        auto round = [&](double fill) { return it * (1.34 + 0.45 * fill) + 6.5; };
-        t = (double)full * round(1.) + (rest ? round((double)rest / (double)cus) : 0.);
+        start = 7.4;
+        t = (double)full * (it * 1.53 + 6.6) + it * (1.25 + 0.14 * fill * fill) + start;
     }
-    if (ksplit > 1) t += 3. + (double)ksplit * (double)M * (double)N * 4. * 1.3 / 4.5e6;
+    // what the L2s fetch: an XCD's band is `part` of the splits of some tiles in
+    // groups of 8 rows (decode in the kernel)
+    const bool band = w % 8 == 0;
+    const long tiles = band ? std::max(1L, w / 8 / ksplit) : (tm * tn + 7) / 8;
+    const long rows = std::min({8L, tm, band ? tiles : tm});
+    const long cols = std::min(tn, band ? (tiles + rows - 1) / rows : tiles);
+    const double part =
+        band ? (double)std::min((long)ksplit, w / 8) / (double)ksplit : 1.;
+    const double mb = 8. * (double)(rows + cols) * (double)ts * (double)K * 2e-6 * part;
+    t = std::max(t, mb * 0.119 + start);
+    if (ksplit > 1)
+        t += 3.7 + (double)ksplit * (0.43 + (double)M * (double)N * 4e-6 * 0.43);
     return t;
 }
 

@@ -569,9 +569,26 @@ static void fast_kernel_launch(const FastOp& a, const FastOp& b, const gf::Opnd&
 // Few-row products (gemm_skinny.hpp) up to this many rows, four 16-row tiles a
 // wave; from 65 on the large tile.  Measured (this at 64 rows / large tile at
 // 65, us): 1024 x 3088 8.2 / 15.1, 1024 x 1024 7.7 / 13.1, 4096 x 1024
-// 11.1 / 18.3, 1024 x 32000 27.1 / 26.4; transposed weights (dA) 9.4 / 17.4,
-// 7.8 / 13.2, 8.4 / 15.4, 29.6 / 38.6.
+// 11.1 / 18.3; transposed weights (dA) 9.4 / 17.4, 7.8 / 13.2, 8.4 / 15.4,
+// 32000 x 1024 29.6 / 38.6.  (Large weights: skinny_size.)
 constexpr long kSkinnyRows = 64;
+
+// Whether the few-row kernel is the faster one for an aligned product: while the
+// weights are small, or where the tile kernel would have too few workgroups, an
+// epilogue that cannot be split over columns that do not fill the chip.  Large
+// weights it streams at 2 to 3 TB/s, the tiles at up to 6.  Measured, weights
+// from the caches (us, k x n: this / tiles, 1 row and 64 rows):
+//   forward  1024 x  8192  6.9 / 10.3,   8.0 / 10.4   2048 x  6144  10.1 / -, 13.8 / -
+//            1024 x 16384 12.0 /  9.8,  14.9 / 14.5   4096 x  4096  14.3 / 13.1, 18.2 / 17.9
+//            1024 x 32000 22.2 / 16.1,  28.4 / 16.3   8192 x 28672   158 / 79, 236 / 98
+//   dA       2048 x  8192  7.2 / 10.7,  13.4 / 14.7   1024 x 32000  11.9 / 14.8, 24.0 / 15.9
+//            4096 x 14336 26.8 / 21.1,  45.8 / 26.2   1024 x 50304  18.0 / 16.8, 39.5 / 18.4
+//   GELU     4096 x 14336 37.6 / 92.6,  48.2 / 96.4   8192 x 28672   158 / 195, 238 / 198
+static bool skinny_size(const FastOp& b, long M, long N, long K, bool may_split) {
+    const long w = N * K, cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    if (!may_split && N < 96 * cus) return true;  // under three quarters of a round
+    return b.kc ? w <= (M <= 16 ? 1L << 25 : 1L << 24) : w < 1L << 24;
+}
 
 // whether gemm_skinny_kernel takes the problem
 static bool skinny_ok(const FastOp& a, const FastOp& b, long M, long N, long K) {
@@ -675,7 +692,8 @@ static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
                            (!ea.aux || (ea.ldaux % 8 == 0 && aligned_to(ea.aux, 16)));
     const bool plain = !pa && !pb && K % 8 == 0 && out_whole;
     if constexpr (EPI != gf::EPI_DGELU)
-        if (skinny_ok(a, b, M, N, K))
+        if (skinny_ok(a, b, M, N, K) &&
+            (!plain || skinny_size(b, M, N, K, EPI != gf::EPI_GELU_AUX)))
             return skinny_launch<T, EPI>(a, b, M, N, K, ea, plain, name, st);
     if (!plain && (double)M * (double)N * (double)K < (double)kPadMinWork) return -1;
     const Tiling tl = plan_tiling(M, N, K, (EPI == gf::EPI_PLAIN || EPI == gf::EPI_RESID) &&

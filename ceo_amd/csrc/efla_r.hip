@@ -1203,6 +1203,16 @@ inline void r_coeff(int d, const void* k, float* c, float* dc, int H, long T, fl
                     dc, H, T, beta, (long)ntok);
 }
 
+// Whether d = 32 stays on the LDS-resident kernels: one launch, all (b, h) at
+// once, and no more tokens than the register-resident ones' launches cost.
+// Measured (LDS / register, us; (b, h) x tokens): forward 1 x 1 6.9 / 9.9,
+// 128 x 4 9.2 / 10.2, 128 x 5 10.7 / 10.1, 1024 x 1 14.3 / 10.4; backward
+// 128 x 1 14.1 / 15.8, 128 x 2 21.4 / 16.1, 1024 x 1 48.5 / 16.3.
+inline bool r_lds_d32(size_t nbh, size_t T, size_t tokens) {
+    const size_t ncu = device_cu_count() > 0 ? device_cu_count() : 256;
+    return T <= tokens && nbh <= ncu;
+}
+
 // chunk_size as the forward's segment length: 16, 32 or 64 tokens staged in
 // LDS at once (the largest not above it, at least 16; 0 picks 32)
 inline int r_segment(size_t chunk_size) {
@@ -1421,9 +1431,10 @@ extern "C" int efla_forward_hip(const void* k, const void* v, void* state, void*
     // the register-resident path: d = 32 / 64 / 128, k and v aligned for d /
     // 8-byte row loads (the coefficient kernel's, the segment staging's) and
     // output for 8-byte row pieces, at most 2^35 tokens (d = 32: not in a capture,
-    // since the LDS-resident kernel needs no scratch)
+    // since the LDS-resident kernel needs no scratch, and from five tokens on)
     const bool fast = (head_dim == 128 || head_dim == 64 ||
-                       (head_dim == 32 && workspace_optional(stream))) &&
+                       (head_dim == 32 && !r_lds_d32(nbh, seq_len, 4) &&
+                        workspace_optional(stream))) &&
                       (uintptr_t)k % (head_dim / 8) == 0 && (uintptr_t)v % (head_dim / 8) == 0 &&
                       (uintptr_t)output % 8 == 0 && nbh * seq_len <= ((size_t)1 << 35);
     if (fast) {
@@ -1492,9 +1503,10 @@ extern "C" int efla_backward_hip(const void* grad_output, const void* k, const v
     if (head_dim > (size_t)MAXD || nbh > (size_t)INT32_MAX) return kInvalidConfiguration;
     // the register-resident path: d = 32 / 64 / 128, k, dO and v aligned for d /
     // 8-byte row loads (the coefficient kernel's, the segment staging's) and
-    // grad_k for 8-byte row pieces, at most 2^35 tokens
+    // grad_k for 8-byte row pieces, at most 2^35 tokens (d = 32: from two tokens on)
     const size_t ra = head_dim / 8;
-    const bool fast = (head_dim == 128 || head_dim == 64 || head_dim == 32) &&
+    const bool fast = (head_dim == 128 || head_dim == 64 ||
+                       (head_dim == 32 && !r_lds_d32(nbh, seq_len, 1))) &&
                       (uintptr_t)k % ra == 0 && (uintptr_t)grad_output % ra == 0 &&
                       (uintptr_t)v % ra == 0 && (uintptr_t)grad_k % 8 == 0 &&
                       nbh * seq_len <= ((size_t)1 << 35);

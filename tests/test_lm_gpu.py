@@ -146,3 +146,31 @@ def test_cross_entropy_row_with_inf_or_nan(bad):
     loss, grad = cross_entropy_forward_backward(z.cuda(), t.cuda())
     assert loss.isnan().tolist() == [False, True, False]
     assert grad.isnan().all(1).tolist() == [False, True, False] and not grad[0].isnan().any()
+
+
+# The three entries agree with each other and in both paths (rows of whole 16-byte
+# pieces up to 65536 logits in registers, others looped): ordinary rows to the bounds
+# above, and a row with +inf or NaN gives NaN for its loss and its whole gradient.
+@pytest.mark.parametrize("V", [1000, 1001, 32000, 32001, 40000, 65536, 65544])
+def test_cross_entropy_entries_and_paths_agree(V):
+    from ceo_amd.nn import (cross_entropy_backward, cross_entropy_forward,
+                            cross_entropy_forward_backward)
+
+    announce(f"cross_entropy entries V={V}")
+    g = torch.Generator().manual_seed(V)
+    z = (torch.randn(4, V, generator=g) * 3).to(torch.bfloat16)
+    z[2, V // 3], z[3, V - 1] = float("inf"), float("nan")
+    t = torch.tensor([V - 1, 5, 1, 2], dtype=torch.int32).cuda()
+    zc, gl = z.cuda(), torch.ones(4, device="cuda")
+    loss, grad = cross_entropy_forward_backward(zc, t)
+    alone = cross_entropy_forward(zc, t), cross_entropy_backward(gl, zc, t)
+    lp = torch.log_softmax(z[:2].double(), -1)
+    rg = lp.exp()
+    rg[torch.arange(2), t[:2].long().cpu()] -= 1
+    ref = -lp.gather(1, t[:2].long().cpu()[:, None])[:, 0] / 4
+    for lo, gr in ((loss, grad), alone):
+        assert lo.isnan().tolist() == [False, False, True, True]
+        assert gr[2:].isnan().all() and not gr[:2].isnan().any()
+        assert ((lo[:2].double().cpu() - ref).abs() / ref.abs().clamp(min=1)).max() <= 1e-5
+        d = (gr[:2].double().cpu() * 4 - rg).abs() - (2.0 ** -8 + 60 * 2.0 ** -22) * rg.abs()
+        assert d.max() <= 1e-5

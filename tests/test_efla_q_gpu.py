@@ -630,3 +630,65 @@ def test_queried_workspace_runs_the_same_plan(B, T, H, K, V):
     got = chunk_efla_bwd(*a4, do, s0, workspace=ws, reuse_forward=True, reuse_states=True)
     for a, b, n in zip(got, ref, ("dq", "dk", "dv", "dbeta", "dh0")):
         assert torch.equal(a, b), n
+
+
+def test_segmented_scans_from_fused_rows(oracle):
+    """Sequences in segments read from, and with gradients written to, column slices
+    of one row per token: the same bits as packed tensors."""
+    from ceo_amd.efla import chunk_efla_bwd, chunk_efla_fwd, new_workspace
+
+    for B, T, H, K, V in ((1, 4100, 2, 128, 128), (2, 2600, 4, 64, 64)):
+        announce(f"segmented scans from fused rows B={B} T={T} H={H} K={K} V={V}")
+        x = oracle.make_efla_inputs(99 + K, B * T, H, K, V, bf16=True)
+        g = {n: to_dev(a, torch.bfloat16, (B, T, H, K) if n in "qk" else
+                       (B, T, H) if n == "beta" else (B, T, H, V)) for n, a in x.items()}
+        s0 = 0.1 * torch.randn(B, H, K, V, generator=torch.Generator().manual_seed(5)).cuda()
+
+        def slices(row):
+            return [row[:, a:a + n].view(B, T, H, -1) for a, n in
+                    ((0, H * K), (H * K, H * K), (2 * H * K, H * V))]
+
+        width = H * (2 * K + V) + 8
+        row, grad = (torch.zeros(B * T, width, dtype=torch.bfloat16, device="cuda")
+                     for _ in range(2))
+        for t, n in zip(slices(row), "qkv"):
+            t.copy_(g[n])
+        views = slices(row)
+        for saved in (False, True):
+            res = []
+            for qkv, out in (((g["q"], g["k"], g["v"]), None), (views, slices(grad))):
+                ws = new_workspace(g["q"], g["v"]) if saved else None
+                o, st = chunk_efla_fwd(*qkv, g["beta"], s0, True, workspace=ws, save_states=saved)
+                gr = chunk_efla_bwd(*qkv, g["beta"], g["do"], s0, workspace=ws,
+                                    reuse_forward=saved, reuse_states=saved, grads_out=out)
+                res.append((o, st) + tuple(t.clone() for t in gr))
+            for a, b, n in zip(*res, ("o", "st", "dq", "dk", "dv", "dbeta", "dh0")):
+                assert torch.equal(a, b), (saved, n)
+            assert not grad[:, width - 8:].any()
+
+
+def test_long_sequence_alone_and_packed_agree(oracle):
+    """A sequence long enough for segments takes them alone; in a packed batch every
+    sequence is one chain.  The two round differently, each within the bf16
+    path's bound of the exact result, so of each other within twice that."""
+    from ceo_amd.efla import chunk_efla_bwd, chunk_efla_fwd
+
+    lens, H, K, V = (4100, 130, 2560), 2, 128, 128
+    announce(f"long sequences alone and packed {lens}")
+    T = sum(lens)
+    x = oracle.make_efla_inputs(1717, T, H, K, V, bf16=True)
+    g = {n: to_dev(a, torch.bfloat16, (1, T, H, K) if n in "qk" else
+                   (1, T, H) if n == "beta" else (1, T, H, V)) for n, a in x.items()}
+    ends = np.cumsum((0,) + lens)
+    cu = torch.tensor(ends, dtype=torch.int32).cuda()
+    a4 = (g["q"], g["k"], g["v"], g["beta"])
+    o, _ = chunk_efla_fwd(*a4, cu_seqlens=cu)
+    grads = chunk_efla_bwd(*a4, g["do"], cu_seqlens=cu)
+    for lo, hi in zip(ends, ends[1:]):
+        one = [t[:, lo:hi].contiguous() for t in a4]
+        o1, _ = chunk_efla_fwd(*one)
+        g1 = chunk_efla_bwd(*one, g["do"][:, lo:hi].contiguous())
+        for a, b in zip((o,) + grads[:4], (o1,) + g1[:4]):
+            assert rel_l2(a[:, lo:hi], b.float().cpu().numpy()) <= 2 * TOL[torch.bfloat16]
+            if hi - lo < 16 * 64:
+                assert torch.equal(a[:, lo:hi], b)

@@ -726,3 +726,115 @@ def test_gemm_small_tile(m, k, n):
     errs["dpre_bias"] = off(pb, dpre.double().sum(0))
     print("  rel-L2:", {n_: f"{v:.2e}" for n_, v in errs.items()}, flush=True)
     assert all(v <= 2.0 ** -8 for v in errs.values()), errs
+
+
+# The 256 x 256 tile with odd sizes: 16 x 16 of them, the last row and column of
+# tiles partial, in every layout and epilogue; and a long contraction over few of
+# them, split into fp32 partials.  Beside the norm, element by element what a norm
+# hides: the last rows, the last columns with their partial 8-element piece and the
+# first ones.  Bound there: the product is rounded once to bf16 (2^-8 of it) after
+# an fp32 sum of k products (k 2^-24 of their magnitudes' sum).
+def _edges(m, n):
+    rows = sorted({0, 127, 128, 255, 256, m - 129, m - 2, m - 1})
+    cols = sorted({0, 7, 255, 256, n - 9, n - 8, n - 3, n - 2, n - 1})
+    return torch.tensor(rows, device="cuda"), torch.tensor(cols, device="cuda")
+
+
+def _check_product(got, a, b, name, extra=None):
+    """got = a b (+ extra) with a, b, extra in 64 bits."""
+    m, n = got.shape
+    ref = a @ b
+    if extra is not None:
+        ref += extra
+    rel = ((got.double() - ref).norm() / ref.norm()).item()
+    rows, cols = _edges(m, n)
+    for g, r, s in ((got[rows], ref[rows], a[rows].abs() @ b.abs()),
+                    (got[:, cols], ref[:, cols], a.abs() @ b[:, cols].abs())):
+        bound = 2.0 ** -8 * r.abs() + a.shape[1] * 2.0 ** -24 * s + 1e-30
+        worst = ((g.double() - r).abs() / bound).max().item()
+        assert worst <= 1.0, (name, worst)
+    print(f"  {name}: rel-L2 {rel:.2e}", flush=True)
+    assert rel <= 2.0 ** -8, name
+
+
+def test_gemm_odd_shapes_256_tile():
+    from ceo_amd import nn
+
+    m, n, k = 4090, 4083, 1031
+    announce(f"gemm odd {m}x{k}x{n}, 256 tiles")
+    g = torch.Generator(device="cuda").manual_seed(256)
+
+    def r(*s):
+        return torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+
+    a, b, bias = r(m, k), r(k, n), r(n)
+    A, B = a.double(), b.double()
+    at, bt = a.T.contiguous(), b.T.contiguous()
+    _check_product(nn.gemm_forward(a, b, bias), A, B, "forward", bias.double())
+    out = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    for ta, tb in ((False, True), (True, False), (True, True)):
+        nn.gemm_ex(at if ta else a, bt if tb else b, out, trans_a=ta, trans_b=tb)
+        _check_product(out, A, B, f"trans {ta} {tb}")
+    # views whose rows start off a 16-byte boundary, nothing written beside them
+    wide, res = torch.zeros(m, n + 13, dtype=torch.bfloat16, device="cuda"), r(m, n + 3)
+    view, c = wide[:, 1:1 + n], res[:, 2:2 + n]
+    nn.gemm_ex(a, b, view, bias=bias, c=c, alpha=0.5, beta=1.0)
+    _check_product(view, 0.5 * A, B, "residual", bias.double() + c.double())
+    assert not wide[:, 0].any() and not wide[:, n + 1:].any()
+    pre, act = nn.gemm_gelu_forward(a, b, bias)
+    _check_product(pre, A, B, "pre", bias.double())
+    ref = torch.nn.functional.gelu(pre.double(), approximate="tanh")
+    # GELU of the rounded pre-activation, once more rounded, its fp32 evaluation
+    # a few units of 2^-24 of the pre-activation
+    assert ((act.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -20 * pre.double().abs()
+            + 1e-30).all()
+
+
+@pytest.mark.parametrize("f", [4083, 4088])
+def test_gemm_gelu_backward_odd_256_tile(f):
+    """dpre of m x f from a contraction of odd length; f = 4088 also sums its
+    columns in the product's epilogue (128 rows at a time)."""
+    from ceo_amd import nn
+
+    m, d = 4090, 1031
+    announce(f"gemm gelu backward {m}x{f}x{d}, 256 tiles")
+    g = torch.Generator(device="cuda").manual_seed(f)
+
+    def r(*s):
+        return torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+
+    dy, w, pre = r(m, d), r(f, d), r(m, f)
+    pb = torch.empty(f, dtype=torch.bfloat16, device="cuda")
+    dpre, _, _ = nn.gemm_gelu_backward(dy, pre, w, pre, need_b=False, out_pre_bias=pb)
+    prod = nn.gemm_ex(dy, w, torch.empty_like(pre), trans_b=True)
+    _check_product(prod, dy.double(), w.double().T, "product")
+    x = pre.double().requires_grad_(True)
+    (one,) = torch.autograd.grad(torch.nn.functional.gelu(x, approximate="tanh").sum(), x)
+    ref = prod.double() * one
+    # the same product, rounded; GELU' in fp32 is off by a few units of 2^-24 of 1
+    bound = 2.0 ** -8 * ref.abs() + 2.0 ** -19 * prod.double().abs() + 1e-30
+    assert ((dpre.double() - ref).abs() <= bound).all()
+    sums = dpre.double().sum(0)
+    scale = dpre.double().abs().sum(0)
+    assert ((pb.double() - sums).abs() <= 2.0 ** -8 * sums.abs() + m * 2.0 ** -24 * scale).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(1021, 1019, 32003), (2045, 1019, 32003)])
+def test_gemm_odd_split_256_tile(m, n, k):
+    from ceo_amd import nn
+
+    announce(f"gemm odd split {m}x{n}x{k}, 256 tiles")
+    g = torch.Generator(device="cuda").manual_seed(k)
+
+    def r(*s):
+        return torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+
+    a, b, c = r(m, k), r(k, n), r(m, n)
+    A, B = a.double(), b.double()
+    at, bt = a.T.contiguous(), b.T.contiguous()
+    out = torch.empty_like(c)
+    for ta, tb in ((False, False), (False, True), (True, False)):
+        nn.gemm_ex(at if ta else a, bt if tb else b, out, trans_a=ta, trans_b=tb)
+        _check_product(out, A, B, f"trans {ta} {tb}")
+    nn.gemm_ex(at, b, out, c=c, beta=1.0, trans_a=True)
+    _check_product(out, A, B, "residual", c.double())

@@ -666,6 +666,18 @@ static int skinny_launch(const FastOp& a, const FastOp& b, long M, long N, long 
 //   2100 x 768 x 16001   fwd  400 / 90    dA 4387 / 116  dB  523 / 89
 //   2500 x 1024 x 4096   dB   269 / 47  (rows read in place: only k is odd)
 constexpr long kPadMinWork = (long)1 << 22;
+// Two operands to pad for a contraction of one or two iterations of the generic
+// kernel are not worth their launches either: with both operands k-contiguous
+// (dA, whose generic form reads them fastest) at any size, in the other forms until
+// the output is large.  (Generic / this, us; k, output:
+//    9, 1001 x 1023  fwd 10.2 / 12.4  dA 10.0 / 12.6  dB 10.5 / 12.5
+//    9, 3001 x 4097  fwd 22.9 / 16.7  dA 21.2 / 18.0  dB 23.8 / 15.2
+//   25, 5000 x 2047  dA 14.4 / 18.5  41, 18.4 / 18.9  65, 28.5 / 20.1
+//   33,  300 x  515  fwd 13.4 / 12.4  dA 11.5 / 12.5  dB 15.4 / 12.7)
+static bool too_short(const FastOp& a, const FastOp& b, long M, long N, long K) {
+    if (a.kc && b.kc) return K <= (M * N < (long)1 << 22 ? 48 : 32);
+    return K <= 32 && M * N < (long)1 << 23;
+}
 // padded copies past this many bytes are not made: such a product stays on the
 // generic kernel, which needs no scratch
 constexpr size_t kPadMaxBytes = (size_t)4 << 30;
@@ -696,6 +708,7 @@ static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
             (!plain || skinny_size(b, M, N, K, EPI != gf::EPI_GELU_AUX)))
             return skinny_launch<T, EPI>(a, b, M, N, K, ea, plain, name, st);
     if (!plain && (double)M * (double)N * (double)K < (double)kPadMinWork) return -1;
+    if (pa && pb && too_short(a, b, M, N, K)) return -1;
     const Tiling tl = plan_tiling(M, N, K, (EPI == gf::EPI_PLAIN || EPI == gf::EPI_RESID) &&
                                                may_split);
     if (tl.tiles > 0x7FFFFFFFL / 64) return plain ? kInvalidConfiguration : -1;

@@ -709,6 +709,11 @@ static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
             return skinny_launch<T, EPI>(a, b, M, N, K, ea, plain, name, st);
     if (!plain && (double)M * (double)N * (double)K < (double)kPadMinWork) return -1;
     if (pa && pb && too_short(a, b, M, N, K)) return -1;
+    // GELU' over rows that are not whole 16-byte pieces: the product and then
+    // gelu_backward are faster, the same values (this form / those, us; m x k x n:
+    // 1001 x 1023 x 64 13.7 / 11.1, x 512 18.1 / 12.8; 5000 x 2047 x 256 38.7 / 28.0;
+    // 16384 x 769 x 256 28.0 / 30.2)
+    if (EPI == gf::EPI_DGELU && !out_whole) return -1;
     const Tiling tl = plan_tiling(M, N, K, (EPI == gf::EPI_PLAIN || EPI == gf::EPI_RESID) &&
                                                may_split);
     if (tl.tiles > 0x7FFFFFFFL / 64) return plain ? kInvalidConfiguration : -1;
@@ -764,8 +769,9 @@ static int fast_launch(const FastOp& a, const FastOp& b, long M, long N, long K,
     if (pb) pad(b, rb, cb, ws + up(head_bytes) + ba, B);
     const bool ragged = !out_whole;
     if (ksplit == 1) {
-        if (ragged)
-            fast_kernel_launch<T, EPI, true>(a, b, A, B, M, N, K, ep, tl, name, st);
+        if (EPI != gf::EPI_DGELU && ragged)
+            fast_kernel_launch<T, EPI == gf::EPI_DGELU ? gf::EPI_PLAIN : EPI, true>(
+                a, b, A, B, M, N, K, ep, tl, name, st);
         else
             fast_kernel_launch<T, EPI, false>(a, b, A, B, M, N, K, ep, tl, name, st);
         return (int)hipPeekAtLastError();
@@ -1070,11 +1076,6 @@ extern "C" int gemm_gelu_backward_hip(const void* grad_c, const void* a, const v
                                 dim3((unsigned)((k + 63) / 64)), dim3(NTH), stream,
                                 (const float*)lease.ptr(), prow, (bf16*)grad_pre_bias,
                                 (long)k);
-                } else if (done == 0 && grad_pre_bias) {
-                    lease.release();  // colsum_bf16 takes its own
-                    const int rc = colsum_bf16((const bf16*)grad_pre, (long)m, (long)k,
-                                               (bf16*)grad_pre_bias, stream);
-                    if (rc != kSuccess) return rc;
                 }
             }
             if (done < 0) {

@@ -46,7 +46,8 @@ namespace q {
 // operands, and small fp32 problems have few workgroups, so their time is these
 // chains' latency.  With four waves of four tiles each, one after the other, the
 // forward and backward of 2 x 256 tokens, 4 heads, d = 64 took 234 us (its seven
-// kernels 237 us together under a trace); with sixteen 175 us (126 us).
+// kernels 237 us together under a trace); with sixteen 175 us (126 us), 155 us
+// (109 us) since the backward reads the states the forward left.
 constexpr int NTH = 1024;  // threads per workgroup
 constexpr int NW = 16;     // waves per workgroup
 constexpr int LDF = 68;   // row stride of the 64x64 fp32 LDS matrices
@@ -946,10 +947,15 @@ static SeqInfo make_seqinfo(const Problem& p, const int32_t* cu_s, const int32_t
 //   1 x 4096 x  8,  64 x 64                102 / 206   69 / 156   57 / 128   42 / 96
 //   1 x 8192 x 32, 128 x 128 (64 chains)   320 / 788  211 / 607  205 / 634  223 / 672
 // The scan's workgroups stay at one per CU (its LDS allows no more).  The
-// plan depends on nothing but the problem's shape and the device, so every call
-// on a problem, with saved states or without, gives the same bits; it keeps
-// the forward's scratch within the fixed array of the entry that allocates
-// nothing, whose results are the same too.
+// plan depends on nothing but the problem's shape and the device: calls without a
+// caller's workspace, or with one of the queried size, give the same bits, with
+// saved states or without.  A smaller workspace that holds one chain's factors is
+// taken too and runs one chain per sequence, with other roundings.  The plan
+// keeps the forward's scratch within the fixed array of the entry that
+// allocates nothing, whose results are then the same; so segments end where the
+// factors and the segments' states pass it (16 heads, d = 128: eight segments up
+// to 33000 tokens, five at 36000, three at 40000, none from 40896 on).  A packed
+// batch runs one chain per sequence whatever their lengths.
 static void plan_segments(Problem* p, int dtype) {
     p->nseg = 1;
     p->segc = p->nt;
@@ -1136,8 +1142,10 @@ static int run_bwd(const Problem& p, const T* q, const T* k, const T* v, const T
 //    8 x 16, 128 x 128    4.8 / 13.4   9.1 / 13.6  14.9 / 13.9  20.8 / 13.6
 //    1 x  4,  64 x  64    3.2 / 10.0   6.7 / 10.0  11.3 / 10.0  16.3 /  9.9
 //  256 x  8,  64 x 128   22.5 / 75.5  43.2 / 74.5  73.5 / 74.8 103.3 / 75.1
-// Only continuations (an initial state) of equal-length sequences take it: a
-// sequence run from its start gives the same bits alone and in a packed batch.
+// Only continuations (an initial state) of equal-length sequences take it, and only
+// without a caller's workspace (which must end up holding T and b for a backward):
+// with one, the same call runs a padded chunk, whose state meets bf16 roundings
+// that the steps do not have.
 constexpr long kStepTokens = 6;
 
 template <typename T, int K, int V>

@@ -21,7 +21,8 @@
 // the logits once and the backward reads them once and writes the gradient
 // once; cross_entropy_forward_backward_hip (no reference counterpart) does
 // both from one read, optionally in place.  Other rows take a looped two-pass
-// path.  A target outside [0, V) gives loss NaN and a zero gradient row.
+// path.  A target outside [0, V) gives loss NaN and a zero gradient row; a row with
+// a +inf or NaN logit gives NaN for its loss and its whole gradient, in both paths.
 #include <hip/hip_runtime.h>
 #include <math.h>
 

@@ -108,6 +108,16 @@ int efla_chunked_scan_hip(void** chunk_states, size_t num_chunks, size_t num_hea
  * {64,128} x {64,128,256} for bf16, d_k = d_v = 64 for fp32.
  * Workspace: pass NULL to use the library's cached buffer for `stream`, or
  * a buffer of at least efla_chunk_*_workspace_size() bytes.
+ *
+ * Which calls give the same bits: a problem of equal-length sequences with NULL,
+ * with a workspace of the queried size, with or without saved factors and
+ * states, from packed tensors or column slices, and from the entry that allocates
+ * nothing.  Other roundings, within the same error of the exact result: a
+ * sequence of 16 chunks or more alone (bf16; it may run as several segments at
+ * once) and in a packed batch (always one chain); a bf16 workspace smaller than
+ * the queried size that still holds one chain's factors (accepted, one chain);
+ * and up to 6 tokens from an initial state, which without a caller's workspace
+ * keep the state in fp32 throughout and with one run a padded chunk.
  * ======================================================================== */
 size_t efla_chunk_fwd_workspace_size(size_t batch_size, size_t seq_len, size_t num_seqs,
                                      size_t num_heads, size_t head_dim_k, size_t head_dim_v,
@@ -366,8 +376,10 @@ int prism_backward_hip(const void* grad_output, const void* u, const void* v, co
  * 128 x 128 x 64 tile kernel, whichever is estimated faster, or, with up to 64
  * rows, a kernel that streams the second operand once.  Operands whose rows are not whole 16-byte
  * pieces (odd sizes, strides or alignments) are first copied into padded rows
- * in the stream's workspace (at most 4 GiB; where that is not to be had, and
- * for products below 2^22 multiply-adds, the generic kernel takes them).
+ * in the stream's workspace, on every call (at most 4 GiB, which the workspace
+ * then holds until it is released; where that is not to be had, in a stream
+ * capture, for products below 2^22 multiply-adds and for short contractions of
+ * two such operands, the generic kernel takes them).
  * fp32 and mixed dtypes run the generic 128 x 128 kernel
  * (efla_rt_set_gemm_backend(1) forces it).  No vendor BLAS is linked.
  * ======================================================================== */

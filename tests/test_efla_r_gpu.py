@@ -380,3 +380,13 @@ def test_backward_d32_row_sums_keep_fp32(oracle):
     worst = float((gk[:, -1].double().cpu().numpy().__abs__() / scale).max())
     print(f"  worst |grad_k| / sum |S w1| = {worst:.2e}", flush=True)
     assert worst <= 8 * 2.0 ** -24
+
+
+# d = 32 at the lines between its two paths: four and five tokens in the forward, one
+# and two in the backward, (b, h) up to and past the CU count.
+@pytest.mark.parametrize("B,T,H", [(1, 1, 3), (1, 2, 3), (2, 4, 5), (2, 5, 5), (2, 1, 150),
+                                   (2, 4, 150)])
+def test_d32_few_tokens(oracle, B, T, H):
+    announce(f"efla_forward_hip / efla_backward_hip d=32 few tokens B={B} T={T} H={H}")
+    k, v, do, s0 = _inputs(oracle, 0x32 + T + H, B, T, H, 32, 0.2)
+    _fwd_bwd_vs_oracle(oracle, k, v, do, s0, B, T, H, 32, 0.8, f"T={T}")

@@ -735,8 +735,8 @@ def test_gemm_small_tile(m, k, n):
 # first ones.  Bound there: the product is rounded once to bf16 (2^-8 of it) after
 # an fp32 sum of k products (k 2^-24 of their magnitudes' sum).
 def _edges(m, n):
-    rows = sorted({0, 127, 128, 255, 256, m - 129, m - 2, m - 1})
-    cols = sorted({0, 7, 255, 256, n - 9, n - 8, n - 3, n - 2, n - 1})
+    rows = sorted({0, 127, 128, 255, 256, m - 129, m - 2, m - 1} & set(range(m)))
+    cols = sorted({0, 7, 255, 256, n - 9, n - 8, n - 3, n - 2, n - 1} & set(range(n)))
     return torch.tensor(rows, device="cuda"), torch.tensor(cols, device="cuda")
 
 
@@ -838,3 +838,51 @@ def test_gemm_odd_split_256_tile(m, n, k):
         _check_product(out, A, B, f"trans {ta} {tb}")
     nn.gemm_ex(at, b, out, c=c, beta=1.0, trans_a=True)
     _check_product(out, A, B, "residual", c.double())
+
+
+# Few rows at the lines where the tile kernel takes over from the one that streams
+# the weights: 2^24 weights (2^25 transposed, up to 16 rows), and with GELU three
+# quarters of a round of columns.
+@pytest.mark.parametrize("m,k,n", [(64, 4096, 4088), (64, 4096, 4096), (16, 1024, 24568),
+                                   (16, 1024, 24576), (17, 1024, 32768), (16, 1024, 32768),
+                                   (1, 1024, 32776)])
+def test_gemm_few_rows_large_weights(m, k, n):
+    from ceo_amd import nn
+
+    announce(f"gemm few rows, large weights {m}x{k}x{n}")
+    g = torch.Generator(device="cuda").manual_seed(m + k + n)
+
+    def r(*s):
+        return torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+
+    a, b, dc, bias = r(m, k), r(k, n), r(m, n), r(n)
+    A, B, D = a.double(), b.double(), dc.double()
+    _check_product(nn.gemm_forward(a, b, bias), A, B, "forward", bias.double())
+    _check_product(nn.gemm_backward(dc, a, b, need_b=False)[0], D, B.T, "dA")
+    pre, act = nn.gemm_gelu_forward(a, b, bias)
+    _check_product(pre, A, B, "pre", bias.double())
+    ref = torch.nn.functional.gelu(pre.double(), approximate="tanh")
+    assert ((act.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -20 * pre.double().abs()
+            + 1e-30).all()
+
+
+# Short contractions of two operands that would be padded, on both sides of the
+# lines between the generic kernel and the padded copies.
+@pytest.mark.parametrize("m,n", [(300, 515), (2051, 2047), (2049, 4099)])
+@pytest.mark.parametrize("k", [31, 33, 47, 49])
+def test_gemm_short_odd_contractions(m, n, k):
+    from ceo_amd import nn
+
+    announce(f"gemm short odd contraction {m}x{k}x{n}")
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+
+    def r(*s):
+        return torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+
+    a, b, bias = r(m, k), r(k, n), r(n)
+    A, B = a.double(), b.double()
+    at, bt, out = a.T.contiguous(), b.T.contiguous(), torch.empty_like(r(m, n))
+    _check_product(nn.gemm_forward(a, b, bias), A, B, "forward", bias.double())
+    for ta, tb in ((False, True), (True, False)):
+        nn.gemm_ex(at if ta else a, bt if tb else b, out, trans_a=ta, trans_b=tb)
+        _check_product(out, A, B, f"trans {ta} {tb}")
